@@ -1,6 +1,6 @@
 // Blocked Householder QR on a chain group, and the solve that uses it.
 //
-// k_qr_blocked factors A P0 = Q R panel by panel (compact WY, Q_p = I - V_p T_p V_p^H,
+// k_qr_pipe (8-column panels, the default) and k_qr_blocked (16) factor A P0 = Q R panel by panel (compact WY, Q_p = I - V_p T_p V_p^H,
 // LAPACK zgeqrf/zlarft conventions). P0 is either the identity or the pre-pivoting
 // order: columns sorted once by decreasing initial norm (ties by index). For the
 // column-graded products DQMC stabilises, (B...B U) diag(D), QR with pre-pivoting is
@@ -17,7 +17,7 @@
 // Per panel p, with one-panel look-ahead: workgroup 0 applies Q_p^H to panel p+1's columns
 // and factors panel p+1 in registers (zlarfg per column, applied to the rest of the panel,
 // with the zlarft inner products formed along the way) while the other workgroups apply
-// Q_p^H to the columns beyond (one wave per column); one group barrier per panel.
+// Q_p^H to the columns beyond.
 #include "chain.hpp"
 
 namespace dqmc {
@@ -65,6 +65,639 @@ __device__ inline void stage_panel(cplx* P, const gcplx* A, const int* perm, int
   }
 }
 
+// ---------------------------------------------------------------------------
+// k_qr_pipe<RQ>: the blocked QR with 8-column panels, RQ = ceil(nmax / 256) rows per thread.
+//
+// What bounds it is workgroup 0's chain of panels: apply panel p to panel p+1's columns, factor
+// them, publish. The trailing updates run on the other workgroups and only have to keep up, so
+// no barrier over the chain group is taken per panel. Instead
+//   * block q (columns 8q .. 8q+7) belongs to workgroup 1 + q mod (W-1) for the whole
+//     factorisation; its owner applies the panels to it in order;
+//   * workgroup 0 publishes each panel (V in A, T in qr_Tf) by flags[0] = number of panels done;
+//   * the owner of block p+2 publishes it after applying panel p (flags[1 + block]); workgroup
+//     0 needs it one panel later and loads it while it writes panel p+1 back.
+// With one group barrier per panel (all workgroups waiting for all) the loads, the barrier and
+// the error-word read it took were about a third of a panel's time.
+//
+// A block is held as the C operand of v_mfma_f64_16x16x4: the 16 columns of a tile are the real
+// (0-7) and imaginary (8-15) parts of the block's 8 columns, lane (li, lk) of wave w holds rows
+// 16 (w + 4 tt) + 4 v + lk, column li. In that layout element v of a tile is also the B operand
+// of k-step v of the same rows, so
+//   [Vr Vi]^T [Xr Xi] (16 x 16, all four real products of V^H X at full tile use) and
+//   X -= [Vr Vi] [[Zr Zi] [-Zi Zr]]
+// take one MFMA per four rows each and no cross-lane sums; the vector form spent more time in
+// its butterflies and lane broadcasts than in the products. For the column steps the panel moves
+// through LDS (the buffer of V, free by then) to rows per thread, row off + tid + 256 q with
+// off = n - 256 RQ: the first rows die first and finished rows are skipped.
+//
+// Measured (one chain, default workgroups, us per factorisation, one group barrier per panel and
+// vector updates -> this): n = 64 163 -> 77, n = 256 631 -> 350, n = 400 1008 -> 730, n = 576
+// 1850 -> 1320, n = 1024 5000 -> 3650. A panel at n = 400 takes 33,800 cycles: 15,700 in the eight
+// column steps, 4,600 writing it back, 3,700 in V^H X, 3,300 for the next block's flag and loads,
+// 2,100 each in the update, the move to rows and the wait for the loads.
+// ---------------------------------------------------------------------------
+// Bounded wait of a whole workgroup for *f >= want: thread 0 polls (relaxed loads, one acquire
+// fence after the last; `seen` is a value it has loaded before), everyone learns the outcome
+// through LDS. false: the wait timed out here
+// or in another workgroup of the chain.
+__device__ inline unsigned flag_load(const unsigned* f) {
+  return __hip_atomic_load((const __attribute__((address_space(1))) unsigned*)f, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool wait_flag(const unsigned* f, unsigned want, unsigned seen, int* error, int* s_fail) {
+  if (threadIdx.x == 0) {
+    int fail = 0;
+    long long spins = 0;
+    for (; seen < want; seen = flag_load(f)) {
+      if ((++spins & 31) == 0) {
+        if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+          fail = 1;
+          break;
+        }
+        if (spins > kSpinLimit) {
+          __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          fail = 1;
+          break;
+        }
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    *s_fail = fail;
+  }
+  __syncthreads();
+  return *s_fail == 0;
+}
+// this wave's outstanding global stores have completed (vmcnt(0), no wait for the LDS)
+__device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// one thread: publish *f = v after a barrier that every wave entered with its stores complete
+// (write-through stores in place of the release fence cost more than the write-back: 8-byte
+// agent-scope stores held workgroup 0 for 8,000 cycles a panel)
+__device__ inline void set_flag(unsigned* f, unsigned v) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  __hip_atomic_store((__attribute__((address_space(1))) unsigned*)f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// sqrt(s) and 1 / sqrt(s) of a normal s > 0: Goldschmidt's iteration from the hardware estimate,
+// then one residual correction of each. One chain of ten dependent operations in place of a
+// square root followed by a division.
+__device__ inline void sqrt_rsqrt(double s, double& root, double& inv) {
+  const double y = __builtin_amdgcn_rsq(s);
+  double g = s * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  root = fma(fma(-g, g, s), h, g);
+  const double i0 = h + h;
+  inv = fma(i0, fma(-i0, root, 1.0), i0);
+}
+// 1 / x of a normal x: two Newton steps from the hardware estimate
+__device__ inline double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+
+template <int RQ>
+__global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef Ar, VecRef Dr, int prepivot, int ps,
+                                                 const int* bmap) {
+  constexpr int NB = 8, V = 2 * NB, LS = 2;  // V doubles per butterfly; after it, lane l holds value l >> LS
+  constexpr int TT = 4 * RQ;                 // 16-row tiles per wave
+  // grid (W, chains), or with a block map a 1-D grid where block b serves chain bmap[b] & 0xFFFF
+  // as workgroup (bmap[b] >> 16) & 0xFF of (bmap[b] >> 24) (workgroup counts per chain)
+  const int bm = bmap ? bmap[blockIdx.x] : 0;
+  const ChainDesc& c = chains[bmap ? (bm & 0xFFFF) : blockIdx.y];
+  const int n = c.n;
+  const int W = bmap ? (bm >> 24) & 0xFF : gridDim.x, w = bmap ? (bm >> 16) & 0xFF : blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = 4;
+  const int li = lane & 15, lk = lane >> 4, lu = li & 7, lim = li >> 3;
+  gcplx* A = gp(matptr(c, Ar));
+  gdouble* D = gp(vecptr(c, Dr));
+  // (every pointer of the descriptor once: a store could change it for all the compiler knows, and
+  // each re-read waits for every load and store in flight)
+  gcplx *Tf = gp(c.qr_Tf), *taug = gp(c.qr_tau);
+  unsigned* flags = c.qr_flags;
+  int* err = c.error;
+  const GroupSync g{c.bar_count, c.bar_gen, c.error, (unsigned int)W};
+  const int nblk = (n + NB - 1) / NB;
+  const int off = n - 256 * RQ;
+  // with many columns per trailing workgroup (at least 128 at the start) a wave takes 16 of them
+  // at a time instead of the workgroup 8: no barriers, but X streams from memory twice
+  const bool mt = W > 1 && n >= 128 * (W - 1);
+
+  extern __shared__ double smem[];
+  cplx* P = reinterpret_cast<cplx*>(smem);  // [NB][ps] panel V (rows k0..n-1 used, row r at 16 + r)
+  // [4][2][64] per-wave partial W of the tile form; [4][8][16] W of the 16-column trailing update
+  double* part = reinterpret_cast<double*>(P + (size_t)NB * ps);
+  cplx* wscr = reinterpret_cast<cplx*>(part);
+  __shared__ int perm[kQrMaxN], lpos[kQrMaxN];
+  __shared__ cplx Tl[NB * NB];     // Tl[j * NB + t] = T(j, t) of the panel in P
+  __shared__ cplx rowb[NB * NB];   // rows k0 .. k0+7 of the panel being factored: R and V
+  __shared__ double4 red[2][V];    // sums of a panel step, by step parity: one partial per wave
+  __shared__ cplx piv[2][NB];      // the pivot row of a panel step, by step parity
+  __shared__ int s_fail;
+
+  // ---- the flags of this factorisation, visible to all before the first wait
+  if (w == 0)
+    for (int e = tid; e <= nblk; e += 256) __hip_atomic_store(flags + e, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // ---- column order
+  if (prepivot) {
+    for (int col = w + W * wave; col < n; col += W * nwaves) {
+      const gcplx* a = A + (size_t)col * n;
+      double acc = 0.0;
+      for (int k = lane; k < n; k += 64) acc += abs2(ld(a + k));
+      acc = wave_sum(acc);
+      if (lane == 0) gp(c.qr_vn)[col] = sqrt(acc);
+    }
+  }
+  wait_stores();
+  group_sync(g);
+  if (group_failed(g)) return;
+  if (prepivot) {
+    double* vn = reinterpret_cast<double*>(P);  // n doubles, before the panel buffer is used
+    for (int k = tid; k < n; k += blockDim.x) vn[k] = gp(c.qr_vn)[k];
+    __syncthreads();
+    for (int col = tid; col < n; col += blockDim.x) {
+      const double v = vn[col];
+      int r = 0;
+      for (int q = 0; q < n; ++q) {
+        const double u = vn[q];
+        r += (u > v || (u == v && q < col)) ? 1 : 0;
+      }
+      lpos[col] = r;
+    }
+    __syncthreads();
+    for (int col = tid; col < n; col += blockDim.x) perm[lpos[col]] = col;
+  } else {
+    for (int k = tid; k < n; k += blockDim.x) perm[k] = lpos[k] = k;
+  }
+  __syncthreads();
+
+  // Every V in P starts at LDS row 16 + k0 with 16 zero rows before it, so that the tile which
+  // straddles row k0 (tiles end at row n - 1, not at multiples of 16 from row 0) needs no masks:
+  // its rows before k0 meet zeros, and keep the finite values they have.
+  v4d X[TT];        // a block in tile layout
+  cplx x[RQ][NB];   // the panel being factored, rows per thread
+  // this thread's rows, re-read per panel: as loop invariants the unrolled addresses and masks
+  // below would be formed once and spill
+  int tr = off + 16 * wave + lk, ta = off + 16 * wave + li, tx = off + tid;
+  // first tile of this wave that reaches row k
+  auto first_tile = [&](int k) __attribute__((always_inline)) { return ((max(k - off, 0) >> 4) - wave + 3) >> 2; };
+
+  // the tiles of the block at logical column kc that reach row kr into X (columns past the last
+  // one repeat it: nothing reads them)
+  auto load_tiles = [&](int kc, int kr) __attribute__((always_inline)) {
+    const int kbc = min(NB, n - kc), t0 = first_tile(kr);
+    const gdouble* a = (const gdouble*)(A + (size_t)perm[kc + min(lu, kbc - 1)] * n) + lim;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      if (tt >= t0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) X[tt][v] = a[2 * max(tr + 64 * tt + 4 * v, 0)];
+      } else {
+        X[tt] = v4d{0.0, 0.0, 0.0, 0.0};  // (defined on every path: not live during the column steps)
+      }
+  };
+  auto store_tiles = [&](int kc, int kr) __attribute__((always_inline)) {
+    const int t0 = first_tile(kr);
+    gdouble* a = (gdouble*)(A + (size_t)perm[min(kc + lu, n - 1)] * n) + lim;
+    const int lo = lu < n - kc ? kr : n;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      if (tt >= t0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (tr + 64 * tt + 4 * v >= lo) a[2 * (tr + 64 * tt + 4 * v)] = X[tt][v];
+      }
+  };
+  // X <- (I - V T^H V^H) X with V (rows >= k0) in P and T in Tl
+  auto apply_tiles = [&](int k0) __attribute__((always_inline)) {
+    const int t0 = first_tile(k0);
+    v4d acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+    const double* pv = reinterpret_cast<const double*>(P + (size_t)lu * ps + 16 + tr) + lim;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      if (tt >= t0) {
+        acc0 = mfma4(pv[2 * (64 * tt)], X[tt][0], acc0);
+        acc1 = mfma4(pv[2 * (64 * tt + 4)], X[tt][1], acc1);
+        acc0 = mfma4(pv[2 * (64 * tt + 8)], X[tt][2], acc0);
+        acc1 = mfma4(pv[2 * (64 * tt + 12)], X[tt][3], acc1);
+      }
+    // Lane (li, lk): row l = lk (lk + 4 for w1) of W = V^H X, component li, from the products
+    // Vr Xr + Vi Xi (li < 8) and Vr Xi - Vi Xr (li >= 8); Vi's rows are 8 further down the tile,
+    // the other component is 8 lanes away. Then the sum over the waves.
+    const double o0 = dpp_move<0x128>(acc0[2] + acc1[2]), o1 = dpp_move<0x128>(acc0[3] + acc1[3]);  // row_ror:8
+    part[wave * 128 + lane] = (acc0[0] + acc1[0]) + (lim ? -o0 : o0);
+    part[wave * 128 + 64 + lane] = (acc0[1] + acc1[1]) + (lim ? -o1 : o1);
+    __syncthreads();
+    const double w0 = (part[lane] + part[128 + lane]) + (part[256 + lane] + part[384 + lane]);
+    const double w1 = (part[64 + lane] + part[192 + lane]) + (part[320 + lane] + part[448 + lane]);
+    // That is the B operand of Z = T^H W: [Zr Zi] = Tr^T [Wr Wi] + Ti^T [Wi -Wr], and element 0
+    // (1) of the product is row lk (lk + 4) of [Zr Zi], the B operand of the update
+    const cplx t0l = Tl[lk * NB + lu], t1l = Tl[(lk + 4) * NB + lu];
+    const double x0 = dpp_move<0x128>(w0), x1 = dpp_move<0x128>(w1);
+    v4d z = {0.0, 0.0, 0.0, 0.0};
+    z = mfma4(lim ? 0.0 : t0l.re, w0, z);
+    z = mfma4(lim ? 0.0 : t1l.re, w1, z);
+    z = mfma4(lim ? 0.0 : t0l.im, lim ? -x0 : x0, z);
+    z = mfma4(lim ? 0.0 : t1l.im, lim ? -x1 : x1, z);
+    // rows of [[Zr Zi] [-Zi Zr]], negated: k-steps 0, 1 (Vr) and 2, 3 (Vi)
+    const double y0 = dpp_move<0x128>(z[0]), y1 = dpp_move<0x128>(z[1]);
+    const double b0 = -z[0], b1 = -z[1], b2 = lim ? -y0 : y0, b3 = lim ? -y1 : y1;
+    const cplx* pa = P + (size_t)lk * ps + 16 + ta;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      if (tt >= t0) {
+        const cplx v0 = pa[64 * tt], v1 = pa[(size_t)4 * ps + 64 * tt];
+        X[tt] = mfma4(v0.re, b0, X[tt]);
+        X[tt] = mfma4(v1.re, b1, X[tt]);
+        X[tt] = mfma4(v0.im, b2, X[tt]);
+        X[tt] = mfma4(v1.im, b3, X[tt]);
+      }
+  };
+  // the published panel at k0 into P as the unit lower trapezoid V, every load before any store
+  auto stage_V = [&](int k0) __attribute__((always_inline)) {
+    const int q0 = max(k0 - off, 0) >> 8;
+    cplx y[RQ][NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const gcplx* a = A + (size_t)perm[k0 + t] * n;
+#pragma unroll
+      for (int q = 0; q < RQ; ++q)
+        if (q >= q0) {
+          const gcplx* src = a + max(tx + 256 * q, k0);
+          y[q][t].re = src->re;
+          y[q][t].im = src->im;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RQ; ++q)
+      if (q >= q0) {
+        const int r = tx + 256 * q;
+        if (r >= k0) {
+#pragma unroll
+          for (int t = 0; t < NB; ++t) {
+            P[(size_t)t * ps + 16 + r].re = r < k0 + t ? 0.0 : r == k0 + t ? 1.0 : y[q][t].re;
+            P[(size_t)t * ps + 16 + r].im = r <= k0 + t ? 0.0 : y[q][t].im;
+          }
+        }
+      }
+    if (tid >= 128) P[(size_t)((tid - 128) >> 4) * ps + k0 + (tid & 15)] = mk(0, 0);  // rows k0 - 16 .. k0 - 1
+  };
+  // the panel at k1, tiles of X that reach row kr, through P into x: rows >= k1 to x (zero before
+  // that; LDS row 0 is zero throughout), rows kr .. k1 - 1 of R to A
+  auto tiles_to_rows = [&](int k1, int kr) __attribute__((always_inline)) {
+    const int t0 = first_tile(kr);
+    double* pd = reinterpret_cast<double*>(P + (size_t)lu * ps + 16 + tr) + lim;
+    __syncthreads();  // every wave has read V
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      if (tt >= t0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) pd[2 * (64 * tt + 4 * v)] = X[tt][v];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const int r = tx + 256 * q;
+      const cplx* src = P + (r >= k1 ? 16 + r : 0);
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        x[q][t].re = src[(size_t)t * ps].re;
+        x[q][t].im = src[(size_t)t * ps].im;
+      }
+    }
+    const int t = tid >> 3, r = kr + (tid & 7);
+    if (tid < NB * NB && r < k1 && k1 + t < n) {
+      const cplx* src = P + (size_t)t * ps + 16 + r;
+      st(A + (size_t)perm[k1 + t] * n + r, mk(src->re, src->im));
+    }
+  };
+  // ---- the column steps of the panel at logical column k0, held in x. Per column t (zlarfg,
+  // then H^H on the columns after it):
+  //   the owner of the pivot row i = k0 + t moves it to LDS and clears its columns >= t, so rows
+  //   above the diagonal need no masks;
+  //   one butterfly sums |x_t|^2 and x_t^H a_u (u > t) over the rows below the pivot, plus
+  //   v_j^H x_t (j < t) for zlarft; after one barrier every thread forms beta, tau and
+  //   1 / (alpha - beta) from the same sums and updates its rows; wave 0 keeps row i of R and V;
+  //   column t of T (zlarft, forward and columnwise): S(j, t) = v_j^H v_t = conj(v_j(i)) +
+  //   v_j^H x_t / (alpha - beta), T(t, t) = tau, T(0:t, t) = -tau T(0:t, 0:t) S(0:t, t), lane j of
+  //   every 16 keeping row j, so that T is ready with the last column.
+  // A step is one wave per SIMD working through a chain of dependent operations, about 200
+  // instructions: its length is what counts, so sums, pivot entries and factors stay one per lane
+  // until the broadcasts, the square root also gives 1 / beta, and the factors of the update
+  // need no other division.
+  cplx trow[NB];   // lane j (of 16): row j of T
+  auto column_steps = [&](int k0) __attribute__((always_inline)) {
+    const int q0 = max(k0 - off, 0) >> 8;  // rows of x[q], q < q0, are finished
+    const int kl = lane & 15;
+    static_for<0, NB>([&](auto tc) __attribute__((always_inline)) {
+      constexpr int t = decltype(tc)::value, par = t & 1;
+      const int i = k0 + t;
+      double v[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = 0.0;
+#pragma unroll
+      for (int q = 0; q < RQ; ++q)
+        if (q >= q0) {
+          if (tx + 256 * q == i) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+              piv[par][u].re = x[q][u].re;
+              piv[par][u].im = x[q][u].im;
+            }
+#pragma unroll
+            for (int u = t; u < NB; ++u) x[q][u] = mk(0, 0);
+          }
+          const cplx xt = x[q][t];
+          v[0] = fma(xt.re, xt.re, fma(xt.im, xt.im, v[0]));
+#pragma unroll
+          for (int u = t + 1; u < NB; ++u) {
+            const int e = 1 + 2 * (u - t - 1);
+            v[e] = fma(xt.re, x[q][u].re, fma(xt.im, x[q][u].im, v[e]));
+            v[e + 1] = fma(xt.re, x[q][u].im, fma(-xt.im, x[q][u].re, v[e + 1]));
+          }
+#pragma unroll
+          for (int j = 0; j < t; ++j) {  // v_j^H x_t below the pivot, for S(j, t)
+            const int e = 1 + 2 * (NB - 1 - t) + 2 * j;
+            v[e] = fma(x[q][j].re, xt.re, fma(x[q][j].im, xt.im, v[e]));
+            v[e + 1] = fma(x[q][j].re, xt.im, fma(-x[q][j].im, xt.re, v[e + 1]));
+          }
+        }
+      wave_reduce_scatter<V>(v);
+      if ((lane & ((1 << LS) - 1)) == 0) reinterpret_cast<double*>(&red[par][lane >> LS])[wave] = v[0];
+      __syncthreads();
+      // lane k of every row of 16: its complex sum, of column t+1+k (k < NB-1-t) or of reflector
+      // k - (NB-1-t), and that column's entry of the pivot row
+      const int k = min(kl, NB - 2), m = k < NB - 1 - t ? t + 1 + k : k - (NB - 1 - t);
+      const double4 q0s = red[par][0], qr = red[par][1 + 2 * k], qi = red[par][2 + 2 * k];
+      const cplx alpha = mk(piv[par][t].re, piv[par][t].im), pm = mk(piv[par][m].re, piv[par][m].im);
+      const double xsq = (q0s.x + q0s.y) + (q0s.z + q0s.w);
+      const cplx raw = mk((qr.x + qr.y) + (qr.z + qr.w), (qi.x + qi.y) + (qi.z + qi.w));
+      // zlarfg: H^H (alpha, x) = (beta, 0), v = (1, x / d), d = alpha - beta, tau = -d / beta.
+      // With nothing below the pivot and a real alpha H = I: 1 / beta is taken as 0, which makes
+      // tau and f zero, and x is zero whatever d is.
+      const bool none = xsq == 0.0 && alpha.im == 0.0;
+      const double ssq = fma(alpha.re, alpha.re, fma(alpha.im, alpha.im, xsq));
+      double nrm, inv;
+      sqrt_rsqrt(none ? 1.0 : ssq, nrm, inv);
+      const double ib = none ? 0.0 : -copysign(inv, alpha.re);
+      const double beta = none ? alpha.re : -copysign(nrm, alpha.re);
+      const cplx d = mk(alpha.re + copysign(nrm, alpha.re), alpha.im);
+      // v^H a_u = a_u(i) + conj(1 / d) x_t^H a_u, times conj(tau) = -conj(d) / beta:
+      // f = -(conj(d) a_u(i) + x_t^H a_u) / beta, which needs no division by |d|^2
+      cplx fl = raw;
+      cfma_cj(fl, d, pm);
+      fl = mk(-ib * fl.re, -ib * fl.im);
+      const double id = recip(fma(d.re, d.re, d.im * d.im));  // |d|^2 <= 4 (|alpha|^2 + xsq)
+      const cplx sc = mk(d.re * id, -d.im * id), tau = mk(-d.re * ib, -d.im * ib);
+      cplx f[NB];
+      static_for<t + 1, NB>([&](auto uc) __attribute__((always_inline)) {
+        constexpr int u = decltype(uc)::value;
+        f[u] = mk(dpp_move<0x150 + (u - t - 1)>(fl.re), dpp_move<0x150 + (u - t - 1)>(fl.im));  // row_newbcast
+      });
+#pragma unroll
+      for (int q = 0; q < RQ; ++q)
+        if (q >= q0) {
+          const cplx vt = sc * x[q][t];
+#pragma unroll
+          for (int u = t + 1; u < NB; ++u) {
+            x[q][u].re = fma(-f[u].re, vt.re, fma(f[u].im, vt.im, x[q][u].re));
+            x[q][u].im = fma(-f[u].re, vt.im, fma(-f[u].im, vt.re, x[q][u].im));
+          }
+          x[q][t] = vt;
+        }
+      if (tid < NB) {  // row i of R (columns >= t) and of V (columns < t)
+        const bool diag = tid == NB - 1, r = k < NB - 1 - t;
+        rowb[t * NB + (diag ? t : m)].re = diag ? beta : r ? pm.re - fl.re : pm.re;
+        rowb[t * NB + (diag ? t : m)].im = diag ? 0.0 : r ? pm.im - fl.im : pm.im;
+      }
+      cplx sj = conj(pm), acc = mk(0, 0);
+      cfma(sj, sc, raw);
+      static_for<0, t>([&](auto lc) __attribute__((always_inline)) {
+        constexpr int l = decltype(lc)::value, src = NB - 1 - t + l;
+        cfma(acc, trow[l], mk(dpp_move<0x150 + src>(sj.re), dpp_move<0x150 + src>(sj.im)));
+      });
+      acc = -(tau * acc);  // (zero on the lanes j >= t)
+      trow[t].re = kl == t ? tau.re : acc.re;
+      trow[t].im = kl == t ? tau.im : acc.im;
+    });
+  };
+  // ---- the factored panel p at k0: V to P, T to Tl; rows >= k0 to A, tau, D and T to global memory
+  auto write_panel = [&](int k0, int p) __attribute__((always_inline)) {
+    const int kb = min(NB, n - k0);
+    gcplx* Tg = Tf + (size_t)p * NB * NB;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      gcplx* a = A + (size_t)perm[k0 + min(t, kb - 1)] * n;
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) {
+        const int r = tx + 256 * q;
+        const cplx xv = x[q][t];
+        if (r >= k0 + NB) {
+          P[(size_t)t * ps + 16 + r].re = xv.re;
+          P[(size_t)t * ps + 16 + r].im = xv.im;
+        }
+        if (t < kb && r >= k0 + NB) st(a + r, xv);
+      }
+    }
+    if (wave == 3) {  // lane (t, u): rows k0 .. k0+7
+      const int t = lane >> 3, u = lane & 7;
+      const cplx e = mk(rowb[lane].re, rowb[lane].im);
+      if (k0 + t < n) {
+        P[(size_t)u * ps + 16 + k0 + t].re = u < t ? e.re : u == t ? 1.0 : 0.0;
+        P[(size_t)u * ps + 16 + k0 + t].im = u < t ? e.im : 0.0;
+        if (u < kb) st(A + (size_t)perm[k0 + u] * n + k0 + t, e);
+        if (t == u) D[k0 + t] = fabs(e.re);
+      }
+    }
+    if (tid >= 64 && tid < 192) P[(size_t)((tid - 64) >> 4) * ps + k0 + (tid & 15)] = mk(0, 0);  // rows k0 - 16 .. k0 - 1
+    if (tid < NB) {  // row tid of T
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        const bool ok = t < kb && tid < kb;
+        const cplx v = mk(ok ? trow[t].re : 0.0, ok ? trow[t].im : 0.0);
+        Tl[tid * NB + t].re = v.re;
+        Tl[tid * NB + t].im = v.im;
+        st(Tg + tid * NB + t, v);
+      }
+    }
+    if (tid < kb) {  // tau: T's diagonal
+      const cplx v = mk(Tl[tid * (NB + 1)].re, Tl[tid * (NB + 1)].im);
+      st(taug + k0 + tid, v);
+    }
+  };
+  const int ws = W == 1 ? 1 : W - 1;  // workgroups of the trailing blocks
+  // Trailing update of panel p (rows >= k0) on the matrix cores (mt), for workgroups w >= 1: the
+  // own blocks from fb on in tiles of two blocks, 16 columns, tile q to wave q mod 4.
+  // Per tile: W = V^H X (K = rows, A(i, k) = conj V(r, i), B(k, j) = X(r, col_j)), then
+  // Z = T^H W with the vector units (lane (j, k) forms Z(k, j) and Z(k + 4, j), exactly its B
+  // operands of the second product), then X -= V Z in 16-row tiles. X streams from global
+  // memory twice (loads four steps ahead); V comes from P (stride ps: conflict-free). When fb is
+  // the block workgroup 0 waits for, wave 0 publishes it after the tile that holds it.
+  auto trailing_mfma = [&](int k0, int fb, int need) __attribute__((always_inline)) {
+    const int vi = min(li, NB - 1);
+    const int nbw = fb < nblk ? (nblk - 1 - fb) / ws + 1 : 0;
+    const int nst = (n - k0) >> 2;
+    cplx* wsc = wscr + wave * 128;
+    for (int q = wave; 2 * q < nbw; q += nwaves) {
+      const int j = 2 * q + (li >> 3);
+      const int cl = (fb + j * ws) * NB + (li & 7);
+      const bool valid = j < nbw && cl < n;
+      gcplx* a = A + (size_t)perm[valid ? cl : n - 1] * n;
+      v4d wr = {0.0, 0.0, 0.0, 0.0}, wi = {0.0, 0.0, 0.0, 0.0};
+      constexpr int PF = 8;  // k-steps of X loaded ahead of the products
+      cplx xb[PF];
+#pragma unroll
+      for (int u = 0; u < PF; ++u) xb[u] = ld(a + k0 + 4 * min(u, nst - 1) + lk);
+      for (int s0 = 0; s0 < nst; s0 += PF) {
+        cplx xc[PF];
+#pragma unroll
+        for (int u = 0; u < PF; ++u) xc[u] = xb[u];
+#pragma unroll
+        for (int u = 0; u < PF; ++u) xb[u] = ld(a + k0 + 4 * min(s0 + PF + u, nst - 1) + lk);
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+          if (s0 + u < nst) {
+            const cplx v = P[(size_t)vi * ps + 16 + k0 + 4 * (s0 + u) + lk];
+            const double vr = li < NB ? v.re : 0.0, vm = li < NB ? v.im : 0.0;
+            const double xr = valid ? xc[u].re : 0.0, xm = valid ? xc[u].im : 0.0;
+            // W += V^H X: re += Vr Xr + Vi Xi, im += Vr Xi - Vi Xr
+            wr = mfma4(vr, xr, wr);
+            wi = mfma4(vr, xm, wi);
+            wr = mfma4(vm, xm, wr);
+            wi = mfma4(-vm, xr, wi);
+          }
+        }
+      }
+      // lane (li, lk) holds W(lk, li) and W(lk + 4, li); every lane needs W(:, li)
+      wsc[lk * 16 + li] = mk(wr[0], wi[0]);
+      wsc[(lk + 4) * 16 + li] = mk(wr[1], wi[1]);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      cplx z0 = mk(0, 0), z1 = mk(0, 0);
+#pragma unroll
+      for (int l = 0; l < NB; ++l) {
+        const cplx wl = wsc[l * 16 + li];
+        cfma_cj(z0, Tl[l * NB + lk], wl);
+        cfma_cj(z1, Tl[l * NB + lk + 4], wl);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // W read before the next tile writes it
+      // X -= V Z over 16-row tiles: element v of lane (li, lk) is row r0 + lk + 4 v, column li
+      cplx cb[4], cn[4];  // the next two row tiles' X, loaded ahead
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        cb[v] = ld(a + min(k0 + lk + 4 * v, n - 1));
+        cn[v] = ld(a + min(k0 + 16 + lk + 4 * v, n - 1));
+      }
+      for (int r0 = k0; r0 < n; r0 += 16) {
+        v4d dr, di;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          dr[v] = cb[v].re;
+          di[v] = cb[v].im;
+          cb[v] = cn[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) cn[v] = ld(a + min(r0 + 32 + lk + 4 * v, n - 1));
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const int ra = r0 + li;
+          const cplx a0 = P[(size_t)(4 * ks + lk) * ps + 16 + min(ra, n - 1)];
+          const double ar = ra < n ? a0.re : 0.0, am = ra < n ? a0.im : 0.0;
+          const cplx z = ks ? z1 : z0;
+          // X -= V Z: re += -Vr Zr + Vi Zi, im += -Vr Zi - Vi Zr
+          dr = mfma4(-ar, z.re, dr);
+          di = mfma4(-ar, z.im, di);
+          dr = mfma4(am, z.im, dr);
+          di = mfma4(-am, z.re, di);
+        }
+        if (valid) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int row = r0 + lk + 4 * v;
+            if (row < n) {
+              st(a + row, mk(dr[v], di[v]));
+            }
+          }
+        }
+      }
+      if (q == 0 && fb == need) {  // (tile 0 is wave 0's: the wave publishes its own stores)
+        wait_stores();
+        if (lane == 0) set_flag(flags + 1 + need, 1u);
+      }
+    }
+  };
+
+  // the rows before row 0: a panel's rows per thread reach them, and they have to be finite
+  if (tid < 128) P[(size_t)(tid >> 4) * ps + (tid & 15)] = mk(0, 0);
+  int own = w - 1;
+  bool loaded = false;  // the next block's tiles are already in X
+  for (int p = -1, k1 = 0; k1 < n; ++p, k1 += NB) {  // apply panel p, factor panel p+1 at k1
+    const int k0 = max(k1 - NB, 0);
+    asm volatile("" : "+v"(tr), "+v"(ta), "+v"(tx));
+    // the first own block beyond panel p+1 (workgroup 0 owns none unless it is alone)
+    int fb = nblk;
+    if (W > 1 && w != 0) loaded = true;
+    if (W == 1) {
+      fb = p < 0 ? nblk : p + 2;
+    } else if (w != 0) {
+      if (p < 0) continue;
+      while (own < p + 2) own += ws;
+      fb = own;
+      if (fb >= nblk) return;  // no block of this workgroup is left
+      if (!mt) load_tiles(fb * NB, k0);  // (own columns: before the panel is there)
+      if (!wait_flag(flags, (unsigned)(p + 1), 0u, err, &s_fail)) return;
+      stage_V(k0);
+      if (tid < NB * NB) Tl[tid] = ld(Tf + (size_t)p * NB * NB + tid);
+      __syncthreads();
+      if (mt) {
+        trailing_mfma(k0, fb, p + 2);
+        continue;
+      }
+    }
+    // the own trailing blocks first, then, on workgroup 0, panel p+1 itself, which stays in X
+    for (;; fb += ws) {
+      const bool next = fb >= nblk;
+      if (next && w != 0) break;
+      const int kc = next ? k1 : fb * NB;
+      if (!loaded) load_tiles(kc, k0);
+      if (p >= 0) apply_tiles(k0);
+      if (next) break;
+      store_tiles(kc, k0);
+      if (W > 1 && fb == p + 2) {
+        wait_stores();
+        __syncthreads();
+        if (tid == 0) set_flag(flags + 1 + fb, 1u);
+      }
+      loaded = false;
+    }
+    if (w != 0) continue;
+    tiles_to_rows(k1, k0);
+    const bool fetch = W > 1 && k1 + NB < n, need = fetch && p >= 0;
+    column_steps(k1);
+    if (need) {
+      // block p+2 carries panel p; its owner has had a panel's time to bring it up to date
+      if (!wait_flag(flags + 1 + (p + 2), 1u, 0u, err, &s_fail)) return;
+    } else {
+      __syncthreads();
+    }
+    if (fetch) load_tiles(k1 + NB, k1);
+    loaded = fetch;
+    write_panel(k1, p + 1);
+    wait_stores();
+    __syncthreads();
+    if (W > 1 && tid == 192) set_flag(flags, (unsigned)(p + 2));
+  }
+  if (w == 0) {
+    for (int k = tid; k < n; k += blockDim.x) {
+      gp(c.qr_perm)[k] = perm[k];
+      gp(c.qr_lpos)[k] = lpos[k];
+    }
+  }
+}
+
+// k_qr_blocked<NB, RQ>: the same factorisation by one group barrier per panel, on the vector
+// units; it serves 16-column panels (twice the panel does not fit k_qr_pipe's tiles).
 // Workgroup 0's panel work keeps the panel in registers: thread tid owns rows r = tid + 256 q
 // (q < RQ) of the NB panel columns. Every cross-thread sum goes through one butterfly
 // reduce-scatter per wave and one LDS exchange, so a panel column costs one barrier.
@@ -85,14 +718,9 @@ __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, Mat
   gcplx* A = gp(matptr(c, Ar));
   gdouble* D = gp(vecptr(c, Dr));
   const GroupSync g{c.bar_count, c.bar_gen, c.error, (unsigned int)W};
-  // the matrix-core trailing update pays off when each trailing workgroup holds many columns
-  // (at least 128 at the start); with few, its tiles are half empty and the block that panel
-  // p+2 needs sits on one wave
-  const bool mt = NB == 8 && W > 1 && n >= 128 * (W - 1);
 
   extern __shared__ double smem[];
   cplx* P = reinterpret_cast<cplx*>(smem);  // [NB][ps] panel V (rows k0..n-1 used)
-  cplx* wscr = P + (size_t)NB * ps;          // [4][8][16] per-wave W of the matrix-core trailing update
   __shared__ int perm[kQrMaxN], lpos[kQrMaxN];
   __shared__ cplx Tl[NB * NB];  // Tl[j * NB + t] = T(j, t)
   __shared__ cplx taul[NB];
@@ -381,102 +1009,6 @@ __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, Mat
     }
   };
   const int ws = W == 1 ? 1 : W - 1, w0 = W == 1 ? 0 : 1;  // trailing workgroups, first one
-  // Trailing update of panel p (rows >= k0) on the matrix cores (mt), for workgroups w >= 1: this workgroup's blocks (block b of the columns beyond k1 + NB goes to
-  // workgroup 1 + b mod (W-1)) in tiles of two blocks, 16 columns, tile q to wave q mod 4.
-  // Per tile: W = V^H X (K = rows, A(i, k) = conj V(r, i), B(k, j) = X(r, col_j)), then
-  // Z = T^H W with the vector units (lane (j, k) forms Z(k, j) and Z(k + 4, j), exactly its B
-  // operands of the second product), then X -= V Z in 16-row tiles. X streams from global
-  // memory twice (loads four steps ahead); V comes from P (stride ps: conflict-free).
-  auto trailing_mfma = [&](int k0, int k1) __attribute__((always_inline)) {
-    const int li = lane & 15, lk = lane >> 4, vi = min(li, NB - 1);
-    const int nbt = (n - k1 - NB + NB - 1) / NB;  // blocks beyond panel p+1
-    const int nbw = nbt > w - 1 ? (nbt - (w - 1) + ws - 1) / ws : 0;
-    const int nst = (n - k0) >> 2;
-    cplx* wsc = wscr + wave * 128;
-    for (int q = wave; 2 * q < nbw; q += nwaves) {
-      const int j = 2 * q + (li >> 3);
-      const int cl = k1 + NB + ((w - 1) + j * ws) * NB + (li & 7);
-      const bool valid = j < nbw && cl < n;
-      gcplx* a = A + (size_t)perm[valid ? cl : min(k1 + NB, n - 1)] * n;
-      v4d wr = {0.0, 0.0, 0.0, 0.0}, wi = {0.0, 0.0, 0.0, 0.0};
-      constexpr int PF = 8;  // k-steps of X loaded ahead of the products
-      cplx xb[PF];
-#pragma unroll
-      for (int u = 0; u < PF; ++u) xb[u] = ld(a + k0 + 4 * min(u, nst - 1) + lk);
-      for (int s0 = 0; s0 < nst; s0 += PF) {
-        cplx xc[PF];
-#pragma unroll
-        for (int u = 0; u < PF; ++u) xc[u] = xb[u];
-#pragma unroll
-        for (int u = 0; u < PF; ++u) xb[u] = ld(a + k0 + 4 * min(s0 + PF + u, nst - 1) + lk);
-#pragma unroll
-        for (int u = 0; u < PF; ++u) {
-          if (s0 + u < nst) {
-            const cplx v = P[(size_t)vi * ps + k0 + 4 * (s0 + u) + lk];
-            const double vr = li < NB ? v.re : 0.0, vm = li < NB ? v.im : 0.0;
-            const double xr = valid ? xc[u].re : 0.0, xm = valid ? xc[u].im : 0.0;
-            // W += V^H X: re += Vr Xr + Vi Xi, im += Vr Xi - Vi Xr
-            wr = mfma4(vr, xr, wr);
-            wi = mfma4(vr, xm, wi);
-            wr = mfma4(vm, xm, wr);
-            wi = mfma4(-vm, xr, wi);
-          }
-        }
-      }
-      // lane (li, lk) holds W(lk, li) and W(lk + 4, li); every lane needs W(:, li)
-      wsc[lk * 16 + li] = mk(wr[0], wi[0]);
-      wsc[(lk + 4) * 16 + li] = mk(wr[1], wi[1]);
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      cplx z0 = mk(0, 0), z1 = mk(0, 0);
-#pragma unroll
-      for (int l = 0; l < NB; ++l) {
-        const cplx wl = wsc[l * 16 + li];
-        cfma_cj(z0, Tl[l * NB + lk], wl);
-        cfma_cj(z1, Tl[l * NB + lk + 4], wl);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // W read before the next tile writes it
-      // X -= V Z over 16-row tiles: element v of lane (li, lk) is row r0 + lk + 4 v, column li
-      cplx cb[4], cn[4];  // the next two row tiles' X, loaded ahead
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        cb[v] = ld(a + min(k0 + lk + 4 * v, n - 1));
-        cn[v] = ld(a + min(k0 + 16 + lk + 4 * v, n - 1));
-      }
-      for (int r0 = k0; r0 < n; r0 += 16) {
-        v4d dr, di;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          dr[v] = cb[v].re;
-          di[v] = cb[v].im;
-          cb[v] = cn[v];
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) cn[v] = ld(a + min(r0 + 32 + lk + 4 * v, n - 1));
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const int ra = r0 + li;
-          const cplx a0 = P[(size_t)(4 * ks + lk) * ps + min(ra, n - 1)];
-          const double ar = ra < n ? a0.re : 0.0, am = ra < n ? a0.im : 0.0;
-          const cplx z = ks ? z1 : z0;
-          // X -= V Z: re += -Vr Zr + Vi Zi, im += -Vr Zi - Vi Zr
-          dr = mfma4(-ar, z.re, dr);
-          di = mfma4(-ar, z.im, di);
-          dr = mfma4(am, z.im, dr);
-          di = mfma4(-am, z.re, di);
-        }
-        if (valid) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = r0 + lk + 4 * v;
-            if (row < n) {
-              a[row].re = dr[v];
-              a[row].im = di[v];
-            }
-          }
-        }
-      }
-    }
-  };
   // One-panel look-ahead: while every other workgroup applies panel p to the columns beyond
   // panel p+1 (in blocks of NB logical columns, block b to workgroup 1 + b mod (W-1)),
   // workgroup 0 applies it to panel p+1's columns and factors panel p+1, so each panel costs
@@ -491,14 +1023,12 @@ __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, Mat
         for (int e = tid; e < NB * NB; e += blockDim.x) Tl[e] = ld(gp(c.qr_Tf) + (size_t)p * NB * NB + e);
         __syncthreads();
       }
-      if (w == 0 || NB != 8 || !mt) load_pj(k0);
+      load_pj(k0);
     }
     // this workgroup's blocks: trailing ones first (kc >= k1 + NB), then, on workgroup 0,
     // panel p+1 itself, which stays in x for the factorisation
     if (p < 0) {
       if (w == 0) load_regs(0, min(NB, n), 0);
-    } else if (NB == 8 && w != 0 && mt) {
-      trailing_mfma(k0, k1);
     } else {
       for (int kc = (w >= w0) ? k1 + NB + (w - w0) * NB : n;; kc += ws * NB) {
         const bool next = kc >= n;
@@ -1029,18 +1559,15 @@ int qr_panel_width(int nmax) {
   return 8;
 }
 
-template <int NB, int RQ>
-hipError_t launch_qr_blocked_nb(hipStream_t s, const ChainDesc* chains, int nchains, int nmax, MatRef A, VecRef D,
-                                int prepivot, int wg, const int* bmap, int nblocks) {
-  int ps = mfma_ld(nmax);
-  const size_t lds = ((size_t)NB * ps + 4 * 128) * sizeof(cplx);
+static hipError_t launch_qr_kernel(const void* fn, size_t lds, hipStream_t s, const ChainDesc* chains, int nchains,
+                                   int ps, MatRef A, VecRef D, int prepivot, int wg, const int* bmap, int nblocks) {
   {
-    hipError_t e = ensure_dynamic_lds((const void*)k_qr_blocked<NB, RQ>, lds);
+    hipError_t e = ensure_dynamic_lds(fn, lds);
     if (e != hipSuccess) return e;
   }
   void* args[] = {(void*)&chains, (void*)&A, (void*)&D, (void*)&prepivot, (void*)&ps, (void*)&bmap};
   const dim3 grid = bmap ? dim3(nblocks, 1) : dim3(wg, nchains);
-  hipError_t e = hipLaunchCooperativeKernel((const void*)k_qr_blocked<NB, RQ>, grid, dim3(256), args, lds, s);
+  hipError_t e = hipLaunchCooperativeKernel(fn, grid, dim3(256), args, lds, s);
   if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
@@ -1049,15 +1576,18 @@ hipError_t launch_qr_blocked(hipStream_t s, const ChainDesc* chains, int nchains
                              int prepivot, int wg, int nb, const int* bmap, int nblocks) {
   if (nmax > kQrMaxN) return hipErrorInvalidValue;
   if (nb == 0) nb = qr_panel_width(nmax);
+  int ps = mfma_ld(nmax);
   if (nb == 16 && nmax <= 512)
-    return launch_qr_blocked_nb<16, 2>(s, chains, nchains, nmax, A, D, prepivot, wg, bmap, nblocks);
-  if (nb == 8 && nmax <= 512)
-    return launch_qr_blocked_nb<8, 2>(s, chains, nchains, nmax, A, D, prepivot, wg, bmap, nblocks);
-  // three rows per thread up to n = 768 (four spill the register-resident panel)
-  if (nb == 8 && nmax <= 768)
-    return launch_qr_blocked_nb<8, 3>(s, chains, nchains, nmax, A, D, prepivot, wg, bmap, nblocks);
-  if (nb == 8) return launch_qr_blocked_nb<8, 4>(s, chains, nchains, nmax, A, D, prepivot, wg, bmap, nblocks);
-  return hipErrorInvalidValue;
+    return launch_qr_kernel((const void*)k_qr_blocked<16, 2>, (size_t)16 * ps * sizeof(cplx), s, chains, nchains, ps, A,
+                            D, prepivot, wg, bmap, nblocks);
+  if (nb != 8) return hipErrorInvalidValue;
+  const void* fn = nmax <= 256   ? (const void*)k_qr_pipe<1>
+                   : nmax <= 512 ? (const void*)k_qr_pipe<2>
+                   : nmax <= 768 ? (const void*)k_qr_pipe<3>
+                                 : (const void*)k_qr_pipe<4>;
+  ps = mfma_ld(nmax + 16);
+  return launch_qr_kernel(fn, ((size_t)8 * ps + 512) * sizeof(cplx), s, chains, nchains, ps, A, D, prepivot, wg, bmap,
+                          nblocks);
 }
 
 template <int NB, int CB>

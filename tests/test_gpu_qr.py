@@ -1,0 +1,43 @@
+"""Blocked QR (k_qr_pipe): factors at the sizes and workgroup counts where its tiles, rows per
+thread and block ownership change.
+
+n = 4 L^2 covers one to four rows per thread (up to n = 256, 512, 768, 1024), last panels of four
+columns (n = 36, 100, 196, 324, 676) and tiles that straddle row 0 (n not a multiple of 16).
+Workgroup counts: one (no flags), two (every trailing block on one workgroup), three and five
+(blocks dealt round robin; the 16-column trailing update where a workgroup holds 128 columns and
+more), and the default.
+
+Tolerances: Householder QR is column-wise backward stable, |A - QR|_j <= c n eps |A_j| with a
+small c, and |Q^H Q - I| <= c n eps; c = 8, eps = 2.2e-16.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd():
+    import dqmc_amd
+    dqmc_amd.load()
+    return dqmc_amd
+
+
+EPS = 2.220446049250313e-16
+
+
+@pytest.mark.parametrize("L", [3, 4, 5, 7, 8, 9, 10, 12, 13, 14, 16])
+def test_blocked_qr_sizes_and_workgroups(amd, L):
+    n = 4 * L * L
+    rng = np.random.default_rng(L)
+    A = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))) * np.exp(rng.uniform(-20, 20, n))
+    c = amd.DQMC(amd.Params(L=L, slices=20, hoppings=(1.0, 0.5, 0.5, 1.0), lam=1.0, r=1.0))
+    for wg in (0, 1, 2, 3, 5):
+        print("blocked QR n=%d workgroups %d" % (n, wg), flush=True)
+        if wg:
+            c.set_groups(wg_qr=wg)
+        U, D, T = c.decompose_udt_prepivoted(A)
+        assert np.abs(U.conj().T @ U - np.eye(n)).max() <= 8 * n * EPS
+        assert (np.abs((U * D) @ T - A) / np.linalg.norm(A, axis=0)).max() <= 8 * n * EPS
+        assert np.all(D > 0)
+    c.close()
