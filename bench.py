@@ -196,8 +196,8 @@ def grad_measure(amd, evals, warmup):
 
     The warm-up evaluations run with every kernel class timed by HIP events on the chain's
     stream; they give the dominant class, its average launch time (the roofline entry, with
-    the flop/byte model of algorithmic_work) and the evaluation's algorithmic FP64 work: the
-    flop-bound classes' launches per evaluation times their model work. The timed
+    the flop/byte model of algorithmic_work); the evaluation's algorithmic FP64 work is that of
+    its factorisations, Green's functions and products. The timed
     evaluations run without events."""
     from dqmc_amd import DQMC, UniformStream, _capi
     p = workload_params(amd, L=12, slices=100, seed=3001)
@@ -221,7 +221,14 @@ def grad_measure(amd, evals, warmup):
     c.close()
     dom = int(np.argmax(ms))
     avg_ms = float(ms[dom]) / max(int(cnt[dom]), 1)
+    # a launch serves several intervals of the evaluation, so the work is counted per evaluation:
+    # R = M / safe_mult intervals, two stack halves of R and R - 1 factorisations, R Green's
+    # functions, 2 M wraps
+    R, sm = p.slices // p.safe_mult, p.safe_mult
+    units = {_capi.K_QRP: 2 * R - 1, _capi.K_QFORM: 2 * R - 1, _capi.K_GEMM: 5 * R - 1, _capi.K_INVERSE: R,
+             _capi.K_APPLY_B: (2 * R - 1) * sm + 2 * p.slices}
     bound, work, unit = algorithmic_work(dom, p.n, 0.0)
+    work *= units.get(dom, 0) * warmup / max(int(cnt[dom]), 1)  # per launch
     if bound == "hbm":
         achieved, peak, runit = work / (avg_ms * 1e-3) / 1e9, PEAK_HBM_GBS, "GB/s"
     else:
@@ -229,8 +236,8 @@ def grad_measure(amd, evals, warmup):
     flop = 0.0
     for k in range(_capi.K_NCLASS):
         b, w, _u = algorithmic_work(k, p.n, 0.0)
-        if b == "mfma" and cnt[k]:
-            flop += w * float(cnt[k]) / warmup
+        if b == "mfma":
+            flop += w * units.get(k, 0)
     eval_tflops = flop * evals / dt / 1e12
     return {"value": evals / dt, "unit": "evals/s", "config": "L=12 beta=10 dtau=0.1 (M=100), n=576",
             "components": int(g.size), "evals": evals, "seconds": dt,

@@ -316,8 +316,12 @@ hipError_t launch_global_shift(hipStream_t s, const ChainDesc* chain, double* ph
 hipError_t launch_global_decide(hipStream_t s, const ChainDesc* chain);
 hipError_t launch_global_restore(hipStream_t s, const double* flag, const RestoreList& r);
 
+// (slice: the same for all chains, or taken per chain from `slices` when non-null)
 hipError_t launch_grad_slice(hipStream_t s, const ChainDesc* chains, int nchains, int Nmax, int slice,
-                             double* const* grad);
+                             double* const* grad, const int* slices = nullptr);
+// the scalars of a chain's interval jobs (job 0 the lowest interval) into the chain: log|det G| of
+// job 0 and, with drift, the last (job 1's) and largest of their drifts
+hipError_t launch_fold_jobs(hipStream_t s, const ChainDesc* chain, const ChainDesc* jobs, int njobs, int drift);
 
 // Fermionic observables of one chain (fermion_measurements.jl:388-899): kind 0 pairing
 // (etpc / zfpc), 1 charge density (etcdc / zfcdc), 2 current-current (zfccc). Sums over

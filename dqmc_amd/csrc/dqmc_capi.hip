@@ -54,6 +54,17 @@ VecRef NV(int id) { return VecRef{VK_NAMED, id}; }
 VecRef DS(int k) { return VecRef{VK_DSTACK, k}; }
 const VecRef NOVEC{-1, 0};
 
+// Jobs: independent pieces of one chain's work (intervals of imaginary time, the two halves of
+// its stack) as descriptors of a batch, so that one launch advances all of them. One block of
+// device memory holds their matrices, scratch and tables.
+struct JobSet {
+  void* mem = nullptr;
+  ChainDesc* d_desc = nullptr;
+  int* d_int = nullptr;         // slices and operator choices per launch
+  double** d_ptr = nullptr;
+  bool failed = false;          // the memory was not to be had: the sequential path serves
+};
+
 struct ChainMem {
   dqmc_params p;
   int L, N, n, M, nelem;
@@ -68,6 +79,7 @@ struct ChainMem {
   double** grad_ptr = nullptr;
   double* mom = nullptr;
   double* phi_bak = nullptr;
+  JobSet grad_jobs;
   // time-displaced Green's function storage (dqmc_tdgf_alloc)
   cplx* tdgf_mat = nullptr;
   double* tdgf_vec = nullptr;
@@ -402,8 +414,9 @@ void chain_free(ChainMem& cm) {
   if (cm.uniforms) (void)hipFree(cm.uniforms);
   if (cm.log_buf) (void)hipFree(cm.log_buf);
   for (void* p : {(void*)cm.grad, (void*)cm.grad_ptr, (void*)cm.mom, (void*)cm.phi_bak, (void*)cm.tdgf_mat,
-                  (void*)cm.tdgf_vec, (void*)cm.gb, (void*)cm.meas})
+                  (void*)cm.tdgf_vec, (void*)cm.gb, (void*)cm.meas, cm.grad_jobs.mem})
     if (p) (void)hipFree(p);
+  cm.grad_jobs = JobSet{};
   cm.meas = cm.meas_etgf = cm.meas_tnb = cm.meas_part = cm.meas_res = nullptr;
   cm.has_etgf = cm.has_hopping = false;
   cm.tdgf_mat = nullptr;
@@ -2346,6 +2359,230 @@ int dqmc_boson_action(dqmc_ctx* ctx, double* S) {
 // build_stack, then one down pass over all slices; at slice l the Green's function G(l)
 // of the stack (stack.jl:336) gives the fermionic part, the bosonic part is analytic.
 // Afterwards scal[S_BOSON_ACTION] = S_B and scal[S_LOGDET] = log|det G|.
+}  // extern "C"
+namespace {
+
+// Takes arrays out of one block: with base == nullptr it only adds up what they need.
+struct Carve {
+  char* base;
+  size_t off = 0;
+  template <class T>
+  T* take(size_t count) {
+    off = (off + 255) & ~(size_t)255;
+    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+    off += count * sizeof(T);
+    return p;
+  }
+};
+// the factorisation scratch, barrier words and scalars of one job
+void carve_scratch(Carve& cv, ChainDesc& d) {
+  const size_t n = d.n;
+  d.qr_vn = cv.take<double>(2 * n);
+  d.qr_cand = cv.take<cplx>((size_t)2 * kMaxWG * n);
+  d.qr_cand_norm = cv.take<double>(2 * kMaxWG);
+  d.qr_cand_pos = cv.take<int>(2 * kMaxWG);
+  d.qr_perm = cv.take<int>(n);
+  d.qr_lpos = cv.take<int>(n);
+  d.qr_tau = cv.take<cplx>(n);
+  d.qr_Tf = cv.take<cplx>(16 * (n + 16));
+  d.qr_flags = cv.take<unsigned int>(1 + (n + 7) / 8);
+  d.inv_piv = cv.take<int>(n);
+  d.inv_bcast = cv.take<cplx>(2 * n);
+  d.bar_count = cv.take<unsigned int>(2);
+  d.bar_gen = d.bar_count ? d.bar_count + 1 : nullptr;
+  d.scal = cv.take<double>(kNumScalar);
+}
+// descriptors and tables to the device, barrier words and scalars cleared
+hipError_t jobs_upload(JobSet& js, const ChainMem& cm, const std::vector<ChainDesc>& h, const std::vector<int>& ints) {
+  hipError_t e = hipMemcpy(js.d_desc, h.data(), h.size() * sizeof(ChainDesc), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(js.d_int, ints.data(), ints.size() * sizeof(int), hipMemcpyHostToDevice);
+  for (const auto& d : h) {
+    if (d.scal == cm.d.scal) continue;  // the chain itself
+    if (e == hipSuccess) e = hipMemset(d.bar_count, 0, 2 * sizeof(unsigned int));
+    if (e == hipSuccess) e = hipMemset(d.scal, 0, kNumScalar * sizeof(double));
+  }
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  return e;
+}
+// a group over `nj` jobs of g's chain on g's stream, the workgroups shared between them
+Group job_group(const Group& g, ChainDesc* d_desc, int nj) {
+  Group j;
+  j.n = g.n;
+  j.N = g.N;
+  j.L = g.L;
+  j.M = g.M;
+  j.s = g.s;
+  j.nelem = g.nelem;
+  j.chkr = g.chkr;
+  j.ngroups = g.ngroups;
+  j.all_checks = g.all_checks;
+  j.stream = g.stream;
+  j.d_desc = d_desc;
+  j.chains.assign(nj, 0);
+  j.greens_route = g.greens_route;
+  j.udt_route = g.udt_route;
+  j.qr_nb = g.qr_nb;
+  j.prof_mask = g.prof_mask;
+  const int per = std::max(1, 256 / nj);
+  j.wg_qr = std::max(1, std::min(g.wg_qr, per));
+  j.wg_inv = std::max((g.n + 511) / 512, std::min(g.wg_inv, per));
+  return j;
+}
+// its timing records go to the chain's group
+void job_group_done(Group& g, Group& j) {
+  g.prof.insert(g.prof.end(), j.prof.begin(), j.prof.end());
+  g.event_pool.insert(g.event_pool.end(), j.event_pool.begin(), j.event_pool.end());
+}
+
+// The gradient needs the Green's function of every slice of one field, with no update in between,
+// so its R = M / safe_mult intervals are independent once the stack's two halves exist: the left
+// and right halves are built side by side (2 jobs, R - 1 factorisations deep instead of 2 R), then
+// the Green's functions at all interval boundaries (R jobs), the wraps and the slices' traces.
+// The sequential pass is bound by the panel chains of 3 R factorisations on one workgroup each;
+// side by side they are R + 1 chains deep and fill the chip: dS/dphi at L = 12, M = 100 (R = 10)
+// 64.3 -> 30.8 ms, an HMC trajectory at L = 6, M = 50 (R = 5) 30.1 -> 13.5 ms.
+// Afterwards the chain is where the sequential pass leaves it: the right half in its stack, the
+// identity in elements 0 and R, G of slice 1 in M_G, log|det G| and the drift in its scalars.
+// Descriptors: R interval jobs (job j starts at slice (j + 1) safe_mult), then the halves.
+constexpr int kMaxGradJobs = 64;  // intervals; bounds the memory (6 n x n each) and keeps 4 workgroups per job
+
+int grad_jobs_create(const Group& g, ChainMem& cm) {
+  JobSet& js = cm.grad_jobs;
+  const int R = g.nelem - 1, sm = g.s;
+  const size_t n = g.n, nn = n * n;
+  std::vector<ChainDesc> h;
+  std::vector<int> ints;
+  // per step of the halves: element read and written by the left (job 0) and right (job 1) half
+  const int roles = 6;
+  for (int half = 0; half < 2; ++half)
+    for (int i = 0; i < R; ++i) {
+      const int src = half ? R - i : i, dst = half ? R - i - 1 : i + 1;
+      ints.insert(ints.end(), {plan_enc(MK_USTACK, src), plan_enc(VK_DSTACK, src), plan_enc(MK_TSTACK, src),
+                               plan_enc(MK_USTACK, dst), plan_enc(VK_DSTACK, dst), plan_enc(MK_TSTACK, dst)});
+    }
+  for (int i = 0; i < R; ++i)  // slices of the halves' operators
+    for (int t = 0; t < sm; ++t) {
+      ints.push_back(i * sm + t);
+      ints.push_back(std::max(0, (R - i) * sm - 1 - t));
+    }
+  ints.push_back(0);  // operator choice of the halves: B, B^dagger
+  ints.push_back(1);
+  for (int t = 0; t < sm; ++t)  // slices of the intervals
+    for (int j = 0; j < R; ++j) ints.push_back((j + 1) * sm - 1 - t);
+  auto layout = [&](Carve& cv) {
+    h.assign(R + 2, cm.d);
+    cplx* lu = cv.take<cplx>(nn * (R + 1));
+    cplx* lt = cv.take<cplx>(nn * (R + 1));
+    double* ld = cv.take<double>(n * (R + 1));
+    js.d_desc = cv.take<ChainDesc>(R + 2);
+    js.d_int = cv.take<int>(ints.size());
+    js.d_ptr = cv.take<double*>(R);
+    for (int j = 0; j < R + 1; ++j) {
+      ChainDesc& d = h[j];
+      carve_scratch(cv, d);
+      if (j == R) {  // the left half
+        d.ustack = lu;
+        d.tstack = lt;
+        d.dstack = ld;
+        d.mat[M_CURU] = cv.take<cplx>(nn);
+        d.mat[M_QRT] = cv.take<cplx>(nn);
+        d.plan = js.d_int;
+        continue;
+      }
+      const int k = j + 1;
+      d.mat[M_UL] = lu + nn * k;
+      d.mat[M_TL] = lt + nn * k;
+      d.vec[V_DL] = ld + n * k;
+      d.mat[M_UR] = cm.d.ustack + nn * k;
+      d.mat[M_TR] = cm.d.tstack + nn * k;
+      d.vec[V_DR] = cm.d.dstack + n * k;
+      if (j > 0) {
+        d.mat[M_G] = cv.take<cplx>(nn);
+        d.mat[M_GRAD] = h[j - 1].mat[M_GW];  // the interval below's Green's function at its start
+      }
+      for (int m : {M_GW, M_TMP, M_TMP2}) d.mat[m] = cv.take<cplx>(nn);
+      for (int v : {V_D1, V_D2, V_D3, V_D4, V_D5}) d.vec[v] = cv.take<double>(n);
+    }
+    h[R + 1].plan = js.d_int ? js.d_int + (size_t)R * roles : nullptr;  // the right half: the chain itself
+  };
+  Carve size{nullptr};
+  layout(size);
+  if (hipMalloc(&js.mem, size.off) != hipSuccess) {
+    (void)hipGetLastError();
+    js = JobSet{};
+    js.failed = true;
+    return 0;
+  }
+  Carve cv{(char*)js.mem};
+  layout(cv);
+  const std::vector<double*> ptr(R, cm.grad);
+  hipError_t e = jobs_upload(js, cm, h, ints);
+  if (e == hipSuccess) e = hipMemcpy(js.d_ptr, ptr.data(), ptr.size() * sizeof(double*), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(js.mem);
+    js = JobSet{};
+    return fail(DQMC_E_HIP, std::string("gradient jobs: ") + hipGetErrorString(e));
+  }
+  return 0;
+}
+
+int grad_parallel(Group& g, ChainMem& cm) {
+  JobSet& js = cm.grad_jobs;
+  const int R = g.nelem - 1, sm = g.s, n = g.n, N = g.N;
+  hipStream_t st = g.stream;
+  const int* d_sli = js.d_int + (size_t)2 * R * 6;
+  const int* d_sel = d_sli + (size_t)2 * R * sm;
+  const int* d_row = d_sel + 2;
+  Ops o(g);
+  RC(o.identity_elem(0));
+  RC(o.identity_elem(R));
+  {
+    ChainDesc* dd = js.d_desc + R;
+    Group both = job_group(g, dd, 2), left = job_group(g, dd, 1);
+    LCHK(launch_identity(st, dd, 1, n, US(0), NOVEC));
+    LCHK(launch_identity(st, dd, 1, n, TS(0), NOVEC));
+    LCHK(launch_ones_vec(st, dd, 1, n, DS(0)));
+    for (int i = 0; i < R; ++i) {
+      Group& h = i + 1 < R ? both : left;  // element 0 of the right half is not needed
+      Ops oh(h);
+      const int nj = h.nch(), p = 6 * i;
+      RC(oh.copy(NM(M_CURU), MatRef{MK_PLAN, p}));
+      for (int t = 0; t < sm; ++t) {
+        ProfScope ps(h, DQMC_K_APPLY_B);
+        LCHK(launch_apply_B_chkr_sel(st, dd, nj, n, N, NM(M_CURU), B_LEFT, B_DAG_LEFT, d_sel,
+                                     d_sli + 2 * ((size_t)i * sm + t), g.ngroups));
+      }
+      LCHK(launch_scale_cols(st, dd, nj, n, NM(M_CURU), VecRef{VK_PLAN, p + 1}));
+      RC(oh.udt(NM(M_CURU), VecRef{VK_PLAN, p + 4}, MatRef{MK_PLAN, p + 3}, NM(M_QRT), true));
+      RC(oh.gemm(MatRef{MK_PLAN, p + 5}, NM(M_QRT), OP_N, MatRef{MK_PLAN, p + 2}, OP_N));
+    }
+    job_group_done(g, both);
+    job_group_done(g, left);
+  }
+  Group all = job_group(g, js.d_desc, R);
+  Ops oa(all);
+  RC(oa.calculate_greens_scalesep());
+  if (g.all_checks) RC(oa.copy(NM(M_GW), NM(M_G)));
+  for (int t = 0; t < sm; ++t) {
+    const int* sl = d_row + (size_t)t * R;
+    {
+      ProfScope ps(all, DQMC_K_APPLY_B);
+      LCHK(launch_apply_B_chkr(st, js.d_desc, R, n, N, NM(M_G), B_INV_LEFT, 0, sl, g.ngroups));
+      LCHK(launch_apply_B_chkr(st, js.d_desc, R, n, N, NM(M_G), B_RIGHT, 0, sl, g.ngroups));
+    }
+    LCHK(launch_grad_slice(st, js.d_desc, R, N, 0, js.d_ptr, sl));
+  }
+  if (g.all_checks && R > 1) LCHK(launch_maxdiff(st, js.d_desc + 1, R - 1, n, NM(M_G), NM(M_GRAD)));
+  LCHK(launch_fold_jobs(st, g.d_desc, js.d_desc, R, g.all_checks ? 1 : 0));
+  job_group_done(g, all);
+  g.cur = 1;
+  g.dir = -1;
+  g.recomputed = g.all_checks && sm == 1 && R > 1;
+  return 0;
+}
+
+}  // namespace
+extern "C" {
 static int grad_enqueue(dqmc_batch* b) {
   Group& g = b->groups[0];
   ChainMem& cm = b->chains[0];
@@ -2357,6 +2594,15 @@ static int grad_enqueue(dqmc_batch* b) {
     HIPCHK(hipMemcpy(cm.grad_ptr, &cm.grad, sizeof(double*), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&cm.mom, sizeof(double) * 3 * cm.N * cm.M));
     HIPCHK(hipMalloc(&cm.phi_bak, sizeof(double) * 3 * cm.N * cm.M));
+  }
+  // the verbatim routes and the dense hopping keep the sequential pass, as do more intervals than jobs
+  if (g.greens_route == 0 && g.udt_route == 0 && g.chkr && g.nelem - 1 <= kMaxGradJobs && !cm.grad_jobs.failed) {
+    if (!cm.grad_jobs.mem && (rc = grad_jobs_create(g, cm))) return rc;
+    if (!cm.grad_jobs.failed) {
+      LCHK(launch_boson_grad(g.stream, g.d_desc, 1, cm.N * cm.M, cm.grad_ptr));
+      LCHK(launch_boson_action(g.stream, g.d_desc, 1, g.N));
+      return grad_parallel(g, cm);
+    }
   }
   if ((rc = o.build_stack())) return rc;
   if ((rc = o.propagate())) return rc;  // -> slice M, direction -1, log det of G(1)

@@ -88,12 +88,13 @@ hipError_t launch_boson_grad(hipStream_t s, const ChainDesc* chains, int nchains
 
 // fermionic part at slice l (0-based) from the current G = G(l+1 in 1-based slices):
 // grad[a,i,l] -= Re tr[(1 - G)_ii  eVop(phi,-1) d_a eVop(phi,+1)]
-__global__ __launch_bounds__(256) void k_grad_slice(const ChainDesc* chains, int slice, double* const* grad) {
+__global__ __launch_bounds__(256) void k_grad_slice(const ChainDesc* chains, int slice, const int* slices,
+                                                    double* const* grad) {
   const ChainDesc& c = chains[blockIdx.y];
   const int N = c.N, n = c.n;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  const int l = slice;
+  const int l = slices ? slices[blockIdx.y] : slice;
   const cplx* G = c.mat[M_G];
   double* gr = grad[blockIdx.y];
   const double* f = c.phi + 3 * ((size_t)i + (size_t)N * l);
@@ -161,8 +162,23 @@ hipError_t launch_daxpy(hipStream_t s, double* y, const double* x, double a, lon
 }
 
 hipError_t launch_grad_slice(hipStream_t s, const ChainDesc* chains, int nchains, int Nmax, int slice,
-                             double* const* grad) {
-  hipLaunchKernelGGL(k_grad_slice, dim3((Nmax + 255) / 256, nchains), dim3(256), 0, s, chains, slice, grad);
+                             double* const* grad, const int* slices) {
+  hipLaunchKernelGGL(k_grad_slice, dim3((Nmax + 255) / 256, nchains), dim3(256), 0, s, chains, slice, slices, grad);
+  return hipGetLastError();
+}
+
+__global__ void k_fold_jobs(const ChainDesc* chain, const ChainDesc* jobs, int njobs, int drift) {
+  if (threadIdx.x != 0) return;
+  double* scal = chain->scal;
+  scal[S_LOGDET] = jobs[0].scal[S_LOGDET];
+  if (!drift || njobs < 2) return;
+  double m = scal[S_DRIFT_MAX];
+  for (int j = 1; j < njobs; ++j) m = fmax(m, jobs[j].scal[S_DRIFT_LAST]);
+  scal[S_DRIFT_LAST] = jobs[1].scal[S_DRIFT_LAST];
+  scal[S_DRIFT_MAX] = m;
+}
+hipError_t launch_fold_jobs(hipStream_t s, const ChainDesc* chain, const ChainDesc* jobs, int njobs, int drift) {
+  hipLaunchKernelGGL(k_fold_jobs, dim3(1), dim3(64), 0, s, chain, jobs, njobs, drift);
   return hipGetLastError();
 }
 
