@@ -46,6 +46,7 @@ int fail(int code, const std::string& msg) {
   } while (0)
 
 constexpr int kMaxWG = 128;
+constexpr int kMaxLocalWG = 256;  // default workgroups of one chain's local updates: one per CU
 
 MatRef NM(int id) { return MatRef{MK_NAMED, id}; }
 MatRef US(int k) { return MatRef{MK_USTACK, k}; }
@@ -448,7 +449,7 @@ int default_groups(Group& g, int batch_chains) {
   // local updates: the windowed variant is fastest with many narrow column blocks (the
   // own columns then fit in LDS beside the window); fall back to the n/8 blocks the other
   // variants were tuned at when the window does not fit
-  g.wg_local = std::max(1, std::min({per, g.n / 4, kMaxWG}));
+  g.wg_local = std::max(1, std::min({per, g.n / 4, kMaxLocalWG}));
   if (local_window_sites(g.n, g.wg_local) < 2) g.wg_local = std::max(1, std::min({per, g.n / 8, kMaxWG}));
   // 8-column panels: each panel's serial part is shorter and the panel stays in registers
   // (the autotuner measures 16 too)

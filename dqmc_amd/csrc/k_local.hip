@@ -255,8 +255,7 @@ struct Proposals {
   long long cur, logi;
   double dS_acc, minratio;
   int nacc, nonreal, i;
-  // an accepted proposal whose field update is deferred (commit_accept): site (-1: none),
-  // exp(-dS) and the new field
+  // the accepted proposal for commit_accept: site (-1: none), exp(-dS) and the new field
   int pend_site;
   double pend_e, pend_n0, pend_n1, pend_n2;
 };
@@ -296,8 +295,7 @@ __device__ inline void commit_accept(const ChainDesc& c, const SliceLds& s, Prop
 // calc_boson_action_diff (action.jl:57-101).
 template <class Diag>
 __device__ int evaluate_proposals(const ChainDesc& c, const SliceLds& s, Proposals& p, LocalShared& sh,
-                                  double box, int dolog, bool logger, Diag diag, int* stop, int limit,
-                                  bool defer = false) {
+                                  double box, int dolog, bool logger, Diag diag, int* stop, int limit) {
   const int N = c.N, lane = threadIdx.x & 63;
   const int row = lane >> 4;  // 16-lane row of the wave: it evaluates site i + row
   const int ea = (lane & 15) >> 2, eb = lane & 3;
@@ -429,7 +427,7 @@ __device__ int evaluate_proposals(const ChainDesc& c, const SliceLds& s, Proposa
         p.pend_n0 = read_lane(nw[0], 16 * g);
         p.pend_n1 = read_lane(nw[1], 16 * g);
         p.pend_n2 = read_lane(nw[2], 16 * g);
-        if (!defer) commit_accept(c, s, p);
+        commit_accept(c, s, p);
         // M^-1 (b, a) = cofactor (a, b) / det M, one entry per lane of row g
         cplx m3[9];
 #pragma unroll
@@ -916,125 +914,306 @@ __global__ __launch_bounds__(256) void k_local_updates_delayed(const ChainDesc* 
 }
 
 // ---------------------------------------------------------------------------
-// Variant 4: windowed delayed updates. The sites of the slice are split into R windows
-// (R even, at most K sites each). Inside a window no workgroup communicates:
-//  * the accepted updates are kept implicitly. With G0 the window's starting G and
-//    Yt = [G0[:, c_b] - E_b]_b the starting site columns of the accepted sites (minus their
-//    unit columns), every factor A_b = (G'[:, c_b] - E_b) M_b^-1 equals Yt P_b for a small
-//    coefficient matrix P_b (4K x 4): P_b = (S_b + sum_{b'<b} P_b' B_b'[:, c_b]) M_b^-1, S_b
-//    selecting block b. Only P_b, the 4x4 blocks A_b(r_j, :) and B_b(:, c_j) at the window's
-//    sites, B_b on the workgroup's own columns, and the current blocks G'(r_j, c_k) between
-//    the window's sites are stored (LDS), so a window's size is not bounded by n x 4 factors;
-//  * decisions read G'(r_j, c_j); new factor pairs need only the stored blocks and G0 on
-//    the own columns.
-// At the window's end each workgroup writes its columns of G0 + Yt W, W = sum_b P_b B_b
-// (formed in place of the B_b), into the partner buffer (M_G and M_GALT alternate; R is
-// even, so the slice ends in M_G), then one group barrier. Global G is read only from the
-// current window's buffer, which no workgroup writes during the window. With TILE the own
-// columns also stay in LDS for the slice.
-// Same arithmetic as update_greens! (local_updates.jl:61-95) up to the order of sums.
+// Variant 4: windowed updates. The sites of the slice are split into R windows of at most K
+// sites. Inside a window no workgroup communicates: with G0 the window's starting G, S the
+// sites accepted so far and F all sites of the window, every workgroup keeps the K x K array
+// of 4 x 4 blocks (LDS)
+//    T_FF = G'(r_j, c_k)   current G between the window's sites not accepted
+//    T_SS = X              G' = G0 + (G0(:, S) - E_S) X G0(S, :)
+//    T_SF = X G0(S, c_k),  T_FS = G0(r_j, S) X.
+// Accepting site i (M = 1 + delta (1 - G'_ii)) is one Gauss-Jordan step on that array:
+// T_jk += A_j B_k with A_j = T_ji M^-1, B_k = delta T_ik, and with A_i = M^-1, B_i = delta the
+// row and the column of i become the products alone (T_ik = M^-1 delta T_ik and so on): one
+// rank-4 product in 16 x 16 tiles on the FP64 matrix cores. Nothing is kept per own column
+// until the window ends; then W = X G0(S, own) and G0 += (G0(:, S) - E_S) W.
+//
+// The chain of one acceptance is what bounds a window, so everything that does not need G is
+// taken out of it. Wave 0 decides, the other waves update T:
+//  * the new field of a site, its delta (four complex numbers: a product of two site blocks
+//    has 7 parameters) and most of the action difference depend on the uniforms' position
+//    only, that is on how many of the window's sites so far were accepted with p > 1 (3 draws
+//    instead of 4). All (site, count) pairs are formed at the window's start by all threads;
+//  * while the others form A and B, wave 0 commits the field and forms the rest of the next
+//    four proposals that does not need G (space neighbours, exp(-dS));
+//  * after them it has four sites' G'_jj from A_j, B_j and the blocks read before, and one
+//    chain of M, its 2 x 2 minors, cofactors (lane-parallel, DPP moves) and determinant.
+// Two barriers per acceptance. Against windows that kept H, U, P and B_b per own column and
+// evaluated proposals from the field on 4 waves, per slice: n = 64 65 -> 43, n = 256 254 -> 178,
+// n = 400 447 -> 287, n = 1024 (128 -> 256 workgroups, own columns now in LDS) 2983 -> 1049,
+// 64 chains of n = 400 2190 -> 1044 us. At n = 400, cycles per slice: decisions 425,000 ->
+// 220,000 (a round of four is one chain of some 300 instructions), factors 168,000 -> 90,000,
+// window ends 358,000 -> 120,000, barriers 141,000 (one contended counter per window).
+//
+// TILE: the own columns of G stay in LDS for the slice and a window's end publishes (in
+// M_GALT) just the columns of the next window's sites, all others read nothing else; the last
+// window writes M_G. Windows' columns are disjoint, so nobody writes what a slower workgroup
+// still reads; at least two windows, as the first reads M_G itself.
+// Otherwise every window streams the own columns from one of M_G and M_GALT to the other (R
+// even, so the slice ends in M_G), with W in chunks of columns that fit the LDS left.
 // ---------------------------------------------------------------------------
-constexpr int kWinMax = 12;     // window sites with LDS-resident own columns
-constexpr int kWinMaxGlob = 12;  // window sites otherwise (Bo and H of the own columns bound it)
-constexpr size_t kWindowLdsMax = 160 * 1024 - 1024;  // the CU's LDS less this kernel's static part
+// sites of a window, in steps of one tile of T: with LDS-resident columns more sites only make
+// the steps on T longer; without, every window less saves a pass over G
+constexpr int kWinStep = 4, kWinMaxTile = 16, kWinMax = 20;
+constexpr int kWinThreads = 512;  // wave 0 decides, seven waves update
+constexpr size_t kWindowLdsMax = 160 * 1024 - 2048;  // the CU's LDS less this kernel's static part
 
-__host__ __device__ inline int window_bo_stride(int n, int wg) { return (n + wg - 1) / wg + 1; }
+// LDS of a slice: field, time and space neighbour sums (3N each), uniforms, old site blocks (4N
+// each), neighbour table (4N ints)
+__host__ __device__ inline size_t win_slice_doubles(int N) { return (size_t)19 * N + (N & 1); }
+__host__ __device__ inline size_t win_entries(int K) { return (size_t)K * (K + 1) / 2; }
 __host__ __device__ inline size_t window_lds_bytes(int n, int N, int wg, int K, bool tile) {
-  const size_t ncs = window_bo_stride(n, wg);
-  const size_t t = tile ? (size_t)(ncs - 1) * n : 0;
-  return slice_lds_doubles(N) * 8 + (t + (size_t)8 * K * ncs + (size_t)48 * K * K + (size_t)32 * K) * 16;
+  const size_t nc = (n + wg - 1) / wg;
+  const size_t t = tile ? nc * n : 0;
+  const size_t scratch = (size_t)32 * K + 7 * win_entries(K);  // A, B, proposals
+  // W takes their place at the window's end: all own columns (TILE) or, behind X, at least 16
+  const size_t cols = tile ? nc : 16;
+  const size_t w = (size_t)4 * K * cols;
+  return win_slice_doubles(N) * 8 + (t + (size_t)4 * K * (4 * K + 1) + (scratch > w ? scratch : w)) * 16;
 }
 
-// End of a window without LDS-resident columns, on the FP64 matrix cores:
-// Gn[:, own] = Gc[:, own] + Yt W as transposed 16 x 16 tiles, D = W^T Yt^T + Gc^T, so that a
-// tile's lane (i, j) holds own column i, row j and every load and store of G covers 16
-// consecutive rows of a column. Each wave takes row blocks of 16; for its block the Yt^T
-// fragments of all accepted sites stay in registers (two doubles per site and lane) while it
-// walks the own columns two tiles at a time (four independent accumulator chains; the next
-// pair's G loads are issued before this pair's products). One complex k-step of four
-// (one accepted site's four columns of Yt) is four real MFMAs:
-// re += Wr Yr - Wi Yi, im += Wr Yi + Wi Yr. v_mfma_f64_16x16x4 lane layout: A(i, k) and
-// B(k, j) on lane i + 16 k (resp. j + 16 k), D(i, j) element v on lane j + 16 ((i - v * 4)):
-// i = lane / 16 + 4 v. m >= 1.
+// keeps what is computed from it where it is used: the kernel's phases would otherwise hold
+// their lane addresses in registers across one another
+__device__ inline int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// 16-byte LDS accesses (a cplx is only known to be 8-byte aligned, and the pairs of 8-byte
+// accesses it takes otherwise run at half the rate); every cplx array of the kernel's LDS
+// starts at a multiple of 16 bytes
+typedef double d2 __attribute__((ext_vector_type(2)));
+__device__ inline cplx l16(const cplx* p) {
+  const d2 v = *reinterpret_cast<const d2*>(p);
+  return mk(v.x, v.y);
+}
+__device__ inline void s16(cplx* p, cplx v) { *reinterpret_cast<d2*>(p) = d2{v.re, v.im}; }
+
+struct __attribute__((aligned(16))) WinShared {
+  cplx delta[16], minv[16];
+  int site[2];  // accepted site, -1 none among the four evaluated, >= s1 the window is done
+  int off;      // uniforms used so far in the slice
+  int accs[kWinMax];
+  double acce[kWinMax];  // exp(-dS) of the accepted
+};
+
+struct WinSlice {
+  double *phl, *tnb, *snb, *ul, *e1c;
+  int* nbl;
+  long long cur0, navail;
+};
+
+__device__ inline WinSlice win_load_slice(const ChainDesc& c, int l, double* smem) {
+  const int N = c.N, M = c.M, tid = threadIdx.x;
+  WinSlice s;
+  s.phl = smem;
+  s.tnb = s.phl + 3 * N;
+  s.snb = s.tnb + 3 * N;
+  s.ul = s.snb + 3 * N;
+  s.e1c = s.ul + 4 * N;
+  s.nbl = reinterpret_cast<int*>(s.e1c + 4 * N);
+  const int le = (l == 0) ? M - 1 : l - 1;  // time_neighbors (lattice.jl:144-153)
+  const int la = (l == M - 1) ? 0 : l + 1;
+  const gdouble *f = gp(c.phi) + (size_t)3 * N * l, *fe = gp(c.phi) + (size_t)3 * N * le,
+                *fa = gp(c.phi) + (size_t)3 * N * la;
+  const gint* nb = gp(c.nb);
+  s.cur0 = *c.ucursor;
+  // at most 4 draws per proposal: this slice consumes no more than 4N uniforms
+  s.navail = min((long long)4 * N, c.n_uniforms - s.cur0);
+  const gdouble* u = gp(c.uniforms) + s.cur0;
+  for (int e = tid; e < 4 * N; e += blockDim.x) {
+    s.nbl[e] = nb[e];
+    if (e < s.navail) s.ul[e] = u[e];
+  }
+  // neighbour sums in the order of calc_boson_action_diff (action.jl:57-101), from global
+  // memory so no barrier is needed before them
+  for (int e = tid; e < 3 * N; e += blockDim.x) {
+    const int i = e / 3, a = e - 3 * i;
+    s.phl[e] = f[e];
+    s.tnb[e] = fa[e] + fe[e];
+    double sn = 0.0;
+    for (int k = 0; k < 4; ++k) sn += f[3 * nb[k * N + i] + a];
+    s.snb[e] = sn;
+  }
+  // each site is visited once per slice, so its old field is the value at kernel start
+  const double lam_dtau = c.lam * c.dtau;
+  for (int i = tid; i < N; i += blockDim.x) {
+    double C, R;
+    cplx S;
+    ev_coeffs_op(lam_dtau, f[3 * i], f[3 * i + 1], f[3 * i + 2], -1.0, C, S, R);
+    s.e1c[4 * i + 0] = C;
+    s.e1c[4 * i + 1] = S.re;
+    s.e1c[4 * i + 2] = S.im;
+    s.e1c[4 * i + 3] = R;
+  }
+  return s;
+}
+
+// The part of a proposal that depends on the site and the uniforms' position only: delta =
+// eV_op(old, -1) eV_op(new, +1) - 1, whose entry (a, b) is number a ^ b of (alpha, beta, gamma,
+// eta), conjugated in rows 1 and 2 (gamma, eta there negated as well), and the new field and
+// the parts of the action difference (calc_boson_action_diff, action.jl:57-101).
+__device__ inline void win_proposal(const ChainDesc& c, const WinSlice& s, int i, long long off, double box,
+                                    cplx* out) {
+  const long long o = min(off, max(s.navail - 4, 0ll));  // in bounds; past the end nothing is accepted
+  const double* u = s.ul + o;
+  double nw[3], old[3], dt_dot = 0.0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    old[a] = s.phl[3 * i + a];
+    nw[a] = old[a] + (-box + 2.0 * box * u[a]);
+    dt_dot += s.tnb[3 * i + a] * (nw[a] - old[a]);
+  }
+  const double old_sq = old[0] * old[0] + old[1] * old[1] + old[2] * old[2];
+  const double new_sq = nw[0] * nw[0] + nw[1] * nw[1] + nw[2] * nw[2];
+  const double sq = new_sq - old_sq;
+  const double C1 = s.e1c[4 * i], R1 = s.e1c[4 * i + 3];
+  const cplx S1 = mk(s.e1c[4 * i + 1], s.e1c[4 * i + 2]);
+  double C2, R2;
+  cplx S2;
+  ev_coeffs_op(c.lam * c.dtau, nw[0], nw[1], nw[2], 1.0, C2, S2, R2);
+  cplx al = mk(C1 * C2, 0.0);
+  cfma(al, S1, conj(S2));
+  al.re = fma(R1, R2, al.re) - 1.0;
+  s16(out + 0, al);
+  s16(out + 1, mk(fma(C1, S2.re, S1.re * C2), fma(C1, S2.im, S1.im * C2)));
+  s16(out + 2, mk(fma(R1, S2.re, -S1.re * R2), fma(R1, S2.im, -S1.im * R2)));
+  s16(out + 3, mk(fma(C1, R2, R1 * C2), 0.0));
+  s16(out + 4, mk(nw[0], nw[1]));
+  if (!c.edrun) {
+    const double k_time = 1.0 / (c.dtau * c.c * c.c);
+    s16(out + 5, mk(nw[2], k_time * (sq - dt_dot)));
+    s16(out + 6, mk(4 * sq, c.dtau * (0.5 * c.r * sq + 0.25 * c.u * (new_sq * new_sq - old_sq * old_sq))));
+  } else {
+    s16(out + 5, mk(nw[2], 0.0));
+    s16(out + 6, mk(0.0, c.dtau * (0.5 * c.r * sq)));
+  }
+}
+
+// End of a window without LDS-resident columns, on the FP64 matrix cores: columns c0 ..
+// c0 + cn - 1 of the own ones, Gn = Gc + Yt W with Yt = Gc(:, S) - E_S, as transposed 16 x 16
+// tiles, D = W^T Yt^T + Gc^T, so that a tile's lane (i, j) holds column i, row j and every load
+// and store of G covers 16 consecutive rows of a column. A wave takes 16 rows by four tiles (64
+// columns) at a time: eight accumulator chains, the next item's 16 loads of G issued before
+// this item's products, Yt's fragments three accepted sites ahead, W's one. One complex k-step of four (one
+// accepted site's four columns of Yt) is four real MFMAs per tile: re += Wr Yr - Wi Yi,
+// im += Wr Yi + Wi Yr. v_mfma_f64_16x16x4 lane layout: A(i, k) and B(k, j) on lane i + 16 k
+// (resp. j + 16 k), D(i, j) element v on lane j + 16 (i - 4 v): i = lane / 16 + 4 v. m >= 1.
 typedef double v4d __attribute__((ext_vector_type(4)));
-__device__ inline void window_end_mfma(const gcplx* __restrict__ Gc, gcplx* __restrict__ Gn, const cplx* W,
-                                       const int* accs, int m, int n, int N, int cb0, int ncol, int ncs) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+__device__ inline void window_end_mfma(const gcplx* __restrict__ Gs, gcplx* __restrict__ Gn, const cplx* W, int ws,
+                                       const int* accs, int m, int n, int N, int cb0, int c0, int cn) {
+  constexpr int NT = 4;
+  const int lane = threadIdx.x & 63, nw = kWinThreads >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  const int nrb = (n + 15) >> 4, ncp = (ncol + 31) >> 5;  // row blocks, pairs of column tiles
-  for (int rb = wave; rb < nrb; rb += nw) {
-    const int row = rb * 16 + li, rr = min(row, n - 1);
-    // G tile loads of a pair of column tiles starting at own column c0
-    auto load_pair = [&](int c0, cplx (&g)[8]) __attribute__((always_inline)) {
+  const int nrb = (n + 15) >> 4, items = nrb * ((cn + 16 * NT - 1) / (16 * NT));
+  const gcplx* Gc = Gs + (size_t)(cb0 + c0) * n;
+  Gn += (size_t)(cb0 + c0) * n;
+  auto load_c = [&](int it, cplx (&g)[4 * NT]) __attribute__((always_inline)) {
+    const int p0 = it / nrb * (16 * NT), rr = min((it % nrb) * 16 + li, n - 1);
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int col = min(c0 + lk + 4 * (v & 3) + 16 * (v >> 2), ncol - 1);
-        g[v] = ld(Gc + (size_t)(cb0 + col) * n + rr);
-      }
-    };
-    // the first two pairs' loads go out before the Yt fragments', and every pair's loads two
-    // pairs ahead of its products
-    cplx nxt[8], nx2[8];
-    load_pair(0, nxt);
-    load_pair(min(32, (ncp - 1) * 32), nx2);
-    double yr[kWinMaxGlob], yi[kWinMaxGlob];
-#pragma unroll
-    for (int b = 0; b < kWinMaxGlob; ++b) {
-      yr[b] = 0.0;
-      yi[b] = 0.0;
-      if (b < m) {  // wave-uniform
-        const int col = accs[b] + lk * N;
-        cplx v = ld(Gc + (size_t)col * n + rr);
-        if (rr == col) v.re -= 1.0;
-        yr[b] = v.re;
-        yi[b] = v.im;
-      }
+    for (int v = 0; v < 4 * NT; ++v) {
+      const int col = min(p0 + lk + 4 * v, cn - 1);
+      g[v] = ld(Gc + (unsigned)(col * n + rr));
     }
-    for (int cp = 0; cp < ncp; ++cp) {
-      const int c0 = cp * 32;
-      v4d ar0, ai0, ar1, ai1;
+  };
+  cplx nxt[4 * NT];
+  if (wave < items) load_c(wave, nxt);
+  for (int it = wave; it < items; it += nw) {
+    const int p0 = it / nrb * (16 * NT), row = (it % nrb) * 16 + li, rr = min(row, n - 1);
+    auto load_y = [&](int b) __attribute__((always_inline)) {
+      const int col = accs[min(b, m - 1)] + lk * N;
+      cplx v = ld(Gs + (unsigned)(col * n + rr));
+      if (rr == col) v.re -= 1.0;
+      return v;
+    };
+    cplx y0 = load_y(0), y1 = load_y(1), y2 = load_y(2);
+    v4d re[NT], im[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        ar0[v] = nxt[v].re;
-        ai0[v] = nxt[v].im;
-        ar1[v] = nxt[v + 4].re;
-        ai1[v] = nxt[v + 4].im;
+        re[t][v] = nxt[4 * t + v].re;
+        im[t][v] = nxt[4 * t + v].im;
       }
+    if (it + nw < items) load_c(it + nw, nxt);
+    const cplx* wr = W + (size_t)lk * ws;
+    int wc[NT];
 #pragma unroll
-      for (int v = 0; v < 8; ++v) nxt[v] = nx2[v];
-      if (cp + 2 < ncp) load_pair(c0 + 64, nx2);
-      const int w0 = min(c0 + li, ncol - 1), w1 = min(c0 + 16 + li, ncol - 1);
+    for (int t = 0; t < NT; ++t) wc[t] = min(p0 + 16 * t + li, cn - 1);
+    const int nt = min(NT, (cn - p0 + 15) >> 4);  // tiles with columns
+    cplx x[NT], xn[NT];
 #pragma unroll
-      for (int b = 0; b < kWinMaxGlob; ++b) {
-        if (b < m) {
-          const cplx* wr = W + (size_t)(4 * b + lk) * ncs;
-          const cplx x0 = wr[w0], x1 = wr[w1];
-          ar0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.re, yr[b], ar0, 0, 0, 0);
-          ai0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.re, yi[b], ai0, 0, 0, 0);
-          ar1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.re, yr[b], ar1, 0, 0, 0);
-          ai1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.re, yi[b], ai1, 0, 0, 0);
-          ar0 = __builtin_amdgcn_mfma_f64_16x16x4f64(-x0.im, yi[b], ar0, 0, 0, 0);
-          ai0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.im, yr[b], ai0, 0, 0, 0);
-          ar1 = __builtin_amdgcn_mfma_f64_16x16x4f64(-x1.im, yi[b], ar1, 0, 0, 0);
-          ai1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.im, yr[b], ai1, 0, 0, 0);
+    for (int t = 0; t < NT; ++t) x[t] = l16(wr + wc[t]);
+#pragma unroll 1
+    for (int b = 0; b < m; ++b) {
+      const cplx y = y0;
+      y0 = y1;
+      y1 = y2;
+      y2 = load_y(b + 3);
+      if (b + 1 < m) wr += 4 * ws;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) xn[t] = l16(wr + wc[t]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t < nt) {
+          re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].re, y.re, re[t], 0, 0, 0);
+          im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].re, y.im, im[t], 0, 0, 0);
+          re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[t].im, y.im, re[t], 0, 0, 0);
+          im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].im, y.re, im[t], 0, 0, 0);
         }
-      }
-      if (row < n) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int ca = c0 + lk + 4 * v, cb = ca + 16;
-          if (ca < ncol) st_nt(Gn + (size_t)(cb0 + ca) * n + row, mk(ar0[v], ai0[v]));
-          if (cb < ncol) st_nt(Gn + (size_t)(cb0 + cb) * n + row, mk(ar1[v], ai1[v]));
-        }
+      for (int t = 0; t < NT; ++t) x[t] = xn[t];
+    }
+    if (row < n) {
+#pragma unroll
+      for (int v = 0; v < 4 * NT; ++v) {
+        const int col = p0 + lk + 4 * v;
+        if (col < cn) st_nt(Gn + (unsigned)(col * n + row), mk(re[v >> 2][v & 3], im[v >> 2][v & 3]));
       }
     }
   }
 }
 
+// W = X G0(S, columns c0 .. c0 + cn - 1 of the own ones), 4m x cn with row stride ws, in
+// 16 x 16 tiles (row tile, column tile) dealt to the waves; X is 4m x 4m with row stride ldx.
+__device__ inline void window_w_mfma(const gcplx* __restrict__ Gc, cplx* W, int ws, const cplx* X, int ldx,
+                                     const int* accs, int m, int n, int N, int cb0, int c0, int cn) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const int nrt = (m + 3) >> 2, nct = (cn + 15) >> 4;
+  for (int t = wave; t < nrt * nct; t += nw) {
+    const int rt = t % nrt, ct = t / nrt;
+    const int col = min(16 * ct + li, cn - 1);
+    const gcplx* g = Gc + (size_t)(cb0 + c0 + col) * n + lk * N;
+    const cplx* x = X + min(16 * rt + li, 4 * m - 1) * ldx + lk;
+    v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+    for (int b0 = 0; b0 < m; b0 += 4) {
+      cplx gb[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) gb[u] = ld(g + accs[min(b0 + u, m - 1)]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (b0 + u < m) {
+          const cplx a = l16(x + 4 * (b0 + u));
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, gb[u].re, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, gb[u].im, im, 0, 0, 0);
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, gb[u].im, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, gb[u].re, im, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * rt + lk + 4 * v, wc = 16 * ct + li;
+      if (row < 4 * m && wc < cn) s16(W + (size_t)row * ws + wc, mk(re[v], im[v]));
+    }
+  }
+}
+
 template <bool TILE>
-__global__ __launch_bounds__(256) void k_local_updates_window(const ChainDesc* chains, int slice, const int* slices,
-                                                              double box, int dolog, int K, int lds_cap,
-                                                              const int* bmap) {
+__global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const ChainDesc* chains, int slice,
+                                                                      const int* slices, double box, int dolog, int K,
+                                                                      int lds_cap, const int* bmap) {
   // grid (W, chains), or with a block map a 1-D grid where block b serves chain bmap[b] & 0xFFFF
   // as workgroup (bmap[b] >> 16) & 0xFF of (bmap[b] >> 24) (workgroup counts per chain)
   const int bm = bmap ? bmap[blockIdx.x] : 0;
@@ -1042,297 +1221,512 @@ __global__ __launch_bounds__(256) void k_local_updates_window(const ChainDesc* c
   const ChainDesc& c = chains[ci];
   const int n = c.n, N = c.N;
   const int W = bmap ? (bm >> 24) & 0xFF : (int)gridDim.x, w = bmap ? (bm >> 16) & 0xFF : (int)blockIdx.x;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = slices ? slices[ci] : slice;
   const GroupSync g{c.bar_count, c.bar_gen, c.error, (unsigned int)W};
   const int cb0 = (int)(((long long)n * w) / W), cb1 = (int)(((long long)n * (w + 1)) / W);
-  const int ncol = cb1 - cb0;
-  const int ncs = window_bo_stride(n, W);
+  const int ncol = cb1 - cb0, ncm = (n + W - 1) / W;
   // K fits the largest chain of the launch; a smaller chain takes the largest window its own
   // layout fits in the allocated LDS (fewer windows, fewer passes of G)
   if (!TILE)
-    for (int k2 = kWinMaxGlob; k2 > K; --k2)
+    for (int k2 = kWinMax; k2 > K; k2 -= kWinStep)
       if (window_lds_bytes(n, N, W, k2, false) <= (size_t)lds_cap) {
         K = k2;
         break;
       }
-  const int K4 = 4 * K;
-
-  extern __shared__ double smem[];
-  const SliceLds s = load_slice(c, l, smem);
-  cplx* T = reinterpret_cast<cplx*>(smem + slice_lds_doubles(N));  // [ncs - 1][n] own columns (TILE)
-  cplx* Bo = T + (TILE ? (size_t)(ncs - 1) * n : 0);  // [K][4][ncs] B_b on own columns
-  // [K][4][ncs] H_j = G'(r_j, own) = G0(r_j, own) + sum_b A_b(r_j, :) B_b(:, own); W at a window's end
-  cplx* Hs = Bo + (size_t)K4 * ncs;
-  cplx* Gp = Hs + (size_t)K4 * ncs;  // [K][K][16]  G'(r_j, c_k)
-  cplx* Pc = Gp + (size_t)16 * K * K;  // [K][4K][4] P_b
-  cplx* Us = Pc + (size_t)16 * K * K;  // [K][4K][4] U_k = sum_b P_b B_b(:, c_k)
-  cplx* Bw = Us + (size_t)16 * K * K;  // [K][16]    B_m(:, c_k) of the update being applied
-  cplx* Ar = Bw + (size_t)16 * K;      // [K][16]    A_m(r_j, :)
-  __shared__ LocalShared sh;
-  __shared__ int accs[kWinMax];  // sites accepted in the current window, in order
-  gcplx* X[2] = {gp(c.mat[M_G]), gp(c.mat[M_GALT])};
   int R = (N + K - 1) / K;
-  R += R & 1;
+  if (TILE)
+    R = max(R, 2);
+  else
+    R += R & 1;
+  const int K4 = 4 * K, ldt = K4 + 1;
+
+  extern __shared__ __attribute__((aligned(16))) double win_smem[];
+  double* const smem = win_smem;
+  const WinSlice s = win_load_slice(c, l, smem);
+  cplx* own = reinterpret_cast<cplx*>(smem + win_slice_doubles(N));  // [ncm][n] own columns (TILE)
+  cplx* T = own + (TILE ? (size_t)ncm * n : 0);                      // [4K][4K + 1]
+  cplx* Aw = T + (size_t)K4 * ldt;                                   // [4K][4]
+  cplx* Bw = Aw + 4 * K4;                                            // [4][4K]
+  cplx* Pw = Bw + 4 * K4;                                            // [K (K + 1) / 2][7] proposals
+  cplx* Wb = Aw;                                                     // W, at the window's end (TILE)
+  __shared__ WinShared sh;
+  gcplx* X[2] = {gp(c.mat[M_G]), gp(c.mat[M_GALT])};
   if (TILE) {
     const gcplx* G0 = X[0] + (size_t)cb0 * n;
     const int tot = ncol * n;
-    for (int e0 = tid; e0 < tot; e0 += 4 * blockDim.x) {
+    for (int e0 = tid; e0 < tot; e0 += 4 * kWinThreads) {
       cplx v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = ld(G0 + min(e0 + q * (int)blockDim.x, tot - 1));
+      for (int q = 0; q < 4; ++q) v[q] = ld(G0 + min(e0 + q * kWinThreads, tot - 1));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (e0 + q * (int)blockDim.x < tot) {
-          T[e0 + q * blockDim.x].re = v[q].re;  // (whole-struct copies from a register array
-          T[e0 + q * blockDim.x].im = v[q].im;  // are lowered through a stack slot)
-        }
+        if (e0 + q * kWinThreads < tot) s16(own + e0 + q * kWinThreads, v[q]);
     }
-    __syncthreads();  // the first window's H rows are read from T
   }
+  if (tid == 0) sh.off = 0;
+  __syncthreads();
 
-  Proposals p{s.cur0, dolog ? *c.log_count : 0, 0.0, c.scal[S_MINRATIO], 0, 0, 0, -1, 0.0, 0.0, 0.0, 0.0};
-  int stop = 0;  // the uniform stream ran out: later windows make no proposals
+  if (wave == 0) __builtin_amdgcn_s_setprio(3);  // its chain bounds the window, its SIMD is shared
+  // Wave 0: row = 16-lane row of the wave, one of four consecutive sites; (ea, eb) = the entry
+  // of its 4 x 4 algebra. A rejection needs p_acc <= 1 and so always draws 4 uniforms, so row r
+  // knows the uniforms site i + r gets if the sites before it are rejected; the rows are resolved
+  // in order and the first acceptance drops the later ones' work.
+  const int row = lane >> 4, ea = (lane >> 2) & 3, eb = lane & 3;
+  const int em = (ea + eb) & 3;  // this lane's entry of delta is (ea, em), see below
+  const int dk = ea ^ em;
+  const bool mid = ea == 1 || ea == 2;
+  const double dsr = mid && dk >= 2 ? -1.0 : 1.0, dsi = mid && dk < 2 ? -1.0 : 1.0;
+  const double csg = (ea + eb) & 1 ? -1.0 : 1.0;
+  const bool odd = ea & 1;
+  const double k_space = 0.5 * c.dtau;
+  const int edrun = __builtin_amdgcn_readfirstlane(c.edrun);
+  const int umax = (int)max(s.navail - 4, 0ll), navail = (int)s.navail;
+  int coff = 0, nacc = 0, nonreal = 0, stop = 0;  // stop: the uniform stream ran out, no more proposals
+  double dS_acc = 0.0, minratio = c.scal[S_MINRATIO];
+  long long logi = dolog ? *c.log_count : 0;
+
   for (int rw = 0; rw < R; ++rw) {
     const int s0 = (int)((long long)rw * N / R), s1 = (int)((long long)(rw + 1) * N / R), kw = s1 - s0;
-    const gcplx* Gc = X[rw & 1];
-    gcplx* Gn = X[(rw + 1) & 1];
-    // Gp[j][k](a, b) = G(r_j + a N, c_k + b N) for the window's sites j, k; U = 0, H = 0
-    // eight loads per thread in flight before the first store (one HBM latency per 2048
-    // entries); the variant without LDS-resident columns has no registers to spare for it
-    if (!TILE)
-      for (int e = tid; e < kw * kw * 16; e += blockDim.x) {
-        const int jk = e >> 4, jj = jk / kw, kk = jk - jj * kw, a = (e >> 2) & 3, b = e & 3;
-        Gp[(jj * K + kk) * 16 + a * 4 + b] = ld(Gc + (size_t)(s0 + kk + b * N) * n + (s0 + jj + a * N));
-      }
-    for (int e0 = 0; TILE && e0 < kw * kw * 16; e0 += 8 * 256) {
-      cplx v[8];
+    const gcplx* Gc = TILE ? X[rw > 0] : X[rw & 1];
+    const int off0 = sh.off;
+    // T = G(r_j, c_k) between the window's sites (consecutive lanes: consecutive rows), the
+    // proposals while the first loads are under way
+    {
+      const int tot = kw * kw * 16, tid = opaque(threadIdx.x);
+      auto src = [&](int e) {
+        const int jj = e % kw, t = e / kw, a = t & 3, b = (t >> 2) & 3, kk = t >> 4;
+        return Gc + (size_t)(s0 + kk + b * N) * n + (s0 + jj + a * N);
+      };
+      auto dst = [&](int e) {
+        const int jj = e % kw, t = e / kw, a = t & 3, b = (t >> 2) & 3, kk = t >> 4;
+        return T + (size_t)(4 * jj + a) * ldt + 4 * kk + b;
+      };
+      cplx v[5];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int e = min(e0 + tid + 256 * j, kw * kw * 16 - 1);
-        const int jk = e >> 4, jj = jk / kw, kk = jk - jj * kw, a = (e >> 2) & 3, b = e & 3;
-        v[j] = ld(Gc + (size_t)(s0 + kk + b * N) * n + (s0 + jj + a * N));
+      for (int q = 0; q < 5; ++q) v[q] = ld(src(min(tid + q * kWinThreads, tot - 1)));
+      for (int e = tid; e < kw * kw; e += kWinThreads) {
+        const int jj = e / kw, d = e - jj * kw;
+        if (d <= jj) win_proposal(c, s, s0 + jj, off0 + 4 * jj - d, box, Pw + 7 * (win_entries(jj) + d));
       }
+      for (int e0 = tid; e0 < tot; e0 += 5 * kWinThreads) {
+        cplx nv[5];
+        if (e0 + 5 * kWinThreads < tot) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int e = e0 + tid + 256 * j;
-        if (e < kw * kw * 16) {
-          const int jk = e >> 4, jj = jk / kw, kk = jk - jj * kw, a = (e >> 2) & 3, b = e & 3;
-          Gp[(jj * K + kk) * 16 + a * 4 + b] = v[j];
+          for (int q = 0; q < 5; ++q) nv[q] = ld(src(min(e0 + (5 + q) * kWinThreads, tot - 1)));
         }
-      }
-    }
-    for (int e = tid; e < kw * K4 * 4; e += blockDim.x) Us[e] = mk(0, 0);
-    // H_j starts as the window's row r_j of G0 on the own columns (so an acceptance reads its
-    // site's rows from LDS); four loads per thread in flight
-    for (int e0 = tid; e0 < kw * 4 * ncs; e0 += 4 * blockDim.x) {
-      cplx v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = min(e0 + u * (int)blockDim.x, kw * 4 * ncs - 1);
-        const int jq = e / ncs, jl = min(e - jq * ncs, ncol - 1), row = s0 + (jq >> 2) + (jq & 3) * N;
-        v[u] = TILE ? T[(size_t)jl * n + row] : ld(Gc + (size_t)(cb0 + jl) * n + row);
-      }
+        for (int q = 0; q < 5; ++q)
+          if (e0 + q * kWinThreads < tot) s16(dst(e0 + q * kWinThreads), v[q]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = e0 + u * (int)blockDim.x;
-        if (e < kw * 4 * ncs) {
-          Hs[e].re = v[u].re;
-          Hs[e].im = v[u].im;
-        }
+        for (int q = 0; q < 5; ++q) v[q] = nv[q];
       }
     }
     __syncthreads();
-    // Per accepted proposal m at window site ii, two barriers: after the evaluation (S1) and
-    // after the factor pair (S2). The sums kept for the sites ahead are then brought up to date
-    // while wave 0 already evaluates the next proposals: wave 0 updates the diagonal blocks
-    // G'(r_j, c_j) it reads, waves 1-3 everything else (off-diagonal blocks, U, H); the next
-    // S1 completes both before the factor pair of the next acceptance reads them.
-    int m = 0, pend = -1;  // pend: window site of the acceptance whose sums are still to update
-    while (!stop) {
-      if (tid < 64) {
-        const int lane = tid & 63, ea = (lane & 15) >> 2, eb = lane & 3;
-        if (pend >= 0) {  // G'(r_j, c_j) += A_m(r_j, :) B_m(:, c_j), j > pend
-          const int ka = kw - pend - 1;
-          for (int e = lane; e < ka * 16; e += 64) {
-            const int jj = pend + 1 + (e >> 4), a = (e >> 2) & 3, b = e & 3;
-            cplx acc = Gp[(jj * K + jj) * 16 + a * 4 + b];
+
+    int m = 0, pend = -1, par = 0;  // pend: window site of the acceptance T is still to be updated with
+    int i = stop ? s1 : s0;         // wave 0: the first site not decided
+    // wave 0: what the next four proposals need besides G
+    cplx dm = mk(0, 0), gpre = mk(0, 0);
+    double n0 = 0, n1 = 0, n2 = 0, ex = 0, u3 = 0;
+    auto prepare = [&]() __attribute__((always_inline)) {
+      const int si = min(i + row, s1 - 1), jj = si - s0;
+      const int d = min(max(off0 + 4 * jj - (coff + 4 * row), 0), jj);
+      const cplx* e = Pw + 7 * (win_entries(jj) + d);
+      const cplx dv = l16(e + dk), f0 = l16(e + 4), f1 = l16(e + 5), f2 = l16(e + 6);
+      gpre = l16(T + (4 * jj + ea) * ldt + 4 * jj + eb);
+      const double *sb = s.snb + 3 * si, *ph = s.phl + 3 * si;
+      const double b0 = sb[0], b1 = sb[1], b2 = sb[2], h0 = ph[0], h1 = ph[1], h2 = ph[2];
+      u3 = s.ul[min(coff + 4 * row, umax) + 3];
+      __builtin_amdgcn_sched_barrier(0);
+      dm = mk(dsr * dv.re, dsi * dv.im);
+      n0 = f0.re;
+      n1 = f0.im;
+      n2 = f1.re;
+      const double ds = b0 * (n0 - h0) + b1 * (n1 - h1) + b2 * (n2 - h2);
+      double dS = f2.im;
+      if (!edrun) dS += f1.im + k_space * (f2.re - 2.0 * ds);
+      ex = exp(-dS);
+    };
+    if (wave == 0) prepare();
+    for (;; par ^= 1) {
+      if (wave == 0) {
+        int site = s1;
+        if (i < s1) {
+          const int jj = min(i + row, s1 - 1) - s0;
+          cplx gv = gpre;
+          if (pend >= 0) {
+            cplx av[4], bv[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) cfma(acc, Ar[jj * 16 + a * 4 + q], Bw[jj * 16 + q * 4 + b]);
-            Gp[(jj * K + jj) * 16 + a * 4 + b] = acc;
+            for (int q = 0; q < 4; ++q) {
+              av[q] = l16(Aw + (4 * jj + ea) * 4 + q);
+              bv[q] = l16(Bw + q * K4 + 4 * jj + eb);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cfma(gv, av[q], bv[q]);
           }
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the wave's writes before its reads
+          // M(ea, eb) = 1 + sum_j delta(ea, ea - j) (1 - G)(ea - j, eb), indices mod 4: quad
+          // broadcasts of the skewed delta, row rotations of 1 - G
+          const cplx gm = mk((ea == eb ? 1.0 : 0.0) - gv.re, -gv.im);
+          cplx mm = mk(ea == eb ? 1.0 : 0.0, 0);
+          cfma(mm, dpp_c<0x00>(dm), gm);
+          cfma(mm, dpp_c<0xFF>(dm), dpp_c<0x124>(gm));
+          cfma(mm, dpp_c<0xAA>(dm), dpp_c<0x128>(gm));
+          cfma(mm, dpp_c<0x55>(dm), dpp_c<0x12C>(gm));
+          // 2 x 2 minors of rows (ea, ea + 1): columns (eb, eb + 1) and (eb, eb + 2), all mod 4
+          const cplx y = dpp_c<0x12C>(mm);
+          const cplx a1 = mm * dpp_c<0x39>(y) - dpp_c<0x39>(mm) * y;
+          const cplx a2 = mm * dpp_c<0x4E>(y) - dpp_c<0x4E>(mm) * y;
+          // cofactor of (ea, eb): row ea ^ 1 against the minors of the other pair of rows (held by
+          // rows 0 and 2)
+          // (the moves need all lanes active, so they stand outside the selections)
+          const cplx p1 = dpp_c<0x12C>(a1), q1 = dpp_c<0x128>(a1), p2 = dpp_c<0x12C>(a2), q2 = dpp_c<0x128>(a2);
+          const cplx yo = dpp_c<0x124>(mm);
+          const cplx b1 = odd ? p1 : q1, b2 = odd ? p2 : q2, pr = odd ? yo : y;
+          cplx cof = dpp_c<0x39>(pr) * dpp_c<0x4E>(b1);
+          cof = cof - dpp_c<0x4E>(pr) * dpp_c<0x39>(b2);
+          cfma(cof, dpp_c<0x93>(pr), dpp_c<0x39>(b1));
+          cof = csg * cof;
+          cplx det = mm * cof;  // summed over the row's four columns
+          det = det + dpp_c<0xB1>(det);
+          det = det + dpp_c<0x4E>(det);
+          const double p = ex * det.re;
+          const bool here = i + row < s1, room = coff + 4 * row + 4 <= navail;
+          const bool acc = here && room && (p > 1.0 || u3 < p);
+          const unsigned long long ev = __ballot(acc || (here && !room)) & 0x0001000100010001ull;
+          const int first = ev ? (__ffsll(ev) - 1) >> 4 : 4;  // the row that ends the round
+          const unsigned long long av = __ballot(acc);
+          const bool got = first < 4 && ((av >> (16 * first)) & 1);
+          // statistics of the proposals made: rows up to `first` (without it if the stream ended)
+          const bool made = here && (row < first || (row == first && got));
+          const int nmade = __popcll(__ballot(made) & 0x0001000100010001ull);
+          if (made) {
+            if (fabs(det.im) > 1e-4 * fabs(det.re)) ++nonreal;
+            if (!(p > 1.0)) minratio = fmin(minratio, fabs(p - u3));
+            if (dolog && w == 0 && (lane & 15) == 0 && logi + row < c.log_cap) {
+              double* lg = c.prop_log + 4 * (logi + row);
+              lg[0] = p;
+              lg[1] = p > 1.0 ? -1.0 : u3;
+              lg[2] = acc;
+              lg[3] = det.im / det.re;
+            }
+          }
+          logi += nmade;
+          if (got) {
+            site = i + first;
+            if (row == first) {
+              // M^-1(eb, ea) = cofactor / det, scaled against overflow of |det|^2
+              const int e2 = -__builtin_amdgcn_frexp_exp(fmax(fabs(det.re), fabs(det.im)));
+              const double dr = ldexp(det.re, e2), di = ldexp(det.im, e2);
+              const double inv = 1.0 / (dr * dr + di * di);
+              const cplx v = cof * mk(dr * inv, -di * inv);
+              s16(sh.minv + eb * 4 + ea, mk(ldexp(v.re, e2), ldexp(v.im, e2)));
+              s16(sh.delta + ea * 4 + em, dm);
+              if ((lane & 15) == 0) {
+                sh.accs[m] = site;
+                sh.acce[m] = ex;
+                s.phl[3 * site] = n0;
+                s.phl[3 * site + 1] = n1;
+                s.phl[3 * site + 2] = n2;
+              }
+            }
+            const bool big = (__ballot(p > 1.0) >> (16 * first)) & 1;
+            coff += 4 * first + (big ? 3 : 4);
+            ++nacc;
+          } else if (first < 4) {  // the stream ended at row `first`
+            stop = 1;
+            coff += 4 * first;
+          } else {
+            coff += 4 * nmade;
+            i += 4;
+            if (i < s1) site = -1;
+          }
         }
-        int st;
-        const int site = evaluate_proposals(
-            c, s, p, sh, box, dolog, w == 0,
-            [&](int j) { return Gp[((j - s0) * (K + 1)) * 16 + ea * 4 + eb]; }, &st, s1, true);
-        if (tid == 0) {
-          sh.site = site;
-          sh.stop = st;
+        if (lane == 0) {
+          sh.site[par] = site;
+          sh.off = coff;
         }
       } else if (pend >= 0) {
-        // the pending acceptance (index m - 1) for the sites ahead (j, k > pend):
-        //   G'(r_j, c_k) += A(r_j, :) B(:, c_k) (j != k),  U_k += P B(:, c_k),  H_j += A(r_j, :) B(:, own)
-        const int t3 = tid - 64, n3 = blockDim.x - 64, mp = m - 1;
-        const int ka = kw - pend - 1;
-        for (int e = t3; e < ka * ka * 16; e += n3) {
-          const int jk = e >> 4, jj = pend + 1 + jk / ka, kk = pend + 1 + jk % ka, a = (e >> 2) & 3, b = e & 3;
-          if (jj == kk) continue;
-          cplx acc = Gp[(jj * K + kk) * 16 + a * 4 + b];
+        // T_jk += A_j B_k; the row and the column of the accepted site start from zero. (K is a
+        // multiple of 4, so tiles stay inside T; what they hold beyond the window's sites is
+        // never read.) All LDS reads of a tile go out before the first use.
+        const int lz = opaque(lane), li = lz & 15, lk = lz >> 4;
+        const int nt = (kw + 3) >> 2, per = (256 + nt - 1) / nt;
+        const cplx* al = Aw + 4 * li + lk;
+        const cplx* bl = Bw + lk * K4 + li;
+        cplx* tl = T + lk * ldt + li;
+        for (int t = wave - 1; t < nt * nt; t += kWinThreads / 64 - 1) {
+          const int ti = (t * per) >> 8, tj = t - ti * nt;  // t / nt for t < 25
+          const cplx a = l16(al + 64 * ti), b = l16(bl + 16 * tj);
+          cplx* tt = tl + 16 * (ti * ldt + tj);
+          cplx o[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) cfma(acc, Ar[jj * 16 + a * 4 + q], Bw[kk * 16 + q * 4 + b]);
-          Gp[(jj * K + kk) * 16 + a * 4 + b] = acc;
-        }
-        const int nu = 16 * m;
-        for (int e = t3; e < ka * nu; e += n3) {
-          const int kk = pend + 1 + e / nu, r2 = e % nu, t = r2 >> 2, q = r2 & 3;
-          cplx acc = Us[((size_t)kk * K4 + t) * 4 + q];
+          for (int v = 0; v < 4; ++v) o[v] = l16(tt + 4 * v * ldt);
+          __builtin_amdgcn_sched_barrier(0);
+          const bool zc = 4 * tj + (li >> 2) == pend;
+          v4d re, im;
 #pragma unroll
-          for (int q2 = 0; q2 < 4; ++q2) cfma(acc, Pc[((size_t)mp * K4 + t) * 4 + q2], Bw[kk * 16 + q2 * 4 + q]);
-          Us[((size_t)kk * K4 + t) * 4 + q] = acc;
-        }
-        const int nh = 4 * ncol;
-        for (int e = t3; e < ka * nh; e += n3) {
-          const int jj = pend + 1 + e / nh, r2 = e % nh, q = r2 / ncol, jl = r2 - q * ncol;
-          cplx acc = Hs[((size_t)jj * 4 + q) * ncs + jl];
+          for (int v = 0; v < 4; ++v) {
+            const bool z = zc || 4 * ti + v == pend;
+            re[v] = z ? 0.0 : o[v].re;
+            im[v] = z ? 0.0 : o[v].im;
+          }
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) cfma(acc, Ar[jj * 16 + q * 4 + k], Bo[((size_t)mp * 4 + k) * ncs + jl]);
-          Hs[((size_t)jj * 4 + q) * ncs + jl] = acc;
+          for (int v = 0; v < 4; ++v) s16(tt + 4 * v * ldt, mk(re[v], im[v]));
         }
       }
-      __syncthreads();  // S1
-      const int site = sh.site;
-      stop = sh.stop;
+      __syncthreads();  // S1: decision made, T up to date
+      const int site = sh.site[par];
       if (site >= s1) break;
+      if (site < 0) {  // four rejections: the next four (T stays as it is)
+        pend = -1;
+        if (wave == 0) prepare();
+        continue;
+      }
       const int ii = site - s0;
-      if (tid < 64) {
-        // wave 0: the accepted proposal's field update, while waves 1-3 form its factor pair
-        commit_accept(c, s, p);
-      } else {
-        const int t3 = tid - 64, n3 = blockDim.x - 64;
-        // B_m on own columns: delta G'(r_i, own) = delta H_i
-        for (int jl = t3; jl < ncol; jl += n3) {
-          cplx g4[4];
+      if (wave == 0) {
+        // the four neighbours' space sums, in the original order (action.jl:57-101), then the
+        // next proposals
+        if (lane < 12) {
+          const int j = s.nbl[(lane / 3) * N + site], a = lane - 3 * (lane / 3);
+          int jn[4];
+          double f[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) g4[q] = Hs[((size_t)ii * 4 + q) * ncs + jl];
+          for (int k = 0; k < 4; ++k) jn[k] = s.nbl[k * N + j];
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            cplx acc = mk(0, 0);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cfma(acc, sh.delta[k * 4 + q], g4[q]);
-            Bo[((size_t)m * 4 + k) * ncs + jl] = acc;
-          }
+          for (int k = 0; k < 4; ++k) f[k] = s.phl[3 * jn[k] + a];
+          __builtin_amdgcn_sched_barrier(0);
+          s.snb[3 * j + a] = ((f[0] + f[1]) + f[2]) + f[3];
         }
-        // B_m(:, c_k) = delta G'(r_i, c_k) and A_m(r_j, :) = G'(r_j, c_i) M^-1 for the sites
-        // ahead (j, k > i: the only ones read again)
-        for (int e = t3; e < kw * 16; e += n3) {
-          const int kk = e >> 4, k = (e >> 2) & 3, b = e & 3;
-          if (kk <= ii) continue;
-          cplx bw = mk(0, 0), ar = mk(0, 0);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the sums before they are read
+        i = site + 1;
+        if (i < s1) prepare();
+      } else {
+        // A_j = T_ji M^-1 (A_i = M^-1) and B_k = delta T_ik (B_i = delta)
+        for (int e = opaque(tid) - 64; e < 32 * kw; e += kWinThreads - 64) {
+          const bool h = e >= 16 * kw;
+          const int f = h ? e - 16 * kw : e, b = f & 3, a = (f >> 2) & 3, j = f >> 4;
+          const cplx* tv = T + (h ? 4 * ii * ldt + 4 * j + b : (4 * j + a) * ldt + 4 * ii);
+          const cplx* sv = h ? sh.delta + 4 * a : sh.minv + b;
+          const int ts = h ? ldt : 1, ss = h ? 1 : 4;
+          cplx x[4], z[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            cfma(bw, sh.delta[k * 4 + q], Gp[(ii * K + kk) * 16 + q * 4 + b]);
-            cfma(ar, Gp[(kk * K + ii) * 16 + k * 4 + q], sh.minv[q * 4 + b]);
+            x[q] = l16(tv + q * ts);
+            z[q] = l16(sv + q * ss);
           }
-          Bw[kk * 16 + k * 4 + b] = bw;
-          Ar[kk * 16 + k * 4 + b] = ar;
-        }
-        // P_m = (S_m + U_i) M^-1 (rows of blocks <= m)
-        for (int e = t3; e < 16 * (m + 1); e += n3) {
-          const int t = e >> 2, k = e & 3;
+          const cplx one = l16((h ? sh.delta : sh.minv) + 4 * a + b);
+          __builtin_amdgcn_sched_barrier(0);
           cplx acc = mk(0, 0);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            cplx v = Us[((size_t)ii * K4 + t) * 4 + q];
-            if (t == 4 * m + q) v.re += 1.0;
-            cfma(acc, v, sh.minv[q * 4 + k]);
-          }
-          Pc[((size_t)m * K4 + t) * 4 + k] = acc;
+          for (int q = 0; q < 4; ++q) cfma(acc, x[q], z[q]);
+          cplx* out = h ? Bw + a * K4 + 4 * j + b : Aw + (4 * j + a) * 4 + b;
+          s16(out, j == ii ? one : acc);
         }
-        if (t3 == 0) accs[m] = site;
       }
-      __syncthreads();  // S2
+      __syncthreads();  // S2: A, B
       pend = ii;
       ++m;
     }
-    // W = sum_b P_b B_b (into the H storage, no longer needed): entry (t, jl) sums over the b
-    // with P_b nonzero in row t (b >= t / 4)
-    cplx* Wb = Hs;
-    for (int e = tid; e < 4 * m * ncol; e += blockDim.x) {
-      const int t = e / ncol, jl = e - t * ncol;
-      cplx acc = mk(0, 0);
-      for (int b = t >> 2; b < m; ++b) {
-        const cplx* pb = Pc + ((size_t)b * K4 + t) * 4;
-        const cplx* bo = Bo + (size_t)b * 4 * ncs + jl;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cfma(acc, pb[q], bo[(size_t)q * ncs]);
-      }
-      Wb[(size_t)t * ncs + jl] = acc;
+    // p.boson_action += -log(exp_delta_S_boson) (local_updates.jl:34), in the order of acceptance
+    if (w == 0 && wave == 0) {
+      const double lg = -log(lane < m ? sh.acce[min(lane, kWinMax - 1)] : 1.0);
+      for (int b = 0; b < m; ++b) dS_acc += read_lane(lg, b);
     }
-    __syncthreads();
-    // own columns of the partner buffer: G0 + Yt W (a plain copy when m = 0)
     if (TILE) {
-      for (int r = tid; r < n; r += blockDim.x)
+      // publish the next window's columns, or the slice's result; W is formed in between, with the
+      // first loads of Yt under way. One row per thread and three accepted sites ahead up to
+      // n = 512, else two rows (W is then read from LDS half as often) and one ahead.
+      const bool last = rw + 1 == R;
+      const int e1 = last ? N : (int)((long long)(rw + 2) * N / R);
+      gcplx* Gn = last ? X[0] : X[1];
+      auto finish = [&](auto rows, auto depth) __attribute__((always_inline)) {
+        constexpr int NR = decltype(rows)::value, DP = decltype(depth)::value;
+        const int r = opaque(tid);
+        int rr[NR];
+#pragma unroll
+        for (int h = 0; h < NR; ++h) rr[h] = min(r + h * kWinThreads, n - 1);
+        auto loady = [&](int b, cplx (&y)[NR][4]) __attribute__((always_inline)) {
+          const int site = __builtin_amdgcn_readfirstlane(sh.accs[min(b, m - 1)]);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const gcplx* col = Gc + (size_t)(site + k * N) * n;
+#pragma unroll
+            for (int h = 0; h < NR; ++h) y[h][k] = ld(col + (unsigned)rr[h]);
+          }
+        };
+        cplx y[DP + 1][NR][4];
+        if (m > 0) {
+#pragma unroll
+          for (int d = 0; d < DP; ++d) loady(d, y[d]);
+        }
+        // W = X G0(S, own), X(4b + a, 4b' + a') = T's block of the accepted sites b, b': four lanes
+        // per entry, lane q of a quad sums column q of the blocks
+        const int lq = r & 3;
+        for (int e = r; e < ((16 * m * ncol + 63) & ~63); e += kWinThreads) {
+          const int en = min(e >> 2, 4 * m * ncol - 1), t = en / ncol, jl = en - t * ncol;
+          const cplx* x = T + (4 * (sh.accs[t >> 2] - s0) + (t & 3)) * ldt + lq;
+          const cplx* o = own + jl * n + lq * N;
+          cplx acc = mk(0, 0);
+          for (int b0 = 0; b0 < m; b0 += 4) {
+            int site[4];
+            cplx xv[4], ov[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) site[u] = sh.accs[min(b0 + u, m - 1)];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              xv[u] = l16(x + 4 * (site[u] - s0));
+              ov[u] = l16(o + site[u]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (b0 + u < m) cfma(acc, xv[u], ov[u]);
+          }
+          acc = acc + dpp_c<0xB1>(acc);
+          acc = acc + dpp_c<0x4E>(acc);
+          if (e < 16 * m * ncol && lq == 0) s16(Wb + en, acc);
+        }
+        __syncthreads();
+        if (r >= n) return;
         for (int j0 = 0; j0 < ncol; j0 += 4) {
-          cplx acc[4];
+          int jc[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) acc[q] = T[(size_t)min(j0 + q, ncol - 1) * n + r];
-          // Yt's row r for accepted site b + 1 is loaded while site b's products are formed
-          cplx yn[4];
-          const int a0 = m > 0 ? accs[0] : 0;  // (accs[0] is unset in a window without acceptances)
+          for (int q = 0; q < 4; ++q) jc[q] = min(j0 + q, ncol - 1);
+          cplx acc[NR][4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) yn[k] = ld(Gc + (size_t)(a0 + k * N) * n + r);
-          for (int b = 0; b < m; ++b) {
-            cplx y[4];
+          for (int h = 0; h < NR; ++h)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              y[k] = yn[k];
-              if (r == accs[b] + k * N) y[k].re -= 1.0;
-            }
-            const int bn = min(b + 1, m - 1);
+            for (int q = 0; q < 4; ++q) acc[h][q] = l16(own + jc[q] * n + rr[h]);
+          if (j0 > 0 && m > 0) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) yn[k] = ld(Gc + (size_t)(accs[bn] + k * N) * n + r);
+            for (int d = 0; d < DP; ++d) loady(d, y[d]);
+          }
+          for (int b0 = 0; b0 < m; b0 += DP + 1) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const cplx* wr = Wb + ((size_t)b * 4 + k) * ncs;
+            for (int d = 0; d <= DP; ++d)
+              if (b0 + d < m) {  // (uniform) site b0 + d is in slot d, the free slot takes DP ahead
+                loady(b0 + d + DP, y[(d + DP) % (DP + 1)]);
+                const int site = __builtin_amdgcn_readfirstlane(sh.accs[b0 + d]);
+                cplx wv[4][4];
 #pragma unroll
-              for (int q = 0; q < 4; ++q) cfma(acc[q], y[k], wr[min(j0 + q, ncol - 1)]);
-            }
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                  for (int q = 0; q < 4; ++q) wv[k][q] = l16(Wb + (4 * (b0 + d) + k) * ncol + jc[q]);
+#pragma unroll
+                for (int h = 0; h < NR; ++h)
+#pragma unroll
+                  for (int k = 0; k < 4; ++k) {
+                    cplx yv = y[d][h][k];
+                    if (site + k * N == rr[h]) yv.re -= 1.0;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) cfma(acc[h][q], yv, wv[k][q]);
+                  }
+              }
           }
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             if (j0 + q < ncol) {
-              T[(size_t)(j0 + q) * n + r].re = acc[q].re;
-              T[(size_t)(j0 + q) * n + r].im = acc[q].im;
-              st_nt(Gn + (size_t)(cb0 + j0 + q) * n + r, acc[q]);
+              const int col = cb0 + j0 + q, cs = col % N;
+              const bool pub = last || (cs >= s1 && cs < e1);
+#pragma unroll
+              for (int h = 0; h < NR; ++h)
+                if (r + h * kWinThreads < n) {
+                  s16(own + (j0 + q) * n + rr[h], acc[h][q]);
+                  if (pub) st_nt(Gn + (size_t)col * n + rr[h], acc[h][q]);
+                }
             }
         }
-    } else if (m == 0) {
-      for (int e = tid; e < ncol * n; e += blockDim.x) {
-        st_nt(Gn + (size_t)cb0 * n + e, ld(Gc + (size_t)cb0 * n + e));
-      }
+      };
+      using std::integral_constant;
+      if (n <= kWinThreads)
+        finish(integral_constant<int, 1>{}, integral_constant<int, 3>{});
+      else
+        finish(integral_constant<int, 2>{}, integral_constant<int, 1>{});
     } else {
-      window_end_mfma(Gc, Gn, Wb, accs, m, n, N, cb0, ncol, ncs);
+      gcplx* Gn = X[(rw + 1) & 1];
+      if (m == 0) {
+        for (int e = tid; e < ncol * n; e += kWinThreads) {
+          st_nt(Gn + (size_t)cb0 * n + e, ld(Gc + (size_t)cb0 * n + e));
+        }
+      } else {
+        // X alone takes T's place, so that W fits for all own columns or for few equal chunks of
+        // them in what is left. The accepted sites ascend, so no entry moves up and none is written
+        // where a later one is still to be read.
+        const int tz = opaque(tid), m4 = 4 * m, ldx = m4 + 1;
+        for (int e0 = 0; e0 < m4 * m4; e0 += 2 * kWinThreads) {
+          cplx xr[2];
+          int xd[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int e = min(e0 + u * kWinThreads + tz, m4 * m4 - 1), xi = e / m4, xj = e - xi * m4;
+            xd[u] = xi * ldx + xj;
+            xr[u] = l16(T + (4 * (sh.accs[xi >> 2] - s0) + (xi & 3)) * ldt + 4 * (sh.accs[xj >> 2] - s0) + (xj & 3));
+          }
+          __syncthreads();
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            if (e0 + u * kWinThreads + tz < m4 * m4) s16(T + xd[u], xr[u]);
+        }
+        cplx* Wn = T + m4 * ldx;
+        const int fit = (int)((lds_cap - ((char*)Wn - (char*)smem)) / (64 * m));
+        const int most = ncol <= fit ? ncol : fit & ~15;
+        const int parts = (ncol + most - 1) / most;
+        const int cs = parts == 1 ? ncol : min(most, ((ncol + parts - 1) / parts + 15) & ~15);
+        for (int c0 = 0; c0 < ncol; c0 += cs) {
+          const int cn = min(cs, ncol - c0);
+          __syncthreads();
+          window_w_mfma(Gc, Wn, cs, T, ldx, sh.accs, m, n, N, cb0, c0, cn);
+          __syncthreads();
+          window_end_mfma(Gc, Gn, Wn, cs, sh.accs, m, n, N, cb0, c0, cn);
+        }
+      }
     }
     if (rw + 1 < R) {
       group_sync(g);
       if (group_failed(g)) return;
     }
   }
-  if (w == 0) finish_slice(c, l, s, p, dolog, stop);
+  // counters and the updated field slice, by workgroup 0 (the field is complete since the last S1)
+  if (w == 0) {
+    for (int e = tid; e < 3 * N; e += kWinThreads) c.phi[(size_t)3 * N * l + e] = s.phl[e];
+    if (wave == 0) {
+      for (int o = 16; o < 64; o += 16) {
+        nonreal += lane == 0 ? __builtin_amdgcn_readlane(nonreal, o) : 0;
+        minratio = fmin(minratio, read_lane(minratio, o));
+      }
+      if (lane == 0) {
+        *c.ucursor = s.cur0 + coff;
+        if (dolog) *c.log_count = logi;
+        c.scal[S_BOSON_ACTION] += dS_acc;
+        c.scal[S_ACC_SLICE] = nacc;
+        c.scal[S_ACC_TOTAL] += nacc;
+        c.scal[S_PROP_TOTAL] += N;
+        c.scal[S_NONREAL] += nonreal;
+        c.scal[S_MINRATIO] = minratio;
+        if (stop) *c.error = 2;
+      }
+    }
+  }
 }
 
 // the window of variant 4 at this shape: its K, and whether the own columns fit in LDS too
 // (preferred when the window keeps at least 4 sites); K = 0 when nothing fits
 int local_window_sites(int nmax, int wg, bool* tile) {
-  for (int K = kWinMax; K >= 4; --K)
+  for (int K = kWinMaxTile; K >= 4 && nmax <= 2 * kWinThreads; K -= kWinStep)
     if (window_lds_bytes(nmax, nmax / 4, wg, K, true) <= kWindowLdsMax) {
       if (tile) *tile = true;
       return K;
     }
   if (tile) *tile = false;
-  for (int K = kWinMaxGlob; K >= 2; --K)
+  for (int K = kWinMax; K >= kWinStep; K -= kWinStep)
     if (window_lds_bytes(nmax, nmax / 4, wg, K, false) <= kWindowLdsMax) return K;
   return 0;
 }
@@ -1359,7 +1753,7 @@ bool local_tile_fits(int nmax, int wg) { return local_lds_tile(nmax, nmax / 4, w
 int local_block_map(const std::vector<int>& n, std::vector<int>& map) {
   const int na = (int)n.size();
   auto kfit = [](int nn, int W) {
-    for (int K = kWinMaxGlob; K >= 2; --K)
+    for (int K = kWinMax; K >= kWinStep; K -= kWinStep)
       if (window_lds_bytes(nn, nn / 4, W, K, false) <= kWindowLdsMax) return K;
     return 0;
   };
@@ -1408,7 +1802,7 @@ hipError_t launch_local_updates(hipStream_t s, const ChainDesc* chains, int ncha
   if (bmap && variant != 4) return hipErrorInvalidValue;
   bool tile = false;
   // with a block map every chain sizes its own window (no LDS-resident columns)
-  int K = bmap ? 2 : variant == 4 ? local_window_sites(nmax, wg, &tile) : 0;
+  int K = bmap ? kWinStep : variant == 4 ? local_window_sites(nmax, wg, &tile) : 0;
   if (variant == 4 && K < 2) return hipErrorInvalidValue;
   const void* fn = variant == 2   ? (const void*)k_local_updates_tile
                    : variant == 3 ? (const void*)k_local_updates_delayed
@@ -1431,7 +1825,8 @@ hipError_t launch_local_updates(hipStream_t s, const ChainDesc* chains, int ncha
   void* args4[] = {(void*)&chains, (void*)&slice, (void*)&slices,  (void*)&box,
                    (void*)&log,    (void*)&K,     (void*)&lds_cap, (void*)&bmap};
   const dim3 grid = bmap ? dim3(nblocks, 1) : dim3(wg, nchains);
-  hipError_t e = hipLaunchCooperativeKernel(fn, grid, dim3(256), variant == 4 ? args4 : args1, lds, s);
+  hipError_t e = hipLaunchCooperativeKernel(fn, grid, dim3(variant == 4 ? kWinThreads : 256),
+                                            variant == 4 ? args4 : args1, lds, s);
   if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
