@@ -84,6 +84,7 @@ struct ChainMem {
   // time-displaced Green's function storage (dqmc_tdgf_alloc)
   cplx* tdgf_mat = nullptr;
   double* tdgf_vec = nullptr;
+  JobSet tdgf_jobs, meas_jobs;
   // global-update backup (gb_u/d/t_stack, gb_greens, gb_hsfield; stack.jl:134-143), one block
   double* gb = nullptr;
   // fermionic measurements (allocated on first use): the equal-time Green's function the
@@ -415,9 +416,10 @@ void chain_free(ChainMem& cm) {
   if (cm.uniforms) (void)hipFree(cm.uniforms);
   if (cm.log_buf) (void)hipFree(cm.log_buf);
   for (void* p : {(void*)cm.grad, (void*)cm.grad_ptr, (void*)cm.mom, (void*)cm.phi_bak, (void*)cm.tdgf_mat,
-                  (void*)cm.tdgf_vec, (void*)cm.gb, (void*)cm.meas, cm.grad_jobs.mem})
+                  (void*)cm.tdgf_vec, (void*)cm.gb, (void*)cm.meas, cm.grad_jobs.mem, cm.tdgf_jobs.mem,
+                  cm.meas_jobs.mem})
     if (p) (void)hipFree(p);
-  cm.grad_jobs = JobSet{};
+  cm.grad_jobs = cm.tdgf_jobs = cm.meas_jobs = JobSet{};
   cm.meas = cm.meas_etgf = cm.meas_tnb = cm.meas_part = cm.meas_res = nullptr;
   cm.has_etgf = cm.has_hopping = false;
   cm.tdgf_mat = nullptr;
@@ -2194,6 +2196,294 @@ int dqmc_effective_greens2greens(dqmc_ctx* ctx, double* G) {
   return check_device_error(ctx->b);
 }
 
+}  // extern "C"
+namespace {
+
+// Takes arrays out of one block: with base == nullptr it only adds up what they need.
+struct Carve {
+  char* base;
+  size_t off = 0;
+  template <class T>
+  T* take(size_t count) {
+    off = (off + 255) & ~(size_t)255;
+    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+    off += count * sizeof(T);
+    return p;
+  }
+};
+// the factorisation scratch, barrier words and scalars of one job
+void carve_scratch(Carve& cv, ChainDesc& d) {
+  const size_t n = d.n;
+  d.qr_vn = cv.take<double>(2 * n);
+  d.qr_cand = cv.take<cplx>((size_t)2 * kMaxWG * n);
+  d.qr_cand_norm = cv.take<double>(2 * kMaxWG);
+  d.qr_cand_pos = cv.take<int>(2 * kMaxWG);
+  d.qr_perm = cv.take<int>(n);
+  d.qr_lpos = cv.take<int>(n);
+  d.qr_tau = cv.take<cplx>(n);
+  d.qr_Tf = cv.take<cplx>(16 * (n + 16));
+  d.qr_flags = cv.take<unsigned int>(1 + (n + 7) / 8);
+  d.inv_piv = cv.take<int>(n);
+  d.inv_bcast = cv.take<cplx>(2 * n);
+  d.bar_count = cv.take<unsigned int>(2);
+  d.bar_gen = d.bar_count ? d.bar_count + 1 : nullptr;
+  d.scal = cv.take<double>(kNumScalar);
+}
+// descriptors and tables to the device, barrier words and scalars cleared
+hipError_t jobs_upload(JobSet& js, const ChainMem& cm, const std::vector<ChainDesc>& h, const std::vector<int>& ints) {
+  hipError_t e = hipMemcpy(js.d_desc, h.data(), h.size() * sizeof(ChainDesc), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(js.d_int, ints.data(), ints.size() * sizeof(int), hipMemcpyHostToDevice);
+  for (const auto& d : h) {
+    if (d.scal == cm.d.scal) continue;  // the chain itself
+    if (e == hipSuccess) e = hipMemset(d.bar_count, 0, 2 * sizeof(unsigned int));
+    if (e == hipSuccess) e = hipMemset(d.scal, 0, kNumScalar * sizeof(double));
+  }
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  return e;
+}
+// a group over `nj` jobs of g's chain on g's stream, the workgroups shared between them
+Group job_group(const Group& g, ChainDesc* d_desc, int nj) {
+  Group j;
+  j.n = g.n;
+  j.N = g.N;
+  j.L = g.L;
+  j.M = g.M;
+  j.s = g.s;
+  j.nelem = g.nelem;
+  j.chkr = g.chkr;
+  j.ngroups = g.ngroups;
+  j.all_checks = g.all_checks;
+  j.stream = g.stream;
+  j.d_desc = d_desc;
+  j.chains.assign(nj, 0);
+  j.greens_route = g.greens_route;
+  j.udt_route = g.udt_route;
+  j.qr_nb = g.qr_nb;
+  j.prof_mask = g.prof_mask;
+  const int per = std::max(1, 256 / nj);
+  j.wg_qr = std::max(1, std::min(g.wg_qr, per));
+  j.wg_inv = std::max((g.n + 511) / 512, std::min(g.wg_inv, per));
+  return j;
+}
+// its timing records go to the chain's group
+void job_group_done(Group& g, Group& j) {
+  g.prof.insert(g.prof.end(), j.prof.begin(), j.prof.end());
+  g.event_pool.insert(g.event_pool.end(), j.event_pool.begin(), j.event_pool.end());
+}
+
+// Time-displaced Green's functions as jobs. The four checkpoint chains do not depend on one
+// another, nor do the 2 R inversions (R = M / safe_mult) once the chains are there, nor the R
+// intervals of the fill. The sequential pass is 4 R + 4 R column-pivoted factorisations and 4 R
+// Gauss-Jordan inverses one after the other, each bound by a group barrier per column: here the
+// chains advance side by side (R pivoted factorisations deep), the inversions in one batch (at
+// most kMaxTdgfJobs at a time, which bounds the memory: four n x n and the scratch each) and the
+// intervals as one launch per slice. An inversion is
+//   [Ua Da Ta + Ub Db Tb]^-1 = Tb^-1 Dbp^-1 N^-1 Dap^-1 Ua^H,
+//   N = Dam Ta Tb^-1 Dbp^-1 + Dap^-1 Ua^H Ub Dbm, Dp = max(D, 1), Dm = min(D, 1),
+// as inv_sum_udts_scalettar, but as with calculate_greens_scalesep N is well conditioned and one
+// unpivoted QR and a solve take the place of two factorisations, an inverse and three products;
+// Tb^-1 likewise. [1 + U D T]^-1 of slice 1 is the case Ua = Da = Ta = 1. L = 8, M = 100:
+// measure_tdgfs 350 -> 42 ms.
+constexpr int kMaxTdgfJobs = 32;
+enum : int { TA_SRC, TA_SD, TA_DD, TA_Q, TA_T, TA_GC, TA_GA, TA_GB, kTdgfChainRoles };
+enum : int { TB_AU, TB_AD, TB_AT, TB_BU, TB_BD, TB_BT, TB_RES, TB_NEG, kTdgfInvRoles };
+
+struct TdgfLayout {
+  int R, sm, slots, rounds;
+  size_t chain_plan, inv_plan, fill_plan, chain_slices, sel, fill_slices, fill_sel;  // offsets into d_int
+  explicit TdgfLayout(const Group& g) {
+    R = g.M / g.s;
+    sm = g.s;
+    slots = std::min(2 * R, kMaxTdgfJobs);
+    rounds = (2 * R + slots - 1) / slots;
+    chain_plan = 0;
+    inv_plan = chain_plan + (size_t)4 * R * kTdgfChainRoles;
+    fill_plan = inv_plan + (size_t)slots * rounds * kTdgfInvRoles;
+    chain_slices = fill_plan + (size_t)2 * R * (sm - 1) * 2;
+    sel = chain_slices + (size_t)R * sm * 4;
+    fill_slices = sel + 2;
+    fill_sel = fill_slices + (size_t)(sm - 1) * R;
+  }
+};
+
+// the batched slice operators need a checkerboard; the fill from both sides of M / 2 meets at a
+// checkpoint for even R only; the verbatim routes keep the sequential pass
+bool tdgf_parallel_ok(const Group& g) {
+  return g.greens_route == 0 && g.udt_route == 0 && g.chkr && (g.M / g.s) % 2 == 0 && g.M % g.s == 0;
+}
+
+int tdgf_jobs_create(Group& g, ChainMem& cm) {
+  JobSet& js = cm.tdgf_jobs;
+  const TdgfLayout lo(g);
+  const Ops o(g);
+  const int R = lo.R, sm = lo.sm;
+  const size_t n = g.n, nn = n * n;
+  auto em = [](MatRef r) { return plan_enc(r.kind, r.idx); };
+  auto ev = [](VecRef r) { return plan_enc(r.kind, r.idx); };
+  std::vector<int> ints;
+  for (int q = 0; q < 4; ++q) {  // chains 0, 1 multiply from the right, 2, 3 from the left; 1, 3 run down
+    const bool rm = q < 2, down = q & 1;
+    for (int i = 0; i < R; ++i) {
+      const int k = down ? R - 1 - i : i, kp = i == 0 ? k : down ? k + 1 : k - 1;
+      const MatRef qo = rm ? (i == 0 ? o.XU(q, k) : NM(M_QRQ)) : o.XU(q, k);
+      const MatRef to = rm ? o.XT(q, k) : (i == 0 ? o.XT(q, k) : NM(M_QRT));
+      ints.insert(ints.end(), {em(rm ? o.XT(q, kp) : o.XU(q, kp)), ev(o.XD(q, kp)), ev(o.XD(q, k)), em(qo), em(to),
+                               em(rm ? o.XU(q, k) : o.XT(q, k)), em(rm ? o.XU(q, kp) : NM(M_QRT)),
+                               em(rm ? NM(M_QRQ) : o.XT(q, kp))});
+    }
+  }
+  for (int sl = 0; sl < lo.slots; ++sl)
+    for (int c = 0; c < lo.rounds; ++c) {
+      const int J = std::min(c * lo.slots + sl, 2 * R - 1), z = J / R, i = J % R, qa = 2 * z, qb = 2 * z + 1;
+      const MatRef res = z ? o.G0T(i * sm + 1) : o.GT0(i * sm + 1);
+      ints.insert(ints.end(),
+                  {em(i ? o.XU(qa, i - 1) : NM(M_IDENT)), ev(i ? o.XD(qa, i - 1) : NV(V_ONES)),
+                   em(i ? o.XT(qa, i - 1) : NM(M_IDENT)), em(o.XU(qb, i)), ev(o.XD(qb, i)), em(o.XT(qb, i)), em(res),
+                   z ? em(res) : -1});
+    }
+  auto fill_tau = [&](int i, int t) { return i >= R / 2 ? i * sm + 2 + t : (i + 1) * sm - t; };
+  for (int z = 0; z < 2; ++z)
+    for (int i = 0; i < R; ++i)
+      for (int t = 0; t < sm - 1; ++t) {
+        const int tau = fill_tau(i, t), from = i >= R / 2 ? tau - 1 : tau + 1;
+        ints.insert(ints.end(), {em(z ? o.G0T(tau) : o.GT0(tau)), em(z ? o.G0T(from) : o.GT0(from))});
+      }
+  for (int i = 0; i < R; ++i)
+    for (int j = 0; j < sm; ++j)
+      for (int q = 0; q < 4; ++q) ints.push_back(q & 1 ? (R - i) * sm - 1 - j : i * sm + j);
+  ints.push_back(0);
+  ints.push_back(1);
+  for (int t = 0; t < sm - 1; ++t)
+    for (int i = 0; i < R; ++i) ints.push_back(i >= R / 2 ? fill_tau(i, t) - 1 : fill_tau(i, t));
+  for (int i = 0; i < R; ++i) ints.push_back(i >= R / 2 ? 0 : 1);
+  std::vector<ChainDesc> h;
+  auto layout = [&](Carve& cv) {
+    h.assign(4 + lo.slots + 2 * R, cm.d);
+    js.d_desc = cv.take<ChainDesc>(h.size());
+    js.d_int = cv.take<int>(ints.size());
+    for (int j = 0; j < 4 + lo.slots + 2 * R; ++j) {
+      ChainDesc& d = h[j];
+      if (j < 4) {
+        carve_scratch(cv, d);
+        for (int m : {M_CURU, M_QRQ, M_QRT}) d.mat[m] = cv.take<cplx>(nn);
+        d.plan = js.d_int + lo.chain_plan + (size_t)j * R * kTdgfChainRoles;
+      } else if (j < 4 + lo.slots) {
+        carve_scratch(cv, d);
+        for (int m : {M_TMP, M_TMP2, M_TMP3, M_QRT}) d.mat[m] = cv.take<cplx>(nn);
+        for (int v : {V_D1, V_D2, V_D3, V_D4, V_D5}) d.vec[v] = cv.take<double>(n);
+        d.plan = js.d_int + lo.inv_plan + (size_t)(j - 4) * lo.rounds * kTdgfInvRoles;
+      } else {
+        d.plan = js.d_int + lo.fill_plan + (size_t)(j - 4 - lo.slots) * (sm - 1) * 2;
+      }
+    }
+  };
+  Carve size{nullptr};
+  layout(size);
+  if (hipMalloc(&js.mem, size.off) != hipSuccess) {
+    (void)hipGetLastError();
+    js = JobSet{};
+    js.failed = true;
+    return 0;
+  }
+  Carve cv{(char*)js.mem};
+  layout(cv);
+  const hipError_t e = jobs_upload(js, cm, h, ints);
+  if (e != hipSuccess) {
+    (void)hipFree(js.mem);
+    js = JobSet{};
+    return fail(DQMC_E_HIP, std::string("time-displaced jobs: ") + hipGetErrorString(e));
+  }
+  return 0;
+}
+
+int tdgf_parallel(Group& g, ChainMem& cm) {
+  JobSet& js = cm.tdgf_jobs;
+  const TdgfLayout lo(g);
+  const int R = lo.R, sm = lo.sm, n = g.n, N = g.N;
+  hipStream_t st = g.stream;
+  auto pm = [](int base, int role) { return MatRef{MK_PLAN, base + role}; };
+  auto pv = [](int base, int role) { return VecRef{VK_PLAN, base + role}; };
+  const int* sel = js.d_int + lo.sel;
+  const MatRef cur = NM(M_CURU);
+  {
+    // the chains (bchain_udts), 0 and 1 with operators from the right, 2 and 3 from the left
+    ChainDesc *dr = js.d_desc, *dl = js.d_desc + 2;
+    Group all = job_group(g, js.d_desc, 4);
+    Ops o(all);
+    for (int i = 0; i < R; ++i) {
+      const int b = i * kTdgfChainRoles;
+      if (i == 0)
+        LCHK(launch_identity(st, js.d_desc, 4, n, cur, NOVEC));
+      else
+        RC(o.copy(cur, pm(b, TA_SRC)));
+      {
+        ProfScope ps(all, DQMC_K_APPLY_B);
+        for (int j = 0; j < sm; ++j) {
+          const int* sl = js.d_int + lo.chain_slices + (size_t)(i * sm + j) * 4;
+          LCHK(launch_apply_B_chkr_sel(st, dr, 2, n, N, cur, B_INV_RIGHT, B_RIGHT, sel, sl, g.ngroups));
+          LCHK(launch_apply_B_chkr_sel(st, dl, 2, n, N, cur, B_LEFT, B_INV_LEFT, sel, sl + 2, g.ngroups));
+        }
+      }
+      if (i != 0) {
+        LCHK(launch_scale_rows_copy(st, dr, 2, n, cur, cur, pv(b, TA_SD)));
+        LCHK(launch_scale_cols(st, dl, 2, n, cur, pv(b, TA_SD)));
+      }
+      RC(o.udt(cur, pv(b, TA_DD), pm(b, TA_Q), pm(b, TA_T)));
+      if (i != 0) RC(o.gemm(pm(b, TA_GC), pm(b, TA_GA), OP_N, pm(b, TA_GB), OP_N));
+    }
+    job_group_done(g, all);
+  }
+  for (int c = 0; c < lo.rounds; ++c) {
+    const int nj = std::min(lo.slots, 2 * R - c * lo.slots), b = c * kTdgfInvRoles;
+    ChainDesc* dd = js.d_desc + 4;
+    Group all = job_group(g, dd, nj);
+    Ops o(all);
+    LCHK(launch_split_scales(st, dd, nj, n, pv(b, TB_AD), NV(V_D1), NV(V_D2)));  // 1/Dap, Dam
+    LCHK(launch_split_scales(st, dd, nj, n, pv(b, TB_BD), NV(V_D3), NV(V_D4)));  // 1/Dbp, Dbm
+    RC(o.copy(NM(M_TMP), pm(b, TB_BT)));
+    LCHK(launch_identity(st, dd, nj, n, NM(M_QRT), NOVEC));
+    {
+      ProfScope ps(all, DQMC_K_INVERSE);
+      LCHK(launch_qr_blocked(st, dd, nj, n, NM(M_TMP), NV(V_D5), 0, all.wg_qr, g.qr_nb));
+      LCHK(launch_qr_solve(st, dd, nj, n, NM(M_TMP), NM(M_QRT), g.qr_nb));  // Tb^-1
+    }
+    RC(o.gemm(NM(M_TMP2), pm(b, TB_AT), OP_N, NM(M_QRT), OP_N, NV(V_D2), NV(V_D3)));
+    {
+      ProfScope ps(all, DQMC_K_GEMM);
+      LCHK(launch_gemm(st, dd, nj, n, NM(M_TMP2), pm(b, TB_AU), OP_C, pm(b, TB_BU), OP_N, NV(V_D1), NV(V_D4), 1.0));
+    }
+    LCHK(launch_adjoint(st, dd, nj, n, NM(M_TMP3), pm(b, TB_AU)));
+    LCHK(launch_scale_rows_copy(st, dd, nj, n, NM(M_TMP3), NM(M_TMP3), NV(V_D1)));
+    {
+      ProfScope ps(all, DQMC_K_INVERSE);
+      LCHK(launch_qr_blocked(st, dd, nj, n, NM(M_TMP2), NV(V_D5), 0, all.wg_qr, g.qr_nb));
+      LCHK(launch_qr_solve(st, dd, nj, n, NM(M_TMP2), NM(M_TMP3), g.qr_nb));
+    }
+    LCHK(launch_scale_rows_copy(st, dd, nj, n, NM(M_TMP3), NM(M_TMP3), NV(V_D3)));
+    RC(o.gemm(pm(b, TB_RES), NM(M_QRT), OP_N, NM(M_TMP3), OP_N));
+    RC(o.effective_greens(pm(b, TB_RES)));
+    LCHK(launch_negate(st, dd, nj, n, pm(b, TB_NEG)));
+    job_group_done(g, all);
+  }
+  // fill_tdgf! from the checkpoints, one slice of every interval per launch
+  ChainDesc* df = js.d_desc + 4 + lo.slots;
+  Group all = job_group(g, df, 2 * R);
+  Ops o(all);
+  const int* fs = js.d_int + lo.fill_sel;
+  for (int t = 0; t < sm - 1; ++t) {
+    const int* sl = js.d_int + lo.fill_slices + (size_t)t * R;
+    RC(o.copy(pm(2 * t, 0), pm(2 * t, 1)));
+    ProfScope ps(all, DQMC_K_APPLY_B);
+    LCHK(launch_apply_B_chkr_sel(st, df, R, n, N, pm(2 * t, 0), B_LEFT, B_INV_LEFT, fs, sl, g.ngroups));
+    LCHK(launch_apply_B_chkr_sel(st, df + R, R, n, N, pm(2 * t, 0), B_INV_RIGHT, B_RIGHT, fs, sl, g.ngroups));
+  }
+  job_group_done(g, all);
+  return 0;
+}
+
+}  // namespace
+extern "C" {
+
 int dqmc_tdgf_alloc(dqmc_ctx* ctx) {
   CTX_CHECK(ctx);
   dqmc_batch* b = ctx->b;
@@ -2219,7 +2509,11 @@ int dqmc_tdgf_alloc(dqmc_ctx* ctx) {
   cm.tdgf_vec = (double*)v;
   cm.d.xmat = cm.tdgf_mat;
   cm.d.xvec = cm.tdgf_vec;
-  return upload_desc(b, g);
+  RC(upload_desc(b, g));
+  if (!tdgf_parallel_ok(g)) return 0;
+  LCHK(launch_identity(g.stream, g.d_desc, 1, g.n, NM(M_IDENT), NOVEC));
+  LCHK(launch_ones_vec(g.stream, g.d_desc, 1, g.n, NV(V_ONES)));
+  return tdgf_jobs_create(g, cm);
 }
 
 int dqmc_tdgf_free(dqmc_ctx* ctx) {
@@ -2229,6 +2523,8 @@ int dqmc_tdgf_free(dqmc_ctx* ctx) {
   RC(batch_sync(b));
   if (cm.tdgf_mat) (void)hipFree(cm.tdgf_mat);
   if (cm.tdgf_vec) (void)hipFree(cm.tdgf_vec);
+  if (cm.tdgf_jobs.mem) (void)hipFree(cm.tdgf_jobs.mem);
+  cm.tdgf_jobs = JobSet{};
   cm.tdgf_mat = nullptr;
   cm.tdgf_vec = nullptr;
   cm.d.xmat = nullptr;
@@ -2239,8 +2535,14 @@ int dqmc_tdgf_free(dqmc_ctx* ctx) {
 int dqmc_measure_tdgfs(dqmc_ctx* ctx) {
   CTX_CHECK(ctx);
   if (!ctx->b->chains[0].tdgf_mat) return fail(DQMC_E_STATE, "dqmc_tdgf_alloc has not been called");
-  Ops o(ctx->b->groups[0]);
-  RC(o.measure_tdgfs());
+  Group& g = ctx->b->groups[0];
+  ChainMem& cm = ctx->b->chains[0];
+  if (tdgf_parallel_ok(g) && cm.tdgf_jobs.mem) {
+    RC(tdgf_parallel(g, cm));
+  } else {
+    Ops o(g);
+    RC(o.measure_tdgfs());
+  }
   return batch_sync(ctx->b);
 }
 
@@ -2362,78 +2664,6 @@ int dqmc_boson_action(dqmc_ctx* ctx, double* S) {
 // Afterwards scal[S_BOSON_ACTION] = S_B and scal[S_LOGDET] = log|det G|.
 }  // extern "C"
 namespace {
-
-// Takes arrays out of one block: with base == nullptr it only adds up what they need.
-struct Carve {
-  char* base;
-  size_t off = 0;
-  template <class T>
-  T* take(size_t count) {
-    off = (off + 255) & ~(size_t)255;
-    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
-    off += count * sizeof(T);
-    return p;
-  }
-};
-// the factorisation scratch, barrier words and scalars of one job
-void carve_scratch(Carve& cv, ChainDesc& d) {
-  const size_t n = d.n;
-  d.qr_vn = cv.take<double>(2 * n);
-  d.qr_cand = cv.take<cplx>((size_t)2 * kMaxWG * n);
-  d.qr_cand_norm = cv.take<double>(2 * kMaxWG);
-  d.qr_cand_pos = cv.take<int>(2 * kMaxWG);
-  d.qr_perm = cv.take<int>(n);
-  d.qr_lpos = cv.take<int>(n);
-  d.qr_tau = cv.take<cplx>(n);
-  d.qr_Tf = cv.take<cplx>(16 * (n + 16));
-  d.qr_flags = cv.take<unsigned int>(1 + (n + 7) / 8);
-  d.inv_piv = cv.take<int>(n);
-  d.inv_bcast = cv.take<cplx>(2 * n);
-  d.bar_count = cv.take<unsigned int>(2);
-  d.bar_gen = d.bar_count ? d.bar_count + 1 : nullptr;
-  d.scal = cv.take<double>(kNumScalar);
-}
-// descriptors and tables to the device, barrier words and scalars cleared
-hipError_t jobs_upload(JobSet& js, const ChainMem& cm, const std::vector<ChainDesc>& h, const std::vector<int>& ints) {
-  hipError_t e = hipMemcpy(js.d_desc, h.data(), h.size() * sizeof(ChainDesc), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(js.d_int, ints.data(), ints.size() * sizeof(int), hipMemcpyHostToDevice);
-  for (const auto& d : h) {
-    if (d.scal == cm.d.scal) continue;  // the chain itself
-    if (e == hipSuccess) e = hipMemset(d.bar_count, 0, 2 * sizeof(unsigned int));
-    if (e == hipSuccess) e = hipMemset(d.scal, 0, kNumScalar * sizeof(double));
-  }
-  if (e == hipSuccess) e = hipDeviceSynchronize();
-  return e;
-}
-// a group over `nj` jobs of g's chain on g's stream, the workgroups shared between them
-Group job_group(const Group& g, ChainDesc* d_desc, int nj) {
-  Group j;
-  j.n = g.n;
-  j.N = g.N;
-  j.L = g.L;
-  j.M = g.M;
-  j.s = g.s;
-  j.nelem = g.nelem;
-  j.chkr = g.chkr;
-  j.ngroups = g.ngroups;
-  j.all_checks = g.all_checks;
-  j.stream = g.stream;
-  j.d_desc = d_desc;
-  j.chains.assign(nj, 0);
-  j.greens_route = g.greens_route;
-  j.udt_route = g.udt_route;
-  j.qr_nb = g.qr_nb;
-  j.prof_mask = g.prof_mask;
-  const int per = std::max(1, 256 / nj);
-  j.wg_qr = std::max(1, std::min(g.wg_qr, per));
-  j.wg_inv = std::max((g.n + 511) / 512, std::min(g.wg_inv, per));
-  return j;
-}
-// its timing records go to the chain's group
-void job_group_done(Group& g, Group& j) {
-  g.prof.insert(g.prof.end(), j.prof.begin(), j.prof.end());
-  g.event_pool.insert(g.event_pool.end(), j.event_pool.begin(), j.event_pool.end());
-}
 
 // The gradient needs the Green's function of every slice of one field, with no update in between,
 // so its R = M / safe_mult intervals are independent once the stack's two halves exist: the left
@@ -2757,6 +2987,87 @@ int dqmc_set_hopping_matrix(dqmc_ctx* ctx, const double* T) {
   return 0;
 }
 
+}  // extern "C"
+namespace {
+
+// The Green's function of slice 1 from scratch as two chains side by side: B_M .. B_(l+1) into the
+// left operand and (B_l .. B_1)^H into the right one of calculate_greens, l half the slices,
+// instead of all of them into the right one: half as deep, and fewer factorisations behind each
+// operand. Descriptor 0 is the left chain, under the names of the right operand, 1 the chain
+// itself. L = 8, M = 100: dqmc_measure_greens 35 -> 17 ms.
+int meas_jobs_create(const Group& g, ChainMem& cm) {
+  JobSet& js = cm.meas_jobs;
+  const int R = g.M / g.s, sm = g.s, h1 = R / 2;
+  const size_t nn = (size_t)g.n * g.n;
+  std::vector<int> ints{0, 1};
+  for (int i = 0; i < R - h1; ++i)
+    for (int t = 0; t < sm; ++t) {
+      ints.push_back((h1 + i) * sm + t);
+      ints.push_back(std::max(0, (h1 - i) * sm - 1 - t));
+    }
+  std::vector<ChainDesc> h;
+  auto layout = [&](Carve& cv) {
+    h.assign(2, cm.d);
+    js.d_desc = cv.take<ChainDesc>(2);
+    js.d_int = cv.take<int>(ints.size());
+    ChainDesc& d = h[0];
+    carve_scratch(cv, d);
+    d.mat[M_UR] = cm.d.mat[M_UL];
+    d.mat[M_TR] = cm.d.mat[M_TL];
+    d.vec[V_DR] = cm.d.vec[V_DL];
+    for (int m : {M_CURU, M_QRT, M_TMP}) d.mat[m] = cv.take<cplx>(nn);
+  };
+  Carve size{nullptr};
+  layout(size);
+  if (hipMalloc(&js.mem, size.off) != hipSuccess) {
+    (void)hipGetLastError();
+    js = JobSet{};
+    js.failed = true;
+    return 0;
+  }
+  Carve cv{(char*)js.mem};
+  layout(cv);
+  const hipError_t e = jobs_upload(js, cm, h, ints);
+  if (e != hipSuccess) {
+    (void)hipFree(js.mem);
+    js = JobSet{};
+    return fail(DQMC_E_HIP, std::string("measurement jobs: ") + hipGetErrorString(e));
+  }
+  return 0;
+}
+
+int meas_chains(Group& g, ChainMem& cm) {
+  JobSet& js = cm.meas_jobs;
+  const int R = g.M / g.s, sm = g.s, n = g.n;
+  hipStream_t st = g.stream;
+  Group both = job_group(g, js.d_desc, 2), left = job_group(g, js.d_desc, 1);
+  LCHK(launch_identity(st, js.d_desc, 2, n, NM(M_UR), NOVEC));
+  LCHK(launch_identity(st, js.d_desc, 2, n, NM(M_TR), NOVEC));
+  LCHK(launch_ones_vec(st, js.d_desc, 2, n, NV(V_DR)));
+  for (int i = 0; i < R - R / 2; ++i) {
+    Group& h = i < R / 2 ? both : left;
+    Ops o(h);
+    const int nj = h.nch();
+    RC(o.copy(NM(M_CURU), NM(M_UR)));
+    {
+      ProfScope ps(h, DQMC_K_APPLY_B);
+      for (int t = 0; t < sm; ++t)
+        LCHK(launch_apply_B_chkr_sel(st, js.d_desc, nj, n, g.N, NM(M_CURU), B_LEFT, B_DAG_LEFT, js.d_int,
+                                     js.d_int + 2 + 2 * (size_t)(i * sm + t), g.ngroups));
+    }
+    LCHK(launch_scale_cols(st, js.d_desc, nj, n, NM(M_CURU), NV(V_DR)));
+    RC(o.udt(NM(M_CURU), NV(V_DR), NM(M_UR), NM(M_QRT)));
+    RC(o.gemm(NM(M_TMP), NM(M_QRT), OP_N, NM(M_TR), OP_N));
+    RC(o.copy(NM(M_TR), NM(M_TMP)));
+  }
+  job_group_done(g, both);
+  job_group_done(g, left);
+  return 0;
+}
+
+}  // namespace
+extern "C" {
+
 int dqmc_measure_greens(dqmc_ctx* ctx, double* G) {
   // measure_greens (fermion_measurements.jl:225-229): calc_greens(mc, 1) (from scratch, as
   // calc_greens_and_logdet :1061-1101), then effective_greens2greens! (:1125-1141)
@@ -2766,10 +3077,17 @@ int dqmc_measure_greens(dqmc_ctx* ctx, double* G) {
   ChainMem& cm = b->chains[0];
   RC(meas_alloc(cm));
   Ops o(g);
-  RC(o.bchain(1, g.M, B_DAG_LEFT, NM(M_UR), NV(V_DR), NM(M_TR)));
-  LCHK(launch_identity(g.stream, g.d_desc, 1, g.n, NM(M_UL), NOVEC));
-  LCHK(launch_identity(g.stream, g.d_desc, 1, g.n, NM(M_TL), NOVEC));
-  LCHK(launch_ones_vec(g.stream, g.d_desc, 1, g.n, NV(V_DL)));
+  // the batched slice operators need a checkerboard; the verbatim routes keep the one chain
+  const bool halves = g.greens_route == 0 && g.udt_route == 0 && g.chkr && g.M % g.s == 0 && g.M / g.s >= 2;
+  if (halves && !cm.meas_jobs.mem && !cm.meas_jobs.failed) RC(meas_jobs_create(g, cm));
+  if (halves && cm.meas_jobs.mem) {
+    RC(meas_chains(g, cm));
+  } else {
+    RC(o.bchain(1, g.M, B_DAG_LEFT, NM(M_UR), NV(V_DR), NM(M_TR)));
+    LCHK(launch_identity(g.stream, g.d_desc, 1, g.n, NM(M_UL), NOVEC));
+    LCHK(launch_identity(g.stream, g.d_desc, 1, g.n, NM(M_TL), NOVEC));
+    LCHK(launch_ones_vec(g.stream, g.d_desc, 1, g.n, NV(V_DL)));
+  }
   double* sc = cm.d.scal;
   HIPCHK(hipMemcpyAsync(sc + S_LOGDET_SAVE, sc + S_LOGDET, sizeof(double), hipMemcpyDeviceToDevice, g.stream));
   RC(o.copy(NM(M_GW), NM(M_G)));
