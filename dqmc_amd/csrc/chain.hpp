@@ -98,6 +98,7 @@ struct ChainDesc {
   cplx* lu_diag;          // [2][N][16] diagonal site blocks published between rounds
   cplx* ld_A;             // [16][n][4] pending left factors of the delayed local updates
   cplx* ld_B;             // [16][4][n] pending right factors
+  unsigned int* win_flags;  // [256] flag_sync words of the windowed updates; never above bar_gen between kernels
   int* ld_cmd;            // [2] command and pending count of a flush round
   // local updates
   const double* uniforms; // host-drawn uniform stream (device copy)

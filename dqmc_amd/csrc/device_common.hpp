@@ -104,6 +104,12 @@ __device__ inline void st_nt(gcplx* p, cplx v) {
   __builtin_nontemporal_store(v.im, &p->im);
 }
 
+// write-through store: it has reached memory once the wave's store counter is back at zero
+__device__ inline void st_wt(gcplx* p, cplx v) {
+  __hip_atomic_store(&p->re, v.re, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&p->im, v.im, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---------------------------------------------------------------------------
 // Reductions (wave64)
 //
@@ -311,6 +317,41 @@ __device__ inline void group_sync(const GroupSync& g) {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
+}
+
+// Barrier of a group whose workgroups publish by write-through stores (st_wt) and read what the
+// others published from cache lines that they have not touched since the kernel began: it needs
+// neither the write-back nor the invalidation of the XCD's L2, which every workgroup would issue
+// by itself and which take the longer the more workgroups share an XCD, and no shared counter:
+// workgroup w sets its word of `flags` to `target` once all its waves' stores have reached
+// memory, and thread t waits for word t. Targets grow from call to call (wrapping); false when a
+// wait ran out or the group has failed. W <= blockDim.x. 256 workgroups: 47,000 cycles per barrier
+// with group_sync, 27,000 without its fences, 18,000 with the
+// words (of which the wait for the slowest workgroup's columns is the larger part).
+__device__ inline bool flag_sync(unsigned int* flags, unsigned int target, int w, int W, int* error) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (W <= 1) {
+    __syncthreads();
+    return true;
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t == 0) __hip_atomic_store(flags + w, target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  bool ok = true;
+  if (t < W) {
+    long long spins = 0;
+    while ((int)(__hip_atomic_load(flags + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
+      if ((++spins & 31) == 0) {
+        if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+          ok = false;
+          break;
+        }
+        if (spins > kSpinLimit) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  return !__syncthreads_or(!ok);
 }
 
 }  // namespace dqmc

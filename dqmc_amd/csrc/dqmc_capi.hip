@@ -320,6 +320,8 @@ int chain_create(ChainMem& cm, const dqmc_params* p, const dqmc_operators* o) {
   ALLOC(d.ld_A, cplx, (size_t)16 * 4 * n);
   ALLOC(d.ld_B, cplx, (size_t)16 * 4 * n);
   ALLOC(d.ld_cmd, int, 2);
+  ALLOC(d.win_flags, unsigned int, kMaxLocalWG);
+  HIPCHK(hipMemset(d.win_flags, 0, kMaxLocalWG * sizeof(unsigned int)));
   ALLOC(d.ucursor, long long, 1);
   ALLOC(d.scal, double, kNumScalar);
   ALLOC(d.log_count, long long, 1);

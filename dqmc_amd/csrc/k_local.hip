@@ -1252,6 +1252,12 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
   cplx* Wb = Aw;                                                     // W, at the window's end (TILE)
   __shared__ WinShared sh;
   gcplx* X[2] = {gp(c.mat[M_G]), gp(c.mat[M_GALT])};
+  // TILE: the published columns of the sites behind the first window, at whole cache lines (128
+  // bytes): a line belongs to one column, so nobody has it cached before its window. They fit
+  // M_GALT, as 4 (N - w1) (n + 7) + 7 <= n^2 for w1 >= 2.
+  const int w1 = N / R, ps = (n + 7) & ~7;
+  const unsigned int epoch = TILE ? *c.bar_gen : 0;  // read before the first barrier, moved on after the last
+  gcplx* const pub = (gcplx*)(((uintptr_t)c.mat[M_GALT] + 127) & ~(uintptr_t)127);
   if (TILE) {
     const gcplx* G0 = X[0] + (size_t)cb0 * n;
     const int tot = ncol * n;
@@ -1288,7 +1294,11 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
 
   for (int rw = 0; rw < R; ++rw) {
     const int s0 = (int)((long long)rw * N / R), s1 = (int)((long long)(rw + 1) * N / R), kw = s1 - s0;
-    const gcplx* Gc = TILE ? X[rw > 0] : X[rw & 1];
+    const gcplx* Gc = X[TILE ? 0 : rw & 1];
+    // column of flavour a of a site of this window
+    auto column = [&](int site, int a) __attribute__((always_inline)) {
+      return TILE && rw > 0 ? pub + (unsigned)((4 * (site - w1) + a) * ps) : Gc + (unsigned)((site + a * N) * n);
+    };
     const int off0 = sh.off;
     // T = G(r_j, c_k) between the window's sites (consecutive lanes: consecutive rows), the
     // proposals while the first loads are under way
@@ -1296,7 +1306,7 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
       const int tot = kw * kw * 16, tid = opaque(threadIdx.x);
       auto src = [&](int e) {
         const int jj = e % kw, t = e / kw, a = t & 3, b = (t >> 2) & 3, kk = t >> 4;
-        return Gc + (size_t)(s0 + kk + b * N) * n + (s0 + jj + a * N);
+        return column(s0 + kk, b) + (s0 + jj + a * N);
       };
       auto dst = [&](int e) {
         const int jj = e % kw, t = e / kw, a = t & 3, b = (t >> 2) & 3, kk = t >> 4;
@@ -1545,7 +1555,6 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
       // n = 512, else two rows (W is then read from LDS half as often) and one ahead.
       const bool last = rw + 1 == R;
       const int e1 = last ? N : (int)((long long)(rw + 2) * N / R);
-      gcplx* Gn = last ? X[0] : X[1];
       auto finish = [&](auto rows, auto depth) __attribute__((always_inline)) {
         constexpr int NR = decltype(rows)::value, DP = decltype(depth)::value;
         const int r = opaque(tid);
@@ -1556,7 +1565,7 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
           const int site = __builtin_amdgcn_readfirstlane(sh.accs[min(b, m - 1)]);
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const gcplx* col = Gc + (size_t)(site + k * N) * n;
+            const gcplx* col = column(site, k);
 #pragma unroll
             for (int h = 0; h < NR; ++h) y[h][k] = ld(col + (unsigned)rr[h]);
           }
@@ -1634,13 +1643,15 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             if (j0 + q < ncol) {
-              const int col = cb0 + j0 + q, cs = col % N;
-              const bool pub = last || (cs >= s1 && cs < e1);
+              const int col = cb0 + j0 + q, a = col / N, cs = col - a * N;
+              const bool next = !last && cs >= s1 && cs < e1;
+              gcplx* out = last ? X[0] + (size_t)col * n : pub + (unsigned)((4 * (cs - w1) + a) * ps);
 #pragma unroll
               for (int h = 0; h < NR; ++h)
                 if (r + h * kWinThreads < n) {
                   s16(own + (j0 + q) * n + rr[h], acc[h][q]);
-                  if (pub) st_nt(Gn + (size_t)col * n + rr[h], acc[h][q]);
+                  if (last) st_nt(out + rr[h], acc[h][q]);
+                  if (next) st_wt(out + rr[h], acc[h][q]);
                 }
             }
         }
@@ -1690,8 +1701,15 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
       }
     }
     if (rw + 1 < R) {
-      group_sync(g);
-      if (group_failed(g)) return;
+      if (TILE) {
+        if (!flag_sync(c.win_flags, epoch + 1 + rw, w, W, c.error)) {
+          if (w == 0 && tid == 0) *c.bar_gen = epoch + R;
+          return;
+        }
+      } else {
+        group_sync(g);
+        if (group_failed(g)) return;
+      }
     }
   }
   // counters and the updated field slice, by workgroup 0 (the field is complete since the last S1)
@@ -1703,6 +1721,7 @@ __global__ __launch_bounds__(kWinThreads) void k_local_updates_window(const Chai
         minratio = fmin(minratio, read_lane(minratio, o));
       }
       if (lane == 0) {
+        if (TILE) *c.bar_gen = epoch + R;
         *c.ucursor = s.cur0 + coff;
         if (dolog) *c.log_count = logi;
         c.scal[S_BOSON_ACTION] += dS_acc;
