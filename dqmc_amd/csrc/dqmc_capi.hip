@@ -159,6 +159,7 @@ struct dqmc_batch {
   std::vector<ChainMem> chains;
   std::vector<Group> groups;
   std::vector<int> chain_group;  // chain -> group index
+  int* d_error = nullptr;        // [chains] error words (ChainDesc::error)
   double* d_scratch = nullptr;   // small host-visible staging (detratio etc.)
   bool use_graph = false;
   // merged sweeps of several shape groups (chains of any L and M, one launch per kernel)
@@ -329,9 +330,7 @@ int chain_create(ChainMem& cm, const dqmc_params* p, const dqmc_operators* o) {
   ALLOC(bar, unsigned int, 2);
   d.bar_count = bar;
   d.bar_gen = bar + 1;
-  ALLOC(d.error, int, 1);
   HIPCHK(hipMemset(bar, 0, 2 * sizeof(unsigned int)));
-  HIPCHK(hipMemset(d.error, 0, sizeof(int)));
   HIPCHK(hipMemset(d.ucursor, 0, sizeof(long long)));
   HIPCHK(hipMemset(d.log_count, 0, sizeof(long long)));
   HIPCHK(hipMemset(d.phi, 0, sizeof(double) * 3 * N * cm.M));
@@ -1002,10 +1001,12 @@ struct Ops {
   }
 };
 
+// The chains' error words are one array, so that this is one copy: every call that returns data
+// ends here, and with a copy per chain reading 64 chains' fields and G took 8192 of them (100 ms).
 int check_device_error(dqmc_batch* b) {
-  for (auto& cm : b->chains) {
-    int e = 0;
-    HIPCHK(hipMemcpy(&e, cm.d.error, sizeof(int), hipMemcpyDeviceToHost));
+  std::vector<int> err(b->chains.size());
+  HIPCHK(hipMemcpy(err.data(), b->d_error, err.size() * sizeof(int), hipMemcpyDeviceToHost));
+  for (int e : err) {
     if (e == 1) return fail(DQMC_E_DEVICE, "device: chain-group barrier timed out");
     if (e == 2) return fail(DQMC_E_DEVICE, "device: uniform stream exhausted (upload more with set_uniforms)");
   }
@@ -1036,6 +1037,15 @@ int batch_create(const dqmc_params* p, const dqmc_operators* ops, int nchains, i
       return rc;
     }
   }
+  hipError_t ee = hipMalloc(&b->d_error, nchains * sizeof(int));
+  if (ee == hipSuccess) ee = hipMemset(b->d_error, 0, nchains * sizeof(int));
+  if (ee != hipSuccess) {
+    for (auto& cm : b->chains) chain_free(cm);
+    if (b->d_error) (void)hipFree(b->d_error);
+    delete b;
+    return fail(DQMC_E_HIP, std::string("error words: ") + hipGetErrorString(ee));
+  }
+  for (int i = 0; i < nchains; ++i) b->chains[i].d.error = b->d_error + i;
   // shape groups: identical (L, M, safe_mult, checkerboard, all_checks)
   std::map<std::tuple<int, int, int, int, int>, int> idx;
   b->chain_group.resize(nchains);
@@ -1096,6 +1106,7 @@ int batch_destroy(dqmc_batch* b) {
   }
   for (auto& cm : b->chains) chain_free(cm);
   if (b->d_scratch) (void)hipFree(b->d_scratch);
+  if (b->d_error) (void)hipFree(b->d_error);
   b->drop_mgraphs();
   if (b->mstream) (void)hipStreamDestroy(b->mstream);
   if (b->d_mplan) (void)hipFree(b->d_mplan);
