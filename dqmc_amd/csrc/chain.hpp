@@ -84,8 +84,7 @@ struct ChainDesc {
   // factorization scratch
   double* qr_vn;          // [2n] partial column norms
   cplx* qr_cand;          // [2][W][n] candidate columns (double buffered)
-  double* qr_cand_norm;   // [2][W]
-  int* qr_cand_pos;       // [2][W]
+  unsigned long long* qr_meta;  // [2][W][3] tagged norm (two halves) and position of the candidates
   int* qr_perm;           // [n] logical -> physical column
   int* qr_lpos;           // [n] physical -> logical
   cplx* qr_tau;           // [n]

@@ -306,8 +306,8 @@ int chain_create(ChainMem& cm, const dqmc_params* p, const dqmc_operators* o) {
   ALLOC(d.phi, double, (size_t)3 * N * cm.M);
   ALLOC(d.qr_vn, double, 2 * n);
   ALLOC(d.qr_cand, cplx, (size_t)2 * kMaxWG * n);
-  ALLOC(d.qr_cand_norm, double, 2 * kMaxWG);
-  ALLOC(d.qr_cand_pos, int, 2 * kMaxWG);
+  ALLOC(d.qr_meta, unsigned long long, 6 * kMaxWG);
+  HIPCHK(hipMemset(d.qr_meta, 0, 6 * kMaxWG * sizeof(unsigned long long)));
   ALLOC(d.qr_perm, int, n);
   ALLOC(d.qr_lpos, int, n);
   ALLOC(d.qr_tau, cplx, n);
@@ -2229,8 +2229,7 @@ void carve_scratch(Carve& cv, ChainDesc& d) {
   const size_t n = d.n;
   d.qr_vn = cv.take<double>(2 * n);
   d.qr_cand = cv.take<cplx>((size_t)2 * kMaxWG * n);
-  d.qr_cand_norm = cv.take<double>(2 * kMaxWG);
-  d.qr_cand_pos = cv.take<int>(2 * kMaxWG);
+  d.qr_meta = cv.take<unsigned long long>(6 * kMaxWG);
   d.qr_perm = cv.take<int>(n);
   d.qr_lpos = cv.take<int>(n);
   d.qr_tau = cv.take<cplx>(n);
@@ -2249,6 +2248,7 @@ hipError_t jobs_upload(JobSet& js, const ChainMem& cm, const std::vector<ChainDe
   for (const auto& d : h) {
     if (d.scal == cm.d.scal) continue;  // the chain itself
     if (e == hipSuccess) e = hipMemset(d.bar_count, 0, 2 * sizeof(unsigned int));
+    if (e == hipSuccess) e = hipMemset(d.qr_meta, 0, 6 * kMaxWG * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemset(d.scal, 0, kNumScalar * sizeof(double));
   }
   if (e == hipSuccess) e = hipDeviceSynchronize();

@@ -11,7 +11,12 @@
 //   * at the end of each step every workgroup publishes its best remaining
 //     column (norm, logical position, values) to a double-buffered slot, so the
 //     next step's pivot choice and Householder vector are computed redundantly by
-//     every workgroup from the published copy: one group barrier per column;
+//     every workgroup from the published copy;
+//   * no barrier: the values go out by write-through stores, then three words with the
+//     step's tag, norm and position. Everyone waits for the W tags of the step itself, so a
+//     slot is rewritten (two steps on) only after all have read it. Tags continue from launch
+//     to launch (bar_gen). The own columns stay in LDS where they fit: with the barrier's
+//     fences they came back from memory every step;
 //   * pivot rule and partial-norm downdating follow LAPACK zlaqp2 (first maximum,
 //     tol3z = sqrt(eps) recomputation threshold).
 // Q is then formed column-independently (Q e_j = H_0 ... H_j e_j) with blocks of
@@ -38,6 +43,29 @@ __device__ inline double wave_norm2(const cplx* x, int r0, int n) {
   return wave_sum(acc);
 }
 
+__device__ inline unsigned long long ld_agent(const unsigned long long* p) {
+  return __hip_atomic_load((const __attribute__((address_space(1))) unsigned long long*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double ld_agent(const double* p) {
+  return __hip_atomic_load((const __attribute__((address_space(1))) double*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_agent(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store((__attribute__((address_space(1))) unsigned long long*)p, v, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__host__ __device__ inline size_t qrp_lds_bytes(int n, int W, bool res) {
+  const size_t nc = (n + W - 1) / W;
+  return nc * 16 + (res ? nc * n * sizeof(cplx) : 0);
+}
+
+// Bound by the chain of a column step: the candidates' words and the winner's column out of
+// memory, the norm, the update of the own columns, the next candidate into memory. RES: own columns
+// in LDS. n = 256, 32 workgroups on each of 4 chains: 3.3 -> 1.65 ms per factorisation, 6.4 us a
+// column.
+template <bool RES>
 __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar, VecRef Dr) {
   const ChainDesc& c = chains[blockIdx.y];
   const int n = c.n;
@@ -45,41 +73,46 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
   cplx* A = matptr(c, Ar);
   double* D = vecptr(c, Dr);
-  GroupSync g = chain_group(c);
-  // partial column norms of the own columns, indexed by physical column (LDS)
-  __shared__ double vn1[kMaxN], vn2[kMaxN];
   const double tol3z = sqrt(0.5 * 2.220446049250313e-16);
+  const unsigned int epoch = *c.bar_gen;  // no workgroup moves it before all have published
 
+  extern __shared__ __attribute__((aligned(16))) double qrp_smem[];
+  const int ncm = (n + W - 1) / W, ncol = w < n ? (n - w + W - 1) / W : 0;  // own columns w, w + W, ..
+  double *vn1 = qrp_smem, *vn2 = vn1 + ncm;  // partial column norms of the own columns
+  cplx* own = reinterpret_cast<cplx*>(vn2 + ncm);  // [ncm][n] (RES)
   __shared__ int perm[kMaxN], lpos[kMaxN];
   __shared__ cplx v[kMaxN];
   __shared__ double red[8];
-  __shared__ int s_pos, s_win;
+  __shared__ int s_win, s_fail;
   __shared__ double s_best[4];
   __shared__ int s_bestc[4], s_bestl[4];
+  auto column = [&](int cl) { return RES ? own + (size_t)cl * n : A + (size_t)(w + cl * W) * n; };
 
   for (int i = tid; i < n; i += blockDim.x) perm[i] = lpos[i] = i;
-  // initial column norms of own columns
-  for (int col = w + W * wave; col < n; col += W * nwaves) {
-    const double nr = sqrt(wave_norm2(A + (size_t)col * n, 0, n));
-    if (lane == 0) {
-      vn1[col] = nr;
-      vn2[col] = nr;
-    }
-  }
+  if (RES)
+    for (int cl = 0; cl < ncol; ++cl)
+      for (int k = tid; k < n; k += blockDim.x) own[(size_t)cl * n + k] = A[(size_t)(w + cl * W) * n + k];
+  if (tid == 0) s_fail = 0;
   __syncthreads();
+  // initial column norms of own columns
+  for (int cl = wave; cl < ncol; cl += nwaves) {
+    const double nr = sqrt(wave_norm2(column(cl), 0, n));
+    if (lane == 0) vn1[cl] = vn2[cl] = nr;
+  }
 
-  // publish best own column among logical positions >= first
-  auto publish = [&](int first, int buf) {
+  // publish best own column among logical positions >= first, for step `first`
+  auto publish = [&](int first) {
+    const int buf = first & 1;
     double best = -1.0;
     int bestc = -1, bestl = n;
     if (lane == 0) {
-      for (int col = w + W * wave; col < n; col += W * nwaves) {
-        const int lp = lpos[col];
+      for (int cl = wave; cl < ncol; cl += nwaves) {
+        const int lp = lpos[w + cl * W];
         if (lp < first) continue;
-        const double nv = vn1[col];
+        const double nv = vn1[cl];
         if (nv > best || (nv == best && lp < bestl)) {
           best = nv;
-          bestc = col;
+          bestc = cl;
           bestl = lp;
         }
       }
@@ -88,40 +121,57 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
       s_bestl[wave] = bestl;
     }
     __syncthreads();
-    if (tid == 0) {
-      int bw = 0;
-      for (int q = 1; q < nwaves; ++q) {
-        if (s_best[q] > s_best[bw] || (s_best[q] == s_best[bw] && s_bestl[q] < s_bestl[bw])) bw = q;
-      }
-      c.qr_cand_norm[buf * W + w] = s_bestc[bw] >= 0 ? s_best[bw] : -1.0;
-      c.qr_cand_pos[buf * W + w] = s_bestc[bw] >= 0 ? s_bestl[bw] : -1;
-      s_win = s_bestc[bw];
-    }
-    __syncthreads();
-    const int bc = s_win;
+    int bw = 0;
+    for (int q = 1; q < nwaves; ++q)
+      if (s_best[q] > s_best[bw] || (s_best[q] == s_best[bw] && s_bestl[q] < s_bestl[bw])) bw = q;
+    const int bc = s_bestc[bw];
     if (bc >= 0) {
-      cplx* dst = c.qr_cand + ((size_t)buf * W + w) * n;
-      const cplx* src = A + (size_t)bc * n;
-      for (int k = first + tid; k < n; k += blockDim.x) dst[k] = src[k];
+      gcplx* dst = gp(c.qr_cand) + ((size_t)buf * W + w) * n;
+      const cplx* src = column(bc);
+      for (int k = first + tid; k < n; k += blockDim.x) st_wt(dst + k, src[k]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid < 3) {
+      const unsigned long long tag = epoch + 1u + (unsigned)first;
+      const unsigned long long nb = (unsigned long long)__double_as_longlong(bc >= 0 ? s_best[bw] : -1.0);
+      const unsigned long long hi = tid == 0 ? nb >> 32 : tid == 1 ? nb & 0xffffffffu : (unsigned)(bc >= 0 ? s_bestl[bw] : -1);
+      st_agent(c.qr_meta + ((size_t)buf * W + w) * 3 + tid, hi << 32 | (tag & 0xffffffffu));
     }
   };
-
-  publish(0, 0);
-  group_sync(g);
+  __syncthreads();
+  publish(0);
 
   for (int i = 0; i < n; ++i) {
-    if (group_failed(g)) return;
     const int buf = i & 1;
-    // ---- pivot: first maximum of the partial norms over logical positions >= i.
-    // Every candidate slot is read by its own thread (one memory round trip), then
-    // reduced in wave 0 by (norm descending, logical position ascending).
+    // ---- pivot: first maximum of the partial norms over logical positions >= i. Every
+    // candidate's words are awaited by a lane of wave 0, then reduced by (norm descending,
+    // logical position ascending).
     if (wave == 0) {
       double bn = -1.0;
       int bp = n, bw = -1;
+      const unsigned int tag = epoch + 1u + (unsigned)i;
+      bool fail = false;
       for (int q = lane; q < W; q += 64) {
-        const int pq = c.qr_cand_pos[buf * W + q];
-        const double nq = c.qr_cand_norm[buf * W + q];
-        if (pq >= 0 && (bw < 0 || nq > bn || (nq == bn && pq < bp))) {
+        const unsigned long long* m = c.qr_meta + ((size_t)buf * W + q) * 3;
+        unsigned long long m0, m1, m2;
+        long long spins = 0;
+        for (;;) {
+          m0 = ld_agent(m);
+          m1 = ld_agent(m + 1);
+          m2 = ld_agent(m + 2);
+          if ((unsigned)m0 == tag && (unsigned)m1 == tag && (unsigned)m2 == tag) break;
+          if ((++spins & 31) == 0) {
+            if (__hip_atomic_load(c.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+              fail = true;
+              break;
+            }
+            if (spins > kSpinLimit) __hip_atomic_store(c.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        const double nq = __longlong_as_double((long long)((m0 >> 32) << 32 | m1 >> 32));
+        const int pq = (int)(m2 >> 32);
+        if (!fail && pq >= 0 && (bw < 0 || nq > bn || (nq == bn && pq < bp))) {
           bn = nq;
           bp = pq;
           bw = q;
@@ -138,32 +188,36 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
           bw = ow;
         }
       }
+      const bool failed = __ballot(fail) != 0 || bw < 0;
       if (lane == 0) {
         s_win = bw;
-        s_pos = bp;
+        if (failed) {
+          s_fail = 1;
+        } else {
+          const int pc = perm[bp], pi = perm[i];
+          perm[i] = pc;
+          perm[bp] = pi;
+          lpos[pc] = i;
+          lpos[pi] = bp;
+        }
       }
     }
     __syncthreads();
-    if (tid == 0) {
-      const int bp = s_pos;
-      const int pc = perm[bp], pi = perm[i];
-      perm[i] = pc;
-      perm[bp] = pi;
-      lpos[pc] = i;
-      lpos[pi] = bp;
+    if (s_fail) {
+      if (w == 0 && tid == 0) *c.bar_gen = epoch + n + 1;
+      return;
     }
-    __syncthreads();
     const int pc = perm[i];
     const cplx* x = c.qr_cand + ((size_t)buf * W + s_win) * n;
     // ---- Householder reflector (zlarfg) from rows i..n-1 of the pivot column
     double part = 0.0;
     for (int k = i + 1 + tid; k < n; k += blockDim.x) {
-      const cplx xv = x[k];
+      const cplx xv = mk(ld_agent(&x[k].re), ld_agent(&x[k].im));
       v[k] = xv;
       part += abs2(xv);
     }
+    const cplx alpha = mk(ld_agent(&x[i].re), ld_agent(&x[i].im));
     const double xnorm = sqrt(block_sum(part, red));
-    const cplx alpha = x[i];
     cplx tau;
     double beta;
     if (xnorm == 0.0 && alpha.im == 0.0) {
@@ -182,14 +236,14 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
       c.qr_tau[i] = tau;
     }
     if (pc % W == w) {
-      cplx* colp = A + (size_t)pc * n;
+      cplx* colp = column(pc / W);
       for (int k = i + tid; k < n; k += blockDim.x) colp[k] = (k == i) ? mk(beta, 0) : v[k];
     }
     // ---- apply H^H = I - conj(tau) v v^H to own trailing columns, downdate norms
     const cplx ctau = conj(tau);
-    for (int col = w + W * wave; col < n; col += W * nwaves) {
-      if (lpos[col] <= i) continue;
-      cplx* colp = A + (size_t)col * n;
+    for (int cl = wave; cl < ncol; cl += nwaves) {
+      if (lpos[w + cl * W] <= i) continue;
+      cplx* colp = column(cl);
       const cplx d = wave_dotc(v, colp, i, n);
       const cplx f = ctau * d;
       // update rows i..n-1; keep the new row-i entry (lane 0) and the tail norm in registers
@@ -205,31 +259,34 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
       }
       const double aic = sqrt(abs2(mk(__shfl(first.re, 0, 64), __shfl(first.im, 0, 64))));
       const double tailnorm = sqrt(wave_sum(tail));
-      const double v1 = vn1[col];
+      const double v1 = vn1[cl];
       if (v1 != 0.0 && lane == 0) {
         double temp = 1.0 - (aic / v1) * (aic / v1);
         temp = fmax(temp, 0.0);
-        const double ratio = v1 / vn2[col];
+        const double ratio = v1 / vn2[cl];
         const double temp2 = temp * ratio * ratio;
         if (temp2 <= tol3z) {
           // partial norm lost its accuracy: recompute from the trailing rows (zlaqp2)
           const double nr = (i < n - 1) ? tailnorm : 0.0;
-          vn1[col] = nr;
-          vn2[col] = nr;
+          vn1[cl] = nr;
+          vn2[cl] = nr;
         } else {
-          vn1[col] = v1 * sqrt(temp);
+          vn1[cl] = v1 * sqrt(temp);
         }
       }
     }
     __syncthreads();
-    if (i + 1 < n) publish(i + 1, buf ^ 1);
-    group_sync(g);
+    if (i + 1 < n) publish(i + 1);
   }
+  if (RES)
+    for (int cl = 0; cl < ncol; ++cl)
+      for (int k = tid; k < n; k += blockDim.x) A[(size_t)(w + cl * W) * n + k] = own[(size_t)cl * n + k];
   if (w == 0) {
     for (int k = tid; k < n; k += blockDim.x) {
       c.qr_perm[k] = perm[k];
       c.qr_lpos[k] = lpos[k];
     }
+    if (tid == 0) *c.bar_gen = epoch + n + 1;
   }
 }
 
@@ -311,7 +368,13 @@ static hipError_t coop_launch(const void* fn, dim3 grid, void** args, hipStream_
 hipError_t launch_qrp(hipStream_t s, const ChainDesc* chains, int nchains, int nmax, MatRef A, VecRef D, int wg) {
   if (nmax > kMaxN) return hipErrorInvalidValue;
   void* args[] = {(void*)&chains, (void*)&A, (void*)&D};
-  hipError_t e = coop_launch((const void*)k_qrp, dim3(wg, nchains), args, s);
+  // the own columns stay in LDS where they fit beside the static part (v, perm, lpos: 25 KB)
+  const bool res = qrp_lds_bytes(nmax, wg, true) <= 130 * 1024;
+  const void* fn = res ? (const void*)k_qrp<true> : (const void*)k_qrp<false>;
+  const size_t lds = qrp_lds_bytes(nmax, wg, res);
+  hipError_t e = ensure_dynamic_lds(fn, lds);
+  if (e != hipSuccess) return e;
+  e = hipLaunchCooperativeKernel(fn, dim3(wg, nchains), dim3(256), args, lds, s);
   if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
