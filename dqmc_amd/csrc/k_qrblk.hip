@@ -1053,29 +1053,21 @@ __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, Mat
   }
 }
 
-// Column layout of k_qr_solve / k_form_Q_blocked: a workgroup owns CB columns in LDS. With
-// CB <= 4 the four waves split as CB columns x (4 / CB) row slices; with CB > 4 each wave owns
-// CB / 4 columns and all rows, so every V entry read from LDS serves CB / 4 columns.
-template <int CB>
-struct ColLayout {
-  static constexpr int RS = CB >= 4 ? 1 : 4 / CB;   // row slices per column
-  static constexpr int CPW = CB >= 4 ? CB / 4 : 1;  // columns per wave
-};
-
+// k_qr_solve / k_form_Q_blocked: a workgroup owns CB columns in LDS, CB / 4 per wave, so every V
+// entry read from LDS serves CB / 4 columns.
+//
 // x <- (I - V op(T) V^H) x for this wave's CPW columns xc + (jl0 + c) n (rows >= k0); V [NB][n]
 // and T (Tl[j * NB + l] = T(j, l)) in LDS; op = T^H (ADJ, applying Q^H) or T (applying Q).
-// part: LDS for the row-slice sums when RS > 1.
 template <int NB, int CB, bool ADJ>
-__device__ inline void apply_panel_cols(cplx* xc, const cplx* V, const cplx* Tl, cplx* part, int n, int k0, int jl0,
-                                        int rs, int ncol, int lane, int wave) {
-  using Lay = ColLayout<CB>;
-  constexpr int RS = Lay::RS, CPW = Lay::CPW;
+__device__ inline void apply_panel_cols(cplx* xc, const cplx* V, const cplx* Tl, int n, int k0, int jl0, int ncol,
+                                        int lane) {
+  constexpr int CPW = CB / 4;
   cplx wv[CPW][NB];
 #pragma unroll
   for (int c = 0; c < CPW; ++c)
 #pragma unroll
     for (int j = 0; j < NB; ++j) wv[c][j] = mk(0, 0);
-  for (int k = k0 + lane + 64 * rs; k < n; k += 64 * RS) {
+  for (int k = k0 + lane; k < n; k += 64) {
     cplx pj[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) pj[j] = V[(size_t)j * n + k];
@@ -1088,20 +1080,6 @@ __device__ inline void apply_panel_cols(cplx* xc, const cplx* V, const cplx* Tl,
   }
 #pragma unroll
   for (int c = 0; c < CPW; ++c) wave_sum_many<NB>(wv[c]);
-  if (RS > 1) {
-    if (lane == 0) {
-#pragma unroll
-      for (int j = 0; j < NB; ++j) part[wave * NB + j] = wv[0][j];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      cplx sj = mk(0, 0);
-#pragma unroll
-      for (int q = 0; q < RS; ++q) sj += part[(jl0 + CB * q) * NB + j];
-      wv[0][j] = sj;
-    }
-  }
   // z = op(T) w: lane j < NB forms z_j of every column, then every lane reads them
   const int jz = lane & (NB - 1);
   cplx z[CPW][NB];
@@ -1119,7 +1097,7 @@ __device__ inline void apply_panel_cols(cplx* xc, const cplx* V, const cplx* Tl,
     for (int j = 0; j < NB; ++j) z[c][j] = read_lane_c(zl, j);
   }
   if (jl0 < ncol) {  // wave-uniform; columns past ncol of the group are scratch
-    for (int k = k0 + lane + 64 * rs; k < n; k += 64 * RS) {
+    for (int k = k0 + lane; k < n; k += 64) {
       cplx pj[NB];
 #pragma unroll
       for (int j = 0; j < NB; ++j) pj[j] = V[(size_t)j * n + k];
@@ -1137,12 +1115,10 @@ __device__ inline void apply_panel_cols(cplx* xc, const cplx* V, const cplx* Tl,
 // B <- R^-1 Q^H B for a matrix factored by k_qr_blocked without pre-pivoting (Ar holds R and
 // the reflectors, qr_tau / qr_Tf the rest). Every right-hand side is independent: each
 // workgroup owns CB columns of B in LDS, applies the panels' Q_p^H in order, then
-// back-substitutes with R; no synchronisation between workgroups. The four waves split
-// as CB columns x (4 / CB) row slices; with more than one slice per column, the panel's
-// inner products are summed over the slices through LDS.
+// back-substitutes with R; no synchronisation between workgroups. (16-column panels; 8-column
+// ones take k_qr_solve_rows.)
 template <int NB, int CB>
 __global__ __launch_bounds__(256) void k_qr_solve(const ChainDesc* chains, MatRef Ar, MatRef Br) {
-  using Lay = ColLayout<CB>;
   int bx, by;
   xcd_block(bx, by);
   const ChainDesc& c = chains[by];
@@ -1151,7 +1127,7 @@ __global__ __launch_bounds__(256) void k_qr_solve(const ChainDesc* chains, MatRe
   if (j0 >= n) return;
   const int ncol = min(CB, n - j0);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int jl0 = CB >= 4 ? wave * Lay::CPW : wave % CB, rs = CB >= 4 ? 0 : wave / CB;
+  const int jl0 = wave * (CB / 4);
   const gcplx* A = gp(matptr(c, Ar));
   gcplx* B = gp(matptr(c, Br));
   extern __shared__ double smem[];
@@ -1159,7 +1135,6 @@ __global__ __launch_bounds__(256) void k_qr_solve(const ChainDesc* chains, MatRe
   cplx* V = bc + (size_t)CB * n;              // [NB][n]
   __shared__ cplx Tl[NB * NB];
   __shared__ cplx Rd[16 * 16];
-  __shared__ cplx part[Lay::RS > 1 ? 4 * NB : 1];
   for (int r = tid; r < n; r += 256) {
     cplx v[CB];
 #pragma unroll
@@ -1176,7 +1151,7 @@ __global__ __launch_bounds__(256) void k_qr_solve(const ChainDesc* chains, MatRe
     stage_panel<NB>(V, A, nullptr, k0, kb, n, tid, 1);  // columns >= kb zero-filled
     for (int e = tid; e < NB * NB; e += blockDim.x) Tl[e] = ld(gp(c.qr_Tf) + (size_t)p * NB * NB + e);
     __syncthreads();
-    apply_panel_cols<NB, CB, true>(bc, V, Tl, part, n, k0, jl0, rs, ncol, lane, wave);
+    apply_panel_cols<NB, CB, true>(bc, V, Tl, n, k0, jl0, ncol, lane);
   }
   // back substitution R y = z in blocks of 16 rows from the bottom: wave q < CB solves the
   // 16 x 16 diagonal block for column q (lane r holds row lo + r), then every thread takes
@@ -1241,7 +1216,6 @@ __global__ __launch_bounds__(256) void k_qr_solve(const ChainDesc* chains, MatRe
 // in k_qr_solve. Reflector k lives in physical column qr_perm[k] below its diagonal.
 template <int NB, int CB>
 __global__ __launch_bounds__(256) void k_form_Q_blocked(const ChainDesc* chains, MatRef Ar, MatRef Qr) {
-  using Lay = ColLayout<CB>;
   int bx, by;
   xcd_block(bx, by);
   const ChainDesc& c = chains[by];
@@ -1250,14 +1224,13 @@ __global__ __launch_bounds__(256) void k_form_Q_blocked(const ChainDesc* chains,
   if (j0 >= n) return;
   const int ncol = min(CB, n - j0);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int jl0 = CB >= 4 ? wave * Lay::CPW : wave % CB, rs = CB >= 4 ? 0 : wave / CB;
+  const int jl0 = wave * (CB / 4);
   const gcplx* A = gp(matptr(c, Ar));
   gcplx* Q = gp(matptr(c, Qr));
   extern __shared__ double smem[];
   cplx* xc = reinterpret_cast<cplx*>(smem);  // [CB][n]
   cplx* V = xc + (size_t)CB * n;              // [NB][n]
   __shared__ cplx Tl[NB * NB];
-  __shared__ cplx part[Lay::RS > 1 ? 4 * NB : 1];
   for (int r = tid; r < n; r += 256)
 #pragma unroll
     for (int q = 0; q < CB; ++q) {
@@ -1271,7 +1244,7 @@ __global__ __launch_bounds__(256) void k_form_Q_blocked(const ChainDesc* chains,
     stage_panel<NB>(V, A, c.qr_perm, k0, kb, n, tid, 1);  // columns >= kb zero-filled
     for (int e = tid; e < NB * NB; e += blockDim.x) Tl[e] = ld(gp(c.qr_Tf) + (size_t)p * NB * NB + e);
     __syncthreads();
-    apply_panel_cols<NB, CB, false>(xc, V, Tl, part, n, k0, jl0, rs, ncol, lane, wave);
+    apply_panel_cols<NB, CB, false>(xc, V, Tl, n, k0, jl0, ncol, lane);
   }
   __syncthreads();
   for (int r = tid; r < n; r += 256) {
@@ -1286,6 +1259,230 @@ __global__ __launch_bounds__(256) void k_form_Q_blocked(const ChainDesc* chains,
         d->im = v[q].im;
       }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Solve and Q formation with the columns in registers (few chains per launch).
+//
+// A workgroup owns four columns, thread t their rows t + 256 q (RQ = rows per thread). A panel's
+// reflectors go from memory straight into the registers of the threads that own their rows and
+// serve both products there, so each entry is read once per workgroup and never passes LDS:
+// W = V^H X is 32 sums per wave by one butterfly, the four waves' sums meet in LDS (one barrier
+// per panel, two buffers), every wave forms Z = op(T) W by itself (lane = column, reflector and
+// half of the sum). The kernels before it staged V in LDS (one column per workgroup at n > 640,
+// where V alone takes 131 KB). Bound by the chain of a panel: V's latency, the butterfly, the
+// barrier. n = 1024: solve 4.07 -> 1.11 ms, Q 2.49 -> 0.70 ms; n = 400: 0.419 -> 0.293 and 0.189 ->
+// 0.189 ms; n = 256: 0.220 -> 0.160 and 0.098 -> 0.098 ms; n = 576, Q of two chains: 0.57 -> 0.52 ms.
+// ---------------------------------------------------------------------------
+constexpr int kRowCols = 4;
+
+struct RowsShared {
+  double part[2][4][64];  // per wave: the 32 complex sums
+  cplx z[4][32];          // per wave: Z
+};
+
+template <int RQ, bool ADJ>
+__device__ inline void apply_panel_rows(cplx (&x)[RQ][kRowCols], const gcplx* A, const gcplx* Tf, const int* perm,
+                                        int p, int n, RowsShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int k0 = 8 * p;
+  cplx v[RQ][8];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q) {
+    const int r = tid + 256 * q, rr = min(r, n - 1);
+    if (256 * q + 255 >= k0) {  // (uniform) some rows at or below the diagonal
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = min(k0 + j, n - 1);
+        v[q][j] = ld(A + (size_t)(perm ? perm[k] : k) * n + rr);
+      }
+    }
+  }
+  // this lane's half of a row of op(T)
+  const int zc = (lane >> 3) & 3, zj = lane & 7, zh = lane >> 5;
+  cplx t[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) t[u] = ld(Tf + 64 * p + (ADJ ? (4 * zh + u) * 8 + zj : zj * 8 + 4 * zh + u));
+  double w[64];
+#pragma unroll
+  for (int e = 0; e < 64; ++e) w[e] = 0.0;
+#pragma unroll
+  for (int q = 0; q < RQ; ++q) {
+    const int r = tid + 256 * q;
+    if (256 * q + 255 >= k0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = k0 + j;
+        const bool below = r > k && r < n && k < n;
+        v[q][j].re = below ? v[q][j].re : (r == k && k < n) ? 1.0 : 0.0;
+        v[q][j].im = below ? v[q][j].im : 0.0;
+#pragma unroll
+        for (int c = 0; c < kRowCols; ++c) {
+          cplx s = mk(w[2 * (8 * c + j)], w[2 * (8 * c + j) + 1]);
+          cfma_cj(s, v[q][j], x[q][c]);
+          w[2 * (8 * c + j)] = s.re;
+          w[2 * (8 * c + j) + 1] = s.im;
+        }
+      }
+    }
+  }
+  wave_reduce_scatter<64>(w);
+  const int buf = p & 1;
+  sh.part[buf][wave][lane] = w[0];
+  __syncthreads();
+  cplx z = mk(0, 0);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = 2 * (8 * zc + 4 * zh + u);
+    cplx s = mk(0, 0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) s += mk(sh.part[buf][g][e], sh.part[buf][g][e + 1]);
+    if (ADJ)
+      cfma_cj(z, t[u], s);
+    else
+      cfma(z, t[u], s);
+  }
+  z.re += __shfl_xor(z.re, 32, 64);
+  z.im += __shfl_xor(z.im, 32, 64);
+  if (lane < 32) {
+    sh.z[wave][lane].re = z.re;
+    sh.z[wave][lane].im = z.im;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+  for (int c = 0; c < kRowCols; ++c) {
+    cplx zz[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) zz[j] = sh.z[wave][8 * c + j];
+#pragma unroll
+    for (int q = 0; q < RQ; ++q)
+      if (256 * q + 255 >= k0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) cfma(x[q][c], -v[q][j], zz[j]);
+      }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // Z read before the next panel's
+}
+
+template <int RQ>
+__global__ __launch_bounds__(256) void k_form_Q_rows(const ChainDesc* chains, MatRef Ar, MatRef Qr) {
+  int bx, by;
+  xcd_block(bx, by);
+  const ChainDesc& c = chains[by];
+  const int n = c.n, j0 = bx * kRowCols, tid = threadIdx.x;
+  if (j0 >= n) return;
+  const int ncol = min(kRowCols, n - j0);
+  const gcplx* A = gp(matptr(c, Ar));
+  gcplx* Q = gp(matptr(c, Qr));
+  __shared__ RowsShared sh;
+  __shared__ int perm[kQrMaxN];
+  for (int k = tid; k < n; k += 256) perm[k] = c.qr_perm[k];
+  __syncthreads();
+  cplx x[RQ][kRowCols];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int u = 0; u < kRowCols; ++u) x[q][u] = mk(tid + 256 * q == j0 + u ? 1.0 : 0.0, 0.0);
+  for (int p = (j0 + ncol - 1) / 8; p >= 0; --p)  // panels that start beyond the columns leave them alone
+    apply_panel_rows<RQ, false>(x, A, gp(c.qr_Tf), perm, p, n, sh);
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int u = 0; u < kRowCols; ++u)
+      if (tid + 256 * q < n && u < ncol) st(Q + (size_t)(j0 + u) * n + tid + 256 * q, x[q][u]);
+}
+
+template <int RQ>
+__global__ __launch_bounds__(256) void k_qr_solve_rows(const ChainDesc* chains, MatRef Ar, MatRef Br) {
+  int bx, by;
+  xcd_block(bx, by);
+  const ChainDesc& c = chains[by];
+  const int n = c.n, j0 = bx * kRowCols, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (j0 >= n) return;
+  const int ncol = min(kRowCols, n - j0);
+  const gcplx* A = gp(matptr(c, Ar));
+  gcplx* B = gp(matptr(c, Br));
+  __shared__ RowsShared sh;
+  __shared__ cplx Rd[16 * 17], Y[kRowCols][16], S[kRowCols][16];
+  cplx x[RQ][kRowCols];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int u = 0; u < kRowCols; ++u)
+      x[q][u] = ld(B + (size_t)(j0 + min(u, ncol - 1)) * n + min(tid + 256 * q, n - 1));
+  for (int p = 0; 8 * p < n; ++p) apply_panel_rows<RQ, true>(x, A, gp(c.qr_Tf), nullptr, p, n, sh);
+  // back substitution in aligned blocks of 16 rows from the bottom: wave u solves the 16 x 16
+  // diagonal block for column u (lane = row), then every thread takes its rows above
+  for (int hi = n; hi > 0; hi = (hi - 1) & ~15) {
+    const int lo = (hi - 1) & ~15, bs = hi - lo, qb = lo >> 8;
+    {
+      const int kk = tid >> 4, rr = tid & 15;
+      const cplx v = ld(A + (size_t)min(lo + kk, n - 1) * n + min(lo + rr, n - 1));
+      Rd[kk * 17 + rr].re = v.re;  // R(lo + rr, lo + kk)
+      Rd[kk * 17 + rr].im = v.im;
+    }
+    if (((tid ^ lo) & 0xF0) == 0) {  // the sixteen threads whose rows are the block's
+#pragma unroll
+      for (int q = 0; q < RQ; ++q)
+        if (q == qb) {
+#pragma unroll
+          for (int u = 0; u < kRowCols; ++u) {
+            Y[u][tid & 15].re = x[q][u].re;
+            Y[u][tid & 15].im = x[q][u].im;
+          }
+        }
+    }
+    __syncthreads();
+    {
+      const int r = lane & 15;
+      cplx zr = Y[wave][r];
+      const cplx dv = cinv(Rd[min(r, bs - 1) * 18]);
+      for (int k = bs - 1; k >= 0; --k) {
+        const cplx yk = read_lane_c(zr, k) * read_lane_c(dv, k);
+        const cplx rk = Rd[k * 17 + r];
+        if (r < k) zr = zr - rk * yk;
+        if (r == k) zr = yk;
+      }
+      if (lane < 16) {
+        S[wave][r].re = r < bs ? zr.re : 0.0;
+        S[wave][r].im = r < bs ? zr.im : 0.0;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const int r = tid + 256 * q;
+      if (256 * q < lo) {
+        cplx rv[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) rv[k] = ld(A + (size_t)min(lo + k, n - 1) * n + min(r, n - 1));
+        if (r < lo) {
+#pragma unroll
+          for (int u = 0; u < kRowCols; ++u)
+#pragma unroll
+            for (int k = 0; k < 16; ++k) cfma(x[q][u], -rv[k], S[u][k]);
+        }
+      }
+      if (q == qb && r >= lo && r < hi) {
+#pragma unroll
+        for (int u = 0; u < kRowCols; ++u) x[q][u] = mk(S[u][tid & 15].re, S[u][tid & 15].im);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int u = 0; u < kRowCols; ++u)
+      if (tid + 256 * q < n && u < ncol) st(B + (size_t)(j0 + u) * n + tid + 256 * q, x[q][u]);
+}
+
+// rows per thread by size
+template <class K>
+hipError_t launch_rows(K k1, K k2, K k3, K k4, hipStream_t s, const ChainDesc* chains, int nchains, int nmax, MatRef A,
+                       MatRef X) {
+  const K fn = nmax <= 256 ? k1 : nmax <= 512 ? k2 : nmax <= 768 ? k3 : k4;
+  hipLaunchKernelGGL(fn, dim3((nmax + kRowCols - 1) / kRowCols, nchains), dim3(256), 0, s, chains, A, X);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -1651,11 +1848,8 @@ hipError_t launch_form_Q_blocked(hipStream_t s, const ChainDesc* chains, int nch
     const int cb = mfma_cols(nmax);
     if (cb) return launch_mfma_classes(k_form_Q_mfma<16>, k_form_Q_mfma<8>, s, nchains, nmax, chains, A, Q);
   }
-  // many chains fill the chip with fewer, wider column blocks: each reads the reflectors once
-  if (nchains >= kWideColChains && nmax <= 400) return launch_form_Q_blocked_nb<8, 16>(s, chains, nchains, nmax, A, Q);
-  if (nchains >= kWideColChains && nmax <= 576) return launch_form_Q_blocked_nb<8, 8>(s, chains, nchains, nmax, A, Q);
-  if (nmax <= 640) return launch_form_Q_blocked_nb<8, 4>(s, chains, nchains, nmax, A, Q);
-  return launch_form_Q_blocked_nb<8, 1>(s, chains, nchains, nmax, A, Q);
+  return launch_rows(k_form_Q_rows<1>, k_form_Q_rows<2>, k_form_Q_rows<3>, k_form_Q_rows<4>, s, chains, nchains, nmax, A,
+                     Q);
 }
 
 hipError_t launch_qr_solve(hipStream_t s, const ChainDesc* chains, int nchains, int nmax, MatRef A, MatRef B, int nb) {
@@ -1667,8 +1861,8 @@ hipError_t launch_qr_solve(hipStream_t s, const ChainDesc* chains, int nchains, 
     const int cb = mfma_cols(nmax);
     if (cb) return launch_mfma_classes(k_qr_solve_mfma<16>, k_qr_solve_mfma<8>, s, nchains, nmax, chains, A, B);
   }
-  if (nmax <= 640) return launch_qr_solve_nb<8, 4>(s, chains, nchains, nmax, A, B);
-  return launch_qr_solve_nb<8, 1>(s, chains, nchains, nmax, A, B);
+  return launch_rows(k_qr_solve_rows<1>, k_qr_solve_rows<2>, k_qr_solve_rows<3>, k_qr_solve_rows<4>, s, chains, nchains,
+                     nmax, A, B);
 }
 
 }  // namespace dqmc
