@@ -25,128 +25,85 @@ constexpr int KT = 16;  // K chunk
 // (measured on gfx950 with an in-bounds probe of the builtin).
 __device__ inline int kMfmaRow(int lane, int v) { return (lane >> 4) + 4 * v; }
 
-// Shared tile loader: As[r][kk] = op(A)[i0 + r][k0 + kk], Bs[kk][c] = op(B)[k0 + kk][j0 + c].
+// One K chunk of this thread: two entries of op(A) (rows i0 .., K chunk at k0) and two of op(B).
+// Consecutive lanes run along the stored columns.
 template <int OPA, int OPB>
-__device__ inline void load_tiles(const cplx* A, const cplx* B, int n, int i0, int j0, int k0,
-                                  double (*As_re)[KT + 1], double (*As_im)[KT + 1], double (*Bs_re)[GT + 1],
-                                  double (*Bs_im)[GT + 1]) {
-  const int tid = threadIdx.x;
+struct GemmTile {
+  int ar[2], ak[2], bk[2], bc[2];
+  __device__ GemmTile(int tid) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int e = tid + 256 * t;
-    int r, kk;
-    if (OPA == OP_N) {
-      r = e & 31;
-      kk = e >> 5;
-    } else {
-      kk = e & 15;
-      r = e >> 4;
+    for (int t = 0; t < 2; ++t) {
+      const int e = tid + 256 * t;
+      ar[t] = OPA == OP_N ? e & 31 : e >> 4;
+      ak[t] = OPA == OP_N ? e >> 5 : e & 15;
+      bk[t] = OPB == OP_N ? e & 15 : e >> 5;
+      bc[t] = OPB == OP_N ? e >> 4 : e & 31;
     }
-    const int gi = i0 + r, gk = k0 + kk;
-    cplx v = mk(0, 0);
-    if (gi < n && gk < n) v = (OPA == OP_N) ? A[(size_t)gk * n + gi] : conj(A[(size_t)gi * n + gk]);
-    As_re[r][kk] = v.re;
-    As_im[r][kk] = v.im;
   }
+  __device__ void load(const gcplx* A, const gcplx* B, int n, int i0, int j0, int k0, cplx (&a)[2], cplx (&b)[2]) const {
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int e = tid + 256 * t;
-    int kk, cc;
-    if (OPB == OP_N) {
-      kk = e & 15;
-      cc = e >> 4;
-    } else {
-      cc = e & 31;
-      kk = e >> 5;
+    for (int t = 0; t < 2; ++t) {
+      const int gi = min(i0 + ar[t], n - 1), ga = min(k0 + ak[t], n - 1);
+      a[t] = ld(A + (OPA == OP_N ? (size_t)ga * n + gi : (size_t)gi * n + ga));
+      if (OPA != OP_N) a[t] = conj(a[t]);
+      if (i0 + ar[t] >= n || k0 + ak[t] >= n) a[t] = mk(0, 0);
+      const int gb = min(k0 + bk[t], n - 1), gj = min(j0 + bc[t], n - 1);
+      b[t] = ld(B + (OPB == OP_N ? (size_t)gj * n + gb : (size_t)gb * n + gj));
+      if (OPB != OP_N) b[t] = conj(b[t]);
+      if (k0 + bk[t] >= n || j0 + bc[t] >= n) b[t] = mk(0, 0);
     }
-    const int gk = k0 + kk, gj = j0 + cc;
-    cplx v = mk(0, 0);
-    if (gk < n && gj < n) v = (OPB == OP_N) ? B[(size_t)gj * n + gk] : conj(B[(size_t)gk * n + gj]);
-    Bs_re[kk][cc] = v.re;
-    Bs_im[kk][cc] = v.im;
   }
-}
+};
 
-template <int OPA, int OPB>
+// Bound by the latency of a K chunk where a chain's tiles do not fill the chip (n = 64: 4 tiles,
+// n = 400: 169): the next chunk's loads are under way while one is multiplied. NBUF = 2: out of one of
+// two LDS buffers, one barrier per chunk; n = 64 9.4 -> 7.8 us, n = 400 53 -> 33 us, n = 1024 185 -> 181
+// us. NBUF = 1 with many tiles (64 chains of n = 400: 690 us): two buffers halve the workgroups a
+// CU holds, 717 us.
+template <int OPA, int OPB, int NBUF>
 __global__ __launch_bounds__(256) void k_gemm(const ChainDesc* chains, MatRef Cr, MatRef Ar, MatRef Br, VecRef dlr,
                                               VecRef drr, double beta) {
   const ChainDesc& c = chains[blockIdx.z];
   const int n = c.n;
   const int i0 = blockIdx.y * GT, j0 = blockIdx.x * GT;
   if (i0 >= n || j0 >= n) return;
-  const cplx* A = matptr(c, Ar);
-  const cplx* B = matptr(c, Br);
-  cplx* C = matptr(c, Cr);
-  const double* dl = dlr.kind >= 0 ? vecptr(c, dlr) : nullptr;
-  const double* dr = drr.kind >= 0 ? vecptr(c, drr) : nullptr;
+  const gcplx* A = gp(matptr(c, Ar));
+  const gcplx* B = gp(matptr(c, Br));
+  gcplx* C = gp(matptr(c, Cr));
+  const gdouble* dl = dlr.kind >= 0 ? gp(vecptr(c, dlr)) : nullptr;
+  const gdouble* dr = drr.kind >= 0 ? gp(vecptr(c, drr)) : nullptr;
 
-  __shared__ double As_re[GT][KT + 1], As_im[GT][KT + 1];
-  __shared__ double Bs_re[KT][GT + 1], Bs_im[KT][GT + 1];
+  __shared__ double As_re[NBUF][GT][KT + 1], As_im[NBUF][GT][KT + 1];
+  __shared__ double Bs_re[NBUF][KT][GT + 1], Bs_im[NBUF][KT][GT + 1];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wr = w >> 1, wc = w & 1;
+  const GemmTile<OPA, OPB> tile(tid);
   v4d acc_re = {0, 0, 0, 0}, acc_im = {0, 0, 0, 0};
-
-  for (int k0 = 0; k0 < n; k0 += KT) {
-    // A tile: rows i0..i0+31, k k0..k0+15
+  cplx a[2], b[2];
+  tile.load(A, B, n, i0, j0, 0, a, b);
+  for (int k0 = 0, buf = 0; k0 < n; k0 += KT, buf ^= NBUF - 1) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int e = tid + 256 * t;
-      int r, kk;
-      if (OPA == OP_N) {
-        r = e & 31;
-        kk = e >> 5;
-      } else {
-        kk = e & 15;
-        r = e >> 4;
-      }
-      const int gi = i0 + r, gk = k0 + kk;
-      cplx v = mk(0, 0);
-      if (gi < n && gk < n) {
-        if (OPA == OP_N)
-          v = A[(size_t)gk * n + gi];
-        else
-          v = conj(A[(size_t)gi * n + gk]);
-      }
-      As_re[r][kk] = v.re;
-      As_im[r][kk] = v.im;
+      As_re[buf][tile.ar[t]][tile.ak[t]] = a[t].re;
+      As_im[buf][tile.ar[t]][tile.ak[t]] = a[t].im;
+      Bs_re[buf][tile.bk[t]][tile.bc[t]] = b[t].re;
+      Bs_im[buf][tile.bk[t]][tile.bc[t]] = b[t].im;
     }
-    // B tile: k k0..k0+15, cols j0..j0+31
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int e = tid + 256 * t;
-      int kk, cc;
-      if (OPB == OP_N) {
-        kk = e & 15;
-        cc = e >> 4;
-      } else {
-        cc = e & 31;
-        kk = e >> 5;
-      }
-      const int gk = k0 + kk, gj = j0 + cc;
-      cplx v = mk(0, 0);
-      if (gk < n && gj < n) {
-        if (OPB == OP_N)
-          v = B[(size_t)gj * n + gk];
-        else
-          v = conj(B[(size_t)gk * n + gj]);
-      }
-      Bs_re[kk][cc] = v.re;
-      Bs_im[kk][cc] = v.im;
-    }
+    if (k0 + KT < n) tile.load(A, B, n, i0, j0, k0 + KT, a, b);
     __syncthreads();
 #pragma unroll
     for (int kk = 0; kk < KT; kk += 4) {
       const int ar = wr * 16 + (lane & 15), ak = kk + (lane >> 4);
       const int bk = kk + (lane >> 4), bc = wc * 16 + (lane & 15);
-      const double a_re = As_re[ar][ak], a_im = As_im[ar][ak];
-      const double b_re = Bs_re[bk][bc], b_im = Bs_im[bk][bc];
+      const double a_re = As_re[buf][ar][ak], a_im = As_im[buf][ar][ak];
+      const double b_re = Bs_re[buf][bk][bc], b_im = Bs_im[buf][bk][bc];
       acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(a_re, b_re, acc_re, 0, 0, 0);
-      acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a_im, b_im, acc_re, 0, 0, 0);
       acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(a_re, b_im, acc_im, 0, 0, 0);
+      acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a_im, b_im, acc_re, 0, 0, 0);
       acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(a_im, b_re, acc_im, 0, 0, 0);
     }
-    __syncthreads();
+    if (NBUF == 1) __syncthreads();
   }
   const int col = j0 + wc * 16 + (lane & 15);
 #pragma unroll
@@ -158,8 +115,8 @@ __global__ __launch_bounds__(256) void k_gemm(const ChainDesc* chains, MatRef Cr
       if (dr) s *= dr[col];
       cplx val = mk(s * acc_re[v], s * acc_im[v]);
       const size_t o = (size_t)col * n + row;
-      if (beta != 0.0) val = val + beta * C[o];
-      C[o] = val;
+      if (beta != 0.0) val = val + beta * ld(C + o);
+      st(C + o, val);
     }
   }
 }
@@ -167,14 +124,19 @@ __global__ __launch_bounds__(256) void k_gemm(const ChainDesc* chains, MatRef Cr
 hipError_t launch_gemm(hipStream_t s, const ChainDesc* chains, int nchains, int nmax, MatRef C, MatRef A,
                        GemmOp opA, MatRef B, GemmOp opB, VecRef dl, VecRef dr, double beta) {
   dim3 grid((nmax + GT - 1) / GT, (nmax + GT - 1) / GT, nchains);
+  // two buffers as long as every workgroup of the launch can be resident with them (4 per CU)
+  const bool two = (long long)grid.x * grid.y * grid.z <= 4 * 256;
+  auto run = [&](auto one_buf, auto two_buf) {
+    hipLaunchKernelGGL((two ? two_buf : one_buf), grid, dim3(256), 0, s, chains, C, A, B, dl, dr, beta);
+  };
   if (opA == OP_N && opB == OP_N)
-    hipLaunchKernelGGL((k_gemm<OP_N, OP_N>), grid, dim3(256), 0, s, chains, C, A, B, dl, dr, beta);
+    run(k_gemm<OP_N, OP_N, 1>, k_gemm<OP_N, OP_N, 2>);
   else if (opA == OP_N && opB == OP_C)
-    hipLaunchKernelGGL((k_gemm<OP_N, OP_C>), grid, dim3(256), 0, s, chains, C, A, B, dl, dr, beta);
+    run(k_gemm<OP_N, OP_C, 1>, k_gemm<OP_N, OP_C, 2>);
   else if (opA == OP_C && opB == OP_N)
-    hipLaunchKernelGGL((k_gemm<OP_C, OP_N>), grid, dim3(256), 0, s, chains, C, A, B, dl, dr, beta);
+    run(k_gemm<OP_C, OP_N, 1>, k_gemm<OP_C, OP_N, 2>);
   else
-    hipLaunchKernelGGL((k_gemm<OP_C, OP_C>), grid, dim3(256), 0, s, chains, C, A, B, dl, dr, beta);
+    run(k_gemm<OP_C, OP_C, 1>, k_gemm<OP_C, OP_C, 2>);
   return hipGetLastError();
 }
 

@@ -938,11 +938,11 @@ __global__ __launch_bounds__(256) void k_local_updates_delayed(const ChainDesc* 
 //  * after them it has four sites' G'_jj from A_j, B_j and the blocks read before, and one
 //    chain of M, its 2 x 2 minors, cofactors (lane-parallel, DPP moves) and determinant.
 // Two barriers per acceptance. Against windows that kept H, U, P and B_b per own column and
-// evaluated proposals from the field on 4 waves, per slice: n = 64 65 -> 43, n = 256 254 -> 178,
-// n = 400 447 -> 287, n = 1024 (128 -> 256 workgroups, own columns now in LDS) 2983 -> 1049,
-// 64 chains of n = 400 2190 -> 1044 us. At n = 400, cycles per slice: decisions 425,000 ->
-// 220,000 (a round of four is one chain of some 300 instructions), factors 168,000 -> 90,000,
-// window ends 358,000 -> 120,000, barriers 141,000 (one contended counter per window).
+// evaluated proposals from the field on 4 waves, per slice: n = 64 65 -> 43, n = 256 254 -> 164,
+// n = 400 447 -> 262, n = 1024 (128 -> 256 workgroups, own columns now in LDS) 2983 -> 773,
+// 64 chains of n = 400 2190 -> 1050 us. At n = 400, cycles per slice: decisions 425,000 ->
+// 210,000 (a round of four is one chain of some 300 instructions), factors 168,000 -> 87,000,
+// window ends 358,000 -> 134,000, barriers 141,000 -> 75,000 (flag_sync).
 //
 // TILE: the own columns of G stay in LDS for the slice and a window's end publishes (in
 // M_GALT) just the columns of the next window's sites, all others read nothing else; the last

@@ -1744,9 +1744,9 @@ inline size_t mfma_lds(int nmax, int cb) {
   return ((size_t)(cb + 8) * mfma_ld(nmax) + kMfmaScratch) * sizeof(cplx);
 }
 
-// chain counts from which k_form_Q_blocked uses 8 or 16 columns per workgroup (k_qr_solve
-// keeps 4: its time per workgroup is the latency of the panel sequence, and wider blocks
-// measured slower)
+// chain counts from which solve and Q formation take the matrix-core kernels (16 or 8 columns
+// per workgroup); with fewer, the latency of the panel sequence counts and four columns in
+// registers finish sooner
 constexpr int kWideColChains = 8;
 
 // default panel width: 8 (the register-resident panel keeps nb x rows-per-thread values per
