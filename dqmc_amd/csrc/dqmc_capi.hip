@@ -543,42 +543,64 @@ struct Ops {
       LCHK(launch_apply_B_chkr(s(), d(), nc(), g.n, g.N, X, op, slice, nullptr, g.ngroups));
       return 0;
     }
-    // dense: B = eT2 eV, B^-1 = eV^-1 eTinv2, B^dagger = eV eT2^dagger
-    const MatRef T4 = NM(M_TMP4);
+    MatRef at = X;
+    RC(dense_B(at, X, op, slice));
+    return copy(X, NM(M_TMP4));
+  }
+  // Without the checkerboard, B = eT2 eV, B^-1 = eV^-1 eTinv2, B^dagger = eV eT2^dagger: the product
+  // cannot be formed in place, so the matrix moves from `at` to the other one of X and M_TMP4,
+  // and `at` follows it.
+  int dense_B(MatRef& at, MatRef X, BOp op, int slice) {
+    const bool home = at.kind == X.kind && at.idx == X.idx;
+    const MatRef from = at, to = home ? NM(M_TMP4) : X;
+    at = to;
     switch (op) {
       case B_LEFT:
-        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, X, false, 0, 1.0, slice, nullptr));
-        LCHK(launch_gemm(s(), d(), nc(), g.n, T4, NM(M_ET2), OP_N, X, OP_N, NOVEC, NOVEC, 0.0));
-        return copy(X, T4);
+        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, from, false, 0, 1.0, slice, nullptr));
+        LCHK(launch_gemm(s(), d(), nc(), g.n, to, NM(M_ET2), OP_N, from, OP_N, NOVEC, NOVEC, 0.0));
+        return 0;
       case B_RIGHT:
-        LCHK(launch_gemm(s(), d(), nc(), g.n, T4, X, OP_N, NM(M_ET2), OP_N, NOVEC, NOVEC, 0.0));
-        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, T4, true, 1, 1.0, slice, nullptr));
-        return copy(X, T4);
+        LCHK(launch_gemm(s(), d(), nc(), g.n, to, from, OP_N, NM(M_ET2), OP_N, NOVEC, NOVEC, 0.0));
+        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, to, true, 1, 1.0, slice, nullptr));
+        return 0;
       case B_INV_LEFT:
-        LCHK(launch_gemm(s(), d(), nc(), g.n, T4, NM(M_ETINV2), OP_N, X, OP_N, NOVEC, NOVEC, 0.0));
-        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, T4, false, 0, -1.0, slice, nullptr));
-        return copy(X, T4);
+        LCHK(launch_gemm(s(), d(), nc(), g.n, to, NM(M_ETINV2), OP_N, from, OP_N, NOVEC, NOVEC, 0.0));
+        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, to, false, 0, -1.0, slice, nullptr));
+        return 0;
       case B_INV_RIGHT:
-        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, X, true, 1, -1.0, slice, nullptr));
-        LCHK(launch_gemm(s(), d(), nc(), g.n, T4, X, OP_N, NM(M_ETINV2), OP_N, NOVEC, NOVEC, 0.0));
-        return copy(X, T4);
+        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, from, true, 1, -1.0, slice, nullptr));
+        LCHK(launch_gemm(s(), d(), nc(), g.n, to, from, OP_N, NM(M_ETINV2), OP_N, NOVEC, NOVEC, 0.0));
+        return 0;
       case B_DAG_LEFT:
-        LCHK(launch_gemm(s(), d(), nc(), g.n, T4, NM(M_ET2), OP_C, X, OP_N, NOVEC, NOVEC, 0.0));
-        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, T4, false, 2, 1.0, slice, nullptr));
-        return copy(X, T4);
+        LCHK(launch_gemm(s(), d(), nc(), g.n, to, NM(M_ET2), OP_C, from, OP_N, NOVEC, NOVEC, 0.0));
+        LCHK(launch_apply_eV(s(), d(), nc(), g.n, g.N, to, false, 2, 1.0, slice, nullptr));
+        return 0;
     }
     return fail(DQMC_E_ARG, "bad B op");
+  }
+  // X <- op(B_l) X for count slices from `slice` on, step +1 or -1 (left operators)
+  int applyB_run(MatRef X, BOp op, int slice, int step, int count) {
+    if (g.chkr) {
+      for (int t = 0; t < count; ++t) RC(applyB(X, op, slice + step * t));
+      return 0;
+    }
+    MatRef at = X;
+    for (int t = 0; t < count; ++t) RC(dense_B(at, X, op, slice + step * t));
+    return count & 1 ? copy(X, at) : 0;
   }
 
   // wrap_greens! (stack.jl:316-325), slice 1-based as in the reference
   int wrap(MatRef X, int slice, int direction) {
-    int rc;
-    if (direction == -1) {
-      if ((rc = applyB(X, B_INV_LEFT, slice - 2))) return rc;
-      return applyB(X, B_RIGHT, slice - 2);
+    const bool down = direction == -1;
+    const BOp left = down ? B_INV_LEFT : B_LEFT, right = down ? B_RIGHT : B_INV_RIGHT;
+    const int sl = down ? slice - 2 : slice - 1;
+    if (g.chkr) {
+      RC(applyB(X, left, sl));
+      return applyB(X, right, sl);
     }
-    if ((rc = applyB(X, B_LEFT, slice - 1))) return rc;
-    return applyB(X, B_INV_RIGHT, slice - 1);
+    MatRef at = X;  // to M_TMP4 and back
+    RC(dense_B(at, X, left, sl));
+    return dense_B(at, X, right, sl);
   }
 
   int identity_elem(int k) {
@@ -605,8 +627,7 @@ struct Ops {
   int add_left(int idx) {
     int rc;
     if ((rc = copy(NM(M_CURU), US(idx)))) return rc;
-    for (int sl = idx * g.s; sl < (idx + 1) * g.s; ++sl)
-      if ((rc = applyB(NM(M_CURU), B_LEFT, sl))) return rc;
+    if ((rc = applyB_run(NM(M_CURU), B_LEFT, idx * g.s, 1, g.s))) return rc;
     LCHK(launch_scale_cols(s(), d(), nc(), g.n, NM(M_CURU), DS(idx)));
     if ((rc = udt(NM(M_CURU), DS(idx + 1), US(idx + 1), NM(M_QRT), true))) return rc;
     return gemm(TS(idx + 1), NM(M_QRT), OP_N, TS(idx), OP_N);
@@ -616,8 +637,7 @@ struct Ops {
   int add_right(int idx) {
     int rc;
     if ((rc = copy(NM(M_CURU), US(idx + 1)))) return rc;
-    for (int sl = (idx + 1) * g.s - 1; sl >= idx * g.s; --sl)
-      if ((rc = applyB(NM(M_CURU), B_DAG_LEFT, sl))) return rc;
+    if ((rc = applyB_run(NM(M_CURU), B_DAG_LEFT, (idx + 1) * g.s - 1, -1, g.s))) return rc;
     LCHK(launch_scale_cols(s(), d(), nc(), g.n, NM(M_CURU), DS(idx + 1)));
     if ((rc = udt(NM(M_CURU), DS(idx), US(idx), NM(M_QRT), true))) return rc;
     return gemm(TS(idx), NM(M_QRT), OP_N, TS(idx + 1), OP_N);
