@@ -187,7 +187,8 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
 
   extern __shared__ double smem[];
   cplx* P = reinterpret_cast<cplx*>(smem);  // [NB][ps] panel V (rows k0..n-1 used, row r at 16 + r)
-  // [4][2][64] per-wave partial W of the tile form; [4][8][16] W of the 16-column trailing update
+  // [2][4][2][64] per-wave partial W of the tile form (two halves by turns, see apply_tiles);
+  // [4][8][16] W of the 16-column trailing update
   double* part = reinterpret_cast<double*>(P + (size_t)NB * ps);
   cplx* wscr = reinterpret_cast<cplx*>(part);
   __shared__ int perm[kQrMaxN], lpos[kQrMaxN];
@@ -270,7 +271,11 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
           if (tr + 64 * tt + 4 * v >= lo) a[2 * (tr + 64 * tt + 4 * v)] = X[tt][v];
       }
   };
-  // X <- (I - V T^H V^H) X with V (rows >= k0) in P and T in Tl
+  // X <- (I - V T^H V^H) X with V (rows >= k0) in P and T in Tl. Nothing but the barrier in here
+  // orders one block against the next, so a wave that is ahead writes the next block's partial
+  // sums while another still reads this block's: they alternate between two halves of `part`, and
+  // a half is written again only behind the barrier of the block between.
+  int half = 0;
   auto apply_tiles = [&](int k0) __attribute__((always_inline)) {
     const int t0 = first_tile(k0);
     v4d acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
@@ -287,11 +292,13 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
     // Vr Xr + Vi Xi (li < 8) and Vr Xi - Vi Xr (li >= 8); Vi's rows are 8 further down the tile,
     // the other component is 8 lanes away. Then the sum over the waves.
     const double o0 = dpp_move<0x128>(acc0[2] + acc1[2]), o1 = dpp_move<0x128>(acc0[3] + acc1[3]);  // row_ror:8
-    part[wave * 128 + lane] = (acc0[0] + acc1[0]) + (lim ? -o0 : o0);
-    part[wave * 128 + 64 + lane] = (acc0[1] + acc1[1]) + (lim ? -o1 : o1);
+    double* sums = part + half;
+    half ^= 512;
+    sums[wave * 128 + lane] = (acc0[0] + acc1[0]) + (lim ? -o0 : o0);
+    sums[wave * 128 + 64 + lane] = (acc0[1] + acc1[1]) + (lim ? -o1 : o1);
     __syncthreads();
-    const double w0 = (part[lane] + part[128 + lane]) + (part[256 + lane] + part[384 + lane]);
-    const double w1 = (part[64 + lane] + part[192 + lane]) + (part[320 + lane] + part[448 + lane]);
+    const double w0 = (sums[lane] + sums[128 + lane]) + (sums[256 + lane] + sums[384 + lane]);
+    const double w1 = (sums[64 + lane] + sums[192 + lane]) + (sums[320 + lane] + sums[448 + lane]);
     // That is the B operand of Z = T^H W: [Zr Zi] = Tr^T [Wr Wi] + Ti^T [Wi -Wr], and element 0
     // (1) of the product is row lk (lk + 4) of [Zr Zi], the B operand of the update
     const cplx t0l = Tl[lk * NB + lu], t1l = Tl[(lk + 4) * NB + lu];

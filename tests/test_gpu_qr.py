@@ -41,3 +41,26 @@ def test_blocked_qr_sizes_and_workgroups(amd, L):
         assert (np.abs((U * D) @ T - A) / np.linalg.norm(A, axis=0)).max() <= 8 * n * EPS
         assert np.all(D > 0)
     c.close()
+
+
+@pytest.mark.parametrize("L,wgs", [(2, (1, 3)), (4, (1, 3, 4, 8)), (5, (1, 2, 4, 9)), (8, (1, 4, 7, 32)),
+                                   (10, (1, 5, 6, 25, 50)), (12, (1, 6, 25, 72)), (13, (1, 10, 84)), (16, (1, 11, 128))])
+def test_factors_do_not_depend_on_blocks_per_workgroup(amd, L, wgs):
+    """A block's update is the same arithmetic whichever workgroup makes it and whatever that
+    workgroup holds besides (fewer than 128 columns each, beyond that the 16-column form takes
+    over), so U, D and T are equal bit for bit. Where a workgroup holds several blocks, the waves'
+    partial sums of consecutive blocks follow one another through LDS."""
+    n = 4 * L * L
+    rng = np.random.default_rng(50 + L)
+    A = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))) * np.exp(rng.uniform(-20, 20, n))
+    c = amd.DQMC(amd.Params(L=L, slices=20, hoppings=(1.0, 0.5, 0.5, 1.0), lam=1.0, r=1.0))
+    want = None
+    for wg in wgs[::-1]:
+        assert wg == 1 or n < 128 * (wg - 1)
+        print("blocked QR n=%d workgroups %d" % (n, wg), flush=True)
+        c.set_groups(wg_qr=wg)
+        got = c.decompose_udt_prepivoted(A)
+        want = want or got
+        for x, y in zip(got, want):
+            assert np.array_equal(x, y)
+    c.close()
