@@ -100,7 +100,9 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
     if (lane == 0) vn1[cl] = vn2[cl] = nr;
   }
 
-  // publish best own column among logical positions >= first, for step `first`
+  // publish best own column among logical positions >= first, for step `first`. A norm that is
+  // not a number counts as -0.5, behind every number and before "no column" (-1): such columns
+  // come last, in order of position, every step has its candidate, and the factors show the NaN.
   auto publish = [&](int first) {
     const int buf = first & 1;
     double best = -1.0;
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
       for (int cl = wave; cl < ncol; cl += nwaves) {
         const int lp = lpos[w + cl * W];
         if (lp < first) continue;
-        const double nv = vn1[cl];
+        const double nv = vn1[cl] >= 0.0 ? vn1[cl] : -0.5;
         if (nv > best || (nv == best && lp < bestl)) {
           best = nv;
           bestc = cl;
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(256) void k_qrp(const ChainDesc* chains, MatRef Ar,
           bw = ow;
         }
       }
-      const bool failed = __ballot(fail) != 0 || bw < 0;
+      const bool failed = __ballot(fail) != 0;
       if (lane == 0) {
         s_win = bw;
         if (failed) {

@@ -64,3 +64,30 @@ def test_factors_do_not_depend_on_blocks_per_workgroup(amd, L, wgs):
         for x, y in zip(got, want):
             assert np.array_equal(x, y)
     c.close()
+
+
+@pytest.mark.parametrize("L,wg", [(2, 0), (4, 0), (4, 1), (4, 3), (8, 0), (8, 128)])
+def test_pivoted_qr_of_nan_columns(amd, L, wg):
+    """Columns without a norm come last, so the pivots before them are those of the same matrix with
+    zeros there, and D is NaN from the first of them on (one NaN reflector reaches every column);
+    nothing is left of the factorisation before, and the next one is unaffected."""
+    n = 4 * L * L
+    print("pivoted QR with NaN, n=%d workgroups %d" % (n, wg), flush=True)
+    rng = np.random.default_rng(70 + L)
+    A = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    c = amd.DQMC(amd.Params(L=L, slices=20, hoppings=(1.0, 0.5, 0.5, 1.0), lam=1.0, r=1.0))
+    if wg:
+        c.set_groups(wg_qr=wg)
+    first = c.decompose_udt(A)
+    for bad in ([0], [n - 1], [1, n // 2, n - 2], list(range(n))):
+        Z, B = A.copy(), A.copy()
+        Z[:, bad] = 0
+        B[n // 3, bad] = np.nan
+        U, D, T = c.decompose_udt(B)
+        good = n - len(bad)
+        if good:
+            assert np.array_equal(D[:good], c.decompose_udt(Z)[1][:good])
+        assert np.isnan(D[good:]).all() and np.isnan(U).any() and np.isnan(T).any()
+    for x, y in zip(c.decompose_udt(A), first):
+        assert np.array_equal(x, y)
+    c.close()
