@@ -36,6 +36,11 @@ inline int mfma_ld(int nmax) { return nmax + ((17 - (nmax & 15)) & 15); }
 __device__ inline cplx shfl_c(cplx v, int src) { return mk(__shfl(v.re, src, 64), __shfl(v.im, src, 64)); }
 __device__ inline cplx read_lane_c(cplx v, int lane) { return mk(read_lane(v.re, lane), read_lane(v.im, lane)); }
 
+// A column norm as the pre-pivoting order takes it: one that is not a number counts as -1, behind
+// every number. With the NaN itself no comparison would hold and columns would share a rank,
+// which leaves entries of the permutation unset.
+__device__ inline double order_norm(double v) { return v >= 0.0 ? v : -1.0; }
+
 // Panel staging between A (global) and P (LDS, [NB][n], rows k0..n-1 of each column);
 // logical column k is physical column perm[k] (perm == nullptr: the identity).
 // Each thread moves one row of all NB columns per step: the NB loads are issued before
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
   if (group_failed(g)) return;
   if (prepivot) {
     double* vn = reinterpret_cast<double*>(P);  // n doubles, before the panel buffer is used
-    for (int k = tid; k < n; k += blockDim.x) vn[k] = gp(c.qr_vn)[k];
+    for (int k = tid; k < n; k += blockDim.x) vn[k] = order_norm(gp(c.qr_vn)[k]);
     __syncthreads();
     for (int col = tid; col < n; col += blockDim.x) {
       const double v = vn[col];
@@ -748,7 +753,7 @@ __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, Mat
     group_sync(g);
     if (group_failed(g)) return;
     double* vn = reinterpret_cast<double*>(P);  // n doubles, before the panel buffer is used
-    for (int k = tid; k < n; k += blockDim.x) vn[k] = gp(c.qr_vn)[k];
+    for (int k = tid; k < n; k += blockDim.x) vn[k] = order_norm(gp(c.qr_vn)[k]);
     __syncthreads();
     for (int col = tid; col < n; col += blockDim.x) {
       const double v = vn[col];

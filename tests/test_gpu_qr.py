@@ -91,3 +91,29 @@ def test_pivoted_qr_of_nan_columns(amd, L, wg):
     for x, y in zip(c.decompose_udt(A), first):
         assert np.array_equal(x, y)
     c.close()
+
+
+@pytest.mark.parametrize("L,wg,nb", [(2, 0, 8), (4, 0, 8), (4, 1, 8), (4, 3, 16), (8, 0, 8), (10, 0, 16), (16, 0, 8)])
+def test_blocked_qr_of_nan_columns(amd, L, wg, nb):
+    """As for the pivoted QR: the order puts columns without a norm last, by index, so that R of the
+    panels before them is that of the same matrix with zeros there."""
+    n = 4 * L * L
+    print("blocked QR with NaN, n=%d workgroups %d panels of %d" % (n, wg, nb), flush=True)
+    rng = np.random.default_rng(90 + L)
+    A = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    c = amd.DQMC(amd.Params(L=L, slices=20, hoppings=(1.0, 0.5, 0.5, 1.0), lam=1.0, r=1.0))
+    c.set_qr_panel(nb)
+    if wg:
+        c.set_groups(wg_qr=wg)
+    first = c.decompose_udt_prepivoted(A)
+    for bad in ([0], [n - 1], [1, n // 2, n - 2], list(range(n))):
+        Z, B = A.copy(), A.copy()
+        Z[:, bad] = 0
+        B[n // 3, bad] = np.nan
+        U, D, T = c.decompose_udt_prepivoted(B)
+        whole = (n - len(bad)) // nb * nb  # columns of the panels without a NaN
+        assert np.array_equal(D[:whole], c.decompose_udt_prepivoted(Z)[1][:whole])
+        assert np.isnan(D[n - len(bad):]).all() and np.isnan(U).any() and np.isnan(T).any()
+    for x, y in zip(c.decompose_udt_prepivoted(A), first):
+        assert np.array_equal(x, y)
+    c.close()
