@@ -468,7 +468,7 @@ __global__ __launch_bounds__(256) void k_gj_inverse(const ChainDesc* chains, Mat
       __syncthreads();
     }
     if (tid == 0) {
-      s_p = ri[0];
+      s_p = ri[0] < n ? ri[0] : k;  // (nothing but NaN left: no row to move, the inverse is NaN)
       pivl[k] = s_p;
     }
     __syncthreads();
