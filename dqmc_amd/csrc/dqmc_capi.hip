@@ -45,8 +45,8 @@ int fail(int code, const std::string& msg) {
     if (_rc) return _rc; \
   } while (0)
 
-constexpr int kMaxWG = 128;
-constexpr int kMaxLocalWG = 256;  // default workgroups of one chain's local updates: one per CU
+constexpr int kMaxWG = 128;  // most workgroups of one chain's QR and inverse
+constexpr int kMaxLocalWG = 256;  // the same for one chain's local updates: one per CU
 
 MatRef NM(int id) { return MatRef{MK_NAMED, id}; }
 MatRef US(int k) { return MatRef{MK_USTACK, k}; }
@@ -1855,7 +1855,7 @@ int dqmc_ctx_destroy(dqmc_ctx* ctx) {
 
 int dqmc_batch_set_groups(dqmc_batch* b, int wg_qr, int wg_inv, int wg_local) {
   if (!b) return fail(DQMC_E_ARG, "null batch");
-  if (wg_qr > kMaxWG || wg_inv > kMaxWG || wg_local > kMaxWG) return fail(DQMC_E_ARG, "too many workgroups");
+  if (wg_qr > kMaxWG || wg_inv > kMaxWG || wg_local > kMaxLocalWG) return fail(DQMC_E_ARG, "too many workgroups");
   RC(batch_sync(b));
   b->drop_mgraphs();
   for (auto& g : b->groups) {
@@ -3461,11 +3461,16 @@ int autotune_group(dqmc_batch* b, Group& g, double box, int reps, double* rep) {
   // fit, and that candidate is skipped); the groups of a mixed batch run concurrently, so
   // their cooperative grids together must fit one workgroup per CU
   const int total = (int)b->chains.size();
-  const int cap = b->groups.size() == 1 ? std::max(1, std::min({kMaxWG, std::max(1, 1024 / nch), g.n / 2}))
-                                        : std::max(1, std::min({kMaxWG, 256 / total, g.n / 2}));
-  std::vector<int> wgs;
-  for (int w : {1, 2, 3, 4, 6, 8, 12, 16, 25, 32, 50, 64, 100, 128})
-    if (w <= cap) wgs.push_back(w);
+  const int cap = b->groups.size() == 1 ? std::max(1, std::min({kMaxLocalWG, std::max(1, 1024 / nch), g.n / 2}))
+                                        : std::max(1, std::min({kMaxLocalWG, 256 / total, g.n / 2}));
+  // the present count is always among the candidates, so that tuning never ends on a slower one
+  auto candidates = [&](int now) {
+    std::vector<int> wgs;
+    for (int w : {1, 2, 3, 4, 6, 8, 12, 16, 25, 32, 50, 64, 100, 128, 192, 256})
+      if (w <= cap && w != now) wgs.push_back(w);
+    wgs.push_back(now);
+    return wgs;
+  };
   // ---- local updates
   auto reset_local = [&]() -> int {
     if (restore()) return 1;
@@ -3477,8 +3482,9 @@ int autotune_group(dqmc_batch* b, Group& g, double box, int reps, double* rep) {
   };
   float best_local = 1e30f;
   int best_w = g.wg_local, best_v = g.local_variant;
-  for (int w : wgs)
-    for (int v : {4, 2, 3}) {
+  for (int w : candidates(g.wg_local))
+    for (int v : {4, 2, 3, 1}) {
+      if (v == 1 && (g.local_variant != 1 || w != g.wg_local)) continue;
       if (v == 4 && local_window_sites(g.n, w) < 2) continue;
       if (v == 2 && !local_tile_fits(g.n, w)) continue;
       if (v == 3 && !local_delayed_fits(g.n)) continue;
@@ -3506,8 +3512,8 @@ int autotune_group(dqmc_batch* b, Group& g, double box, int reps, double* rep) {
   int best_wq = g.wg_qr, best_nb = g.qr_nb;
   for (int nb : {16, 8}) {
     if (nb == 16 && g.n > 512) continue;
-    for (int w : wgs) {
-      if (w > g.n / nb) continue;
+    for (int w : candidates(g.wg_qr)) {
+      if (w > g.n / nb && (w != g.wg_qr || nb != g.qr_nb)) continue;
       float ms = 0.f;
       const hipError_t e = timed([&]() { return launch_qr_blocked(st, g.d_desc, nch, g.n, MatRef{MK_NAMED, M_TMP},
                                                                   VecRef{VK_NAMED, V_D5}, 1, w, nb); },

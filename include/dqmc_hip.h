@@ -108,7 +108,8 @@ const char* dqmc_last_error(void);
 /* DQMC(p) + initialize_stack (dqmc_framework.jl:105-135, stack.jl:224-242). */
 int dqmc_ctx_create(const dqmc_params* p, const dqmc_operators* ops, int device, dqmc_ctx** out);
 int dqmc_ctx_destroy(dqmc_ctx* ctx);
-/* workgroups per chain for the cooperative kernels (QR, inverse, local updates); 0 = default */
+/* workgroups per chain for the cooperative kernels: QR and inverse up to 128, local updates up to
+ * 256; 0 leaves a count as it is */
 int dqmc_ctx_set_groups(dqmc_ctx* ctx, int wg_qr, int wg_inv, int wg_local);
 /* how calculate_greens (stack.jl:338-369) forms G = [1 + Ul Dl Tl (Ur Dr Tr)^H]^-1:
  * 0 (default) separates the D scales into max(D,1) and min(D,1) and inverts the
@@ -321,7 +322,8 @@ int dqmc_batch_set_merged(dqmc_batch* b, int enable);
 int dqmc_use_graph(dqmc_ctx* ctx, int enable);
 /* Autotuner. No reference counterpart (the reference has one fixed CPU code path). Per
  * shape group: times the local-update kernel over (variant, workgroups per chain) and the
- * blocked QR of the stack over (workgroups per chain, panel width 16 or 8) on the group's
+ * blocked QR of the stack over (workgroups per chain, panel width 16 or 8), the present
+ * settings among them, on the group's
  * current state, `reps` timed launches each after a warm-up, and keeps the fastest. The
  * chains' G, field, scalars and uniform cursor are restored bit for bit (local updates are
  * timed on synthetic uniforms), so tuning does not change the Monte Carlo trajectory. Needs

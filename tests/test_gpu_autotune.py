@@ -81,3 +81,33 @@ def test_batch_autotune_matches_untuned(amd):
         assert bt.stats(k).accepted == bd.stats(k).accepted
     bt.close()
     bd.close()
+
+
+def test_local_workgroups_up_to_one_per_cu(amd):
+    """The default of a lone chain with n = 1024 is 256 workgroups: it can be set by hand, with the
+    same result bit for bit, and the tuner measures it (with at most 128 the own columns leave LDS
+    and the updates take nearly twice as long, so it is what the tuner keeps)."""
+    mod, DQMC = amd
+    from dqmc_amd import UniformStream
+    p = config_params(mod, 16, 20)
+    phi = np.random.default_rng(5).uniform(-1, 1, (3, p.N, p.slices))
+    got = []
+    for counts in ((), (64, 256)):
+        _say("n = 1024, local workgroups set to %s" % (counts,))
+        c = DQMC(p, uniforms=UniformStream(7))
+        c.init(phi)
+        for w in counts:
+            c.set_groups(wg_local=w)
+        c.local_updates()
+        got.append((c.greens, c.hsfield))
+        if counts:
+            for kw in ({"wg_local": 257}, {"wg_qr": 129}, {"wg_inv": 129}):
+                with pytest.raises(mod.DQMCError):
+                    c.set_groups(**kw)
+            _say("n = 1024, autotune")
+            rep = c.autotune(reps=1)
+            _check_report(rep, p.n)
+            assert rep["local_variant"] == 4 and rep["local_workgroups"] > 128
+            assert np.array_equal(c.greens, got[-1][0])
+        c.close()
+    assert all(np.array_equal(x, y) for x, y in zip(*got))
