@@ -139,7 +139,17 @@ struct Group {
   };
   std::vector<Rec> prof;
   std::vector<hipEvent_t> event_pool;
+  // a temporary group (jobs, merged sweeps) draws its events from this group and records into
+  // it: the pool outlives it, and reading the profile returns the events there
+  Group* prof_owner = nullptr;
+  void record(const Rec& r) {
+    if (prof_owner)
+      prof_owner->record(r);
+    else
+      prof.push_back(r);
+  }
   hipEvent_t take_event() {
+    if (prof_owner) return prof_owner->take_event();
     if (!event_pool.empty()) {
       hipEvent_t e = event_pool.back();
       event_pool.pop_back();
@@ -484,7 +494,7 @@ struct ProfScope {
     if (e0) {
       hipEvent_t e1 = g.take_event();
       (void)hipEventRecord(e1, g.stream);
-      g.prof.push_back({cls, e0, e1});
+      g.record({cls, e0, e1});
     }
   }
 };
@@ -1508,7 +1518,7 @@ void merged_descs(dqmc_batch* b, const MergedShape& ms, int T, const int* d_plan
 int merged_enqueue(dqmc_batch* b, const MergedShape& ms, int T, const int* d_plan, const ChainDesc* d_desc,
                    const std::vector<size_t>& set_off, const std::vector<int>& kinds, const std::vector<int>& set_of,
                    double box, int dolog) {
-  const Group& g0 = b->groups[0];
+  Group& g0 = b->groups[0];
   const int nch = ms.nch, s = ms.s;
   const int* d_sel = d_plan + (size_t)nch * T * kPlanRoles;
   const int* d_sli = d_sel + (size_t)T * kMergedApplies * nch;
@@ -1528,6 +1538,7 @@ int merged_enqueue(dqmc_batch* b, const MergedShape& ms, int T, const int* d_pla
   mg.wg_inv = g0.wg_inv;
   mg.local_variant = g0.local_variant;
   mg.prof_mask = g0.prof_mask;
+  mg.prof_owner = &g0;  // (dqmc_batch_profile_read)
   for (int t = 0; t < T; ++t) {
     const std::vector<int>& act = ms.sets[set_of[t]];
     const int na = (int)act.size();
@@ -1608,12 +1619,6 @@ int merged_enqueue(dqmc_batch* b, const MergedShape& ms, int T, const int* d_pla
       LCHK(launch_local_updates(mg.stream, dd, na, an, 0, d_loc + (size_t)t * nch, box, mg.wg_local, dolog, variant,
                                 by_size ? mg.local_map : nullptr, by_size ? mg.local_map_blocks : 0));
     }
-  }
-  // timing records of the pseudo group belong to the first group (dqmc_batch_profile_read)
-  if (!mg.prof.empty()) {
-    Group& gp0 = b->groups[0];
-    gp0.prof.insert(gp0.prof.end(), mg.prof.begin(), mg.prof.end());
-    mg.prof.clear();
   }
   return 0;
 }
@@ -2275,7 +2280,7 @@ hipError_t jobs_upload(JobSet& js, const ChainMem& cm, const std::vector<ChainDe
   return e;
 }
 // a group over `nj` jobs of g's chain on g's stream, the workgroups shared between them
-Group job_group(const Group& g, ChainDesc* d_desc, int nj) {
+Group job_group(Group& g, ChainDesc* d_desc, int nj) {
   Group j;
   j.n = g.n;
   j.N = g.N;
@@ -2293,15 +2298,11 @@ Group job_group(const Group& g, ChainDesc* d_desc, int nj) {
   j.udt_route = g.udt_route;
   j.qr_nb = g.qr_nb;
   j.prof_mask = g.prof_mask;
+  j.prof_owner = &g;
   const int per = std::max(1, 256 / nj);
   j.wg_qr = std::max(1, std::min(g.wg_qr, per));
   j.wg_inv = std::max((g.n + 511) / 512, std::min(g.wg_inv, per));
   return j;
-}
-// its timing records go to the chain's group
-void job_group_done(Group& g, Group& j) {
-  g.prof.insert(g.prof.end(), j.prof.begin(), j.prof.end());
-  g.event_pool.insert(g.event_pool.end(), j.event_pool.begin(), j.event_pool.end());
 }
 
 // Time-displaced Green's functions as jobs. The four checkpoint chains do not depend on one
@@ -2464,7 +2465,6 @@ int tdgf_parallel(Group& g, ChainMem& cm) {
       RC(o.udt(cur, pv(b, TA_DD), pm(b, TA_Q), pm(b, TA_T)));
       if (i != 0) RC(o.gemm(pm(b, TA_GC), pm(b, TA_GA), OP_N, pm(b, TA_GB), OP_N));
     }
-    job_group_done(g, all);
   }
   for (int c = 0; c < lo.rounds; ++c) {
     const int nj = std::min(lo.slots, 2 * R - c * lo.slots), b = c * kTdgfInvRoles;
@@ -2496,7 +2496,6 @@ int tdgf_parallel(Group& g, ChainMem& cm) {
     RC(o.gemm(pm(b, TB_RES), NM(M_QRT), OP_N, NM(M_TMP3), OP_N));
     RC(o.effective_greens(pm(b, TB_RES)));
     LCHK(launch_negate(st, dd, nj, n, pm(b, TB_NEG)));
-    job_group_done(g, all);
   }
   // fill_tdgf! from the checkpoints, one slice of every interval per launch
   ChainDesc* df = js.d_desc + 4 + lo.slots;
@@ -2510,7 +2509,6 @@ int tdgf_parallel(Group& g, ChainMem& cm) {
     LCHK(launch_apply_B_chkr_sel(st, df, R, n, N, pm(2 * t, 0), B_LEFT, B_INV_LEFT, fs, sl, g.ngroups));
     LCHK(launch_apply_B_chkr_sel(st, df + R, R, n, N, pm(2 * t, 0), B_INV_RIGHT, B_RIGHT, fs, sl, g.ngroups));
   }
-  job_group_done(g, all);
   return 0;
 }
 
@@ -2820,8 +2818,6 @@ int grad_parallel(Group& g, ChainMem& cm) {
       RC(oh.udt(NM(M_CURU), VecRef{VK_PLAN, p + 4}, MatRef{MK_PLAN, p + 3}, NM(M_QRT), true));
       RC(oh.gemm(MatRef{MK_PLAN, p + 5}, NM(M_QRT), OP_N, MatRef{MK_PLAN, p + 2}, OP_N));
     }
-    job_group_done(g, both);
-    job_group_done(g, left);
   }
   Group all = job_group(g, js.d_desc, R);
   Ops oa(all);
@@ -2838,7 +2834,6 @@ int grad_parallel(Group& g, ChainMem& cm) {
   }
   if (g.all_checks && R > 1) LCHK(launch_maxdiff(st, js.d_desc + 1, R - 1, n, NM(M_G), NM(M_GRAD)));
   LCHK(launch_fold_jobs(st, g.d_desc, js.d_desc, R, g.all_checks ? 1 : 0));
-  job_group_done(g, all);
   g.cur = 1;
   g.dir = -1;
   g.recomputed = g.all_checks && sm == 1 && R > 1;
@@ -3093,8 +3088,6 @@ int meas_chains(Group& g, ChainMem& cm) {
     RC(o.gemm(NM(M_TMP), NM(M_QRT), OP_N, NM(M_TR), OP_N));
     RC(o.copy(NM(M_TR), NM(M_TMP)));
   }
-  job_group_done(g, both);
-  job_group_done(g, left);
   return 0;
 }
 
