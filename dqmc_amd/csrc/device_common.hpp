@@ -319,6 +319,12 @@ __device__ inline void group_sync(const GroupSync& g) {
   __syncthreads();
 }
 
+// Whether a workgroup's word of flag_sync has arrived at `target`. Nobody passes a barrier before
+// everybody has arrived there, so a word is at the target, one ahead, or still behind -- however far:
+// the counter wraps, and a word that was idle while it advanced by more than half its range (a chain
+// that ran with fewer workgroups for hours and is given more again) is behind as well.
+__host__ __device__ inline bool flag_arrived(unsigned int word, unsigned int target) { return word - target <= 1u; }
+
 // Barrier of a group whose workgroups publish by write-through stores (st_wt) and read what the
 // others published from cache lines that they have not touched since the kernel began: it needs
 // neither the write-back nor the invalidation of the XCD's L2, which every workgroup would issue
@@ -340,7 +346,7 @@ __device__ inline bool flag_sync(unsigned int* flags, unsigned int target, int w
   bool ok = true;
   if (t < W) {
     long long spins = 0;
-    while ((int)(__hip_atomic_load(flags + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
+    while (!flag_arrived(__hip_atomic_load(flags + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), target)) {
       if ((++spins & 31) == 0) {
         if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
           ok = false;
