@@ -1,12 +1,14 @@
 // Blocked Householder QR on a chain group, and the solve that uses it.
 //
-// k_qr_pipe (8-column panels, the default) and k_qr_blocked (16) factor A P0 = Q R panel by panel (compact WY, Q_p = I - V_p T_p V_p^H,
-// LAPACK zgeqrf/zlarft conventions). P0 is either the identity or the pre-pivoting
+// k_qr_pipe (8-column panels, the default) and k_qr_blocked (16) factor A P0 = Q R panel by
+// panel (compact WY, Q_p = I - V_p T_p V_p^H, LAPACK zgeqrf/zlarft conventions). P0 is either
+// the identity or the pre-pivoting
 // order: columns sorted once by decreasing initial norm (ties by index). For the
 // column-graded products DQMC stabilises, (B...B U) diag(D), QR with pre-pivoting is
 // as stable as column-pivoted QR (Bai, Lee, Li, Xu, "Stable solutions of linear systems
 // involving long chain of matrix multiplications", Linear Algebra Appl. 435 (2011)),
-// while needing one group barrier per panel instead of one per column.
+// while the workgroups exchange once per panel (k_qr_pipe by flags, k_qr_blocked by a group
+// barrier) instead of once per column.
 //
 // The output uses the layout of k_qrp (columns never move: logical column k lives in
 // physical column qr_perm[k]; reflector k below the diagonal of that column, R on and
@@ -99,21 +101,22 @@ __device__ inline void stage_panel(cplx* P, const gcplx* A, const int* perm, int
 // vector updates -> this): n = 64 163 -> 77, n = 256 631 -> 350, n = 400 1008 -> 730, n = 576
 // 1850 -> 1320, n = 1024 5000 -> 3650. A panel at n = 400 takes 33,800 cycles: 15,700 in the eight
 // column steps, 4,600 writing it back, 3,700 in V^H X, 3,300 for the next block's flag and loads,
-// 2,100 each in the update, the move to rows and the wait for the loads.
+// 2,100 each in the update, the move to rows and the wait for the loads. Above n = 512 a thread's
+// rows and tiles exceed its 256 registers: RQ = 3 spills 18 of them (76 bytes per lane), RQ = 4 154
+// (548 bytes), inside the panel chain; RQ = 1 and 2 spill none.
 // ---------------------------------------------------------------------------
 // Bounded wait of a whole workgroup for *f >= want: thread 0 polls (relaxed loads, one acquire
-// fence after the last; `seen` is a value it has loaded before), everyone learns the outcome
-// through LDS. false: the wait timed out here
+// fence after the last), everyone learns the outcome through LDS. false: the wait timed out here
 // or in another workgroup of the chain.
 __device__ inline unsigned flag_load(const unsigned* f) {
   return __hip_atomic_load((const __attribute__((address_space(1))) unsigned*)f, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline bool wait_flag(const unsigned* f, unsigned want, unsigned seen, int* error, int* s_fail) {
+__device__ inline bool wait_flag(const unsigned* f, unsigned want, int* error, int* s_fail) {
   if (threadIdx.x == 0) {
     int fail = 0;
     long long spins = 0;
-    for (; seen < want; seen = flag_load(f)) {
+    while (flag_load(f) < want) {
       if ((++spins & 31) == 0) {
         if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
           fail = 1;
@@ -658,7 +661,7 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
       fb = own;
       if (fb >= nblk) return;  // no block of this workgroup is left
       if (!mt) load_tiles(fb * NB, k0);  // (own columns: before the panel is there)
-      if (!wait_flag(flags, (unsigned)(p + 1), 0u, err, &s_fail)) return;
+      if (!wait_flag(flags, (unsigned)(p + 1), err, &s_fail)) return;
       stage_V(k0);
       if (tid < NB * NB) Tl[tid] = ld(Tf + (size_t)p * NB * NB + tid);
       __syncthreads();
@@ -689,7 +692,7 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
     column_steps(k1);
     if (need) {
       // block p+2 carries panel p; its owner has had a panel's time to bring it up to date
-      if (!wait_flag(flags + 1 + (p + 2), 1u, 0u, err, &s_fail)) return;
+      if (!wait_flag(flags + 1 + (p + 2), 1u, err, &s_fail)) return;
     } else {
       __syncthreads();
     }
@@ -719,7 +722,8 @@ template <int NB, int RQ>
 __global__ __launch_bounds__(256) void k_qr_blocked(const ChainDesc* chains, MatRef Ar, VecRef Dr, int prepivot,
                                                     int ps, const int* bmap) {
   constexpr int V = 2 * NB;               // doubles per butterfly
-  constexpr int LS = NB == 8 ? 2 : 1;     // after it, lane l holds value l >> LS
+  constexpr int LS = 1;                   // after it, lane l holds value l >> LS
+  static_assert(NB == 16, "");
   // grid (W, chains), or with a block map a 1-D grid where block b serves chain bmap[b] & 0xFFFF
   // as workgroup (bmap[b] >> 16) & 0xFF of (bmap[b] >> 24) (workgroup counts per chain)
   const int bm = bmap ? bmap[blockIdx.x] : 0;
