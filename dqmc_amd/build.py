@@ -24,7 +24,8 @@ FLAGS = [
 
 # The windowed local-update kernel holds many phases in one loop nest: hoisting their constants
 # and lane addresses out of it spills 27 registers into the loop that decides proposals
-# (reloads of some 800 cycles each on its serial chain); without the hoisting none spill.
+# (reloads of some 800 cycles each on its serial chain); without the hoisting the instance with
+# LDS-resident columns spills none and the other one 4 (20 bytes per lane).
 FILE_FLAGS = {"k_local.hip": ["-mllvm", "-disable-machine-licm"]}
 
 

@@ -273,8 +273,8 @@ hipError_t launch_inverse_gather(hipStream_t s, const ChainDesc* chains, int nch
 // One local-update pass over all sites at `slice` (0-based). variant 1 updates G in global
 // memory after every accepted proposal, 2 keeps each workgroup's column block of G in LDS
 // (needs local_tile_fits), 3 delays the rank-4 updates and flushes them in groups (needs
-// local_delayed_fits), 4 processes the sites in windows with one group barrier per window
-// (needs local_window_sites(nmax, wg) >= 2: the largest window that fits in LDS; *tile
+// local_delayed_fits), 4 processes the sites in windows with one exchange between the
+// workgroups per window (flag words with LDS-resident columns, else a group barrier; needs local_window_sites(nmax, wg) >= 2: the largest window that fits in LDS; *tile
 // tells whether the workgroups' own columns of G stay in LDS as well). bmap (variant 4 only):
 // per-block (chain, workgroup, workgroup count) map of a 1-D grid of nblocks, from
 // local_block_map; each chain then sizes its own window.

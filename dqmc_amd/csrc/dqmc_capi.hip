@@ -2340,8 +2340,10 @@ struct TdgfLayout {
   }
 };
 
-// the batched slice operators need a checkerboard; the fill from both sides of M / 2 meets at a
-// checkpoint for even R only; the verbatim routes keep the sequential pass
+// The jobs apply their slice matrices in place, each its own operator in one launch; without the
+// checkerboard B is a product that needs a second buffer per job (dense_B), which they do not
+// have: the dense hopping keeps the sequential pass. So do the verbatim routes, and odd R, for
+// which the fill from both sides of M / 2 does not meet at a checkpoint.
 bool tdgf_parallel_ok(const Group& g) {
   return g.greens_route == 0 && g.udt_route == 0 && g.chkr && (g.M / g.s) % 2 == 0 && g.M % g.s == 0;
 }
@@ -2854,7 +2856,8 @@ static int grad_enqueue(dqmc_batch* b) {
     HIPCHK(hipMalloc(&cm.mom, sizeof(double) * 3 * cm.N * cm.M));
     HIPCHK(hipMalloc(&cm.phi_bak, sizeof(double) * 3 * cm.N * cm.M));
   }
-  // the verbatim routes and the dense hopping keep the sequential pass, as do more intervals than jobs
+  // the verbatim routes and the dense hopping (see tdgf_parallel_ok) keep the sequential pass, as do
+  // more intervals than jobs
   if (g.greens_route == 0 && g.udt_route == 0 && g.chkr && g.nelem - 1 <= kMaxGradJobs && !cm.grad_jobs.failed) {
     if (!cm.grad_jobs.mem && (rc = grad_jobs_create(g, cm))) return rc;
     if (!cm.grad_jobs.failed) {
@@ -3103,7 +3106,7 @@ int dqmc_measure_greens(dqmc_ctx* ctx, double* G) {
   ChainMem& cm = b->chains[0];
   RC(meas_alloc(cm));
   Ops o(g);
-  // the batched slice operators need a checkerboard; the verbatim routes keep the one chain
+  // the dense hopping (see tdgf_parallel_ok) and the verbatim routes keep the one chain
   const bool halves = g.greens_route == 0 && g.udt_route == 0 && g.chkr && g.M % g.s == 0 && g.M / g.s >= 2;
   if (halves && !cm.meas_jobs.mem && !cm.meas_jobs.failed) RC(meas_jobs_create(g, cm));
   if (halves && cm.meas_jobs.mem) {

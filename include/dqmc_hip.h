@@ -121,15 +121,15 @@ int dqmc_set_greens_route(dqmc_ctx* ctx, int route);
  * sites of a slice: 1 updates G in global memory after every accepted proposal; 2 keeps
  * each workgroup's column block of G in LDS; 3 delays the rank-4 updates (up to 8 pending,
  * decisions from LDS-resident diagonal blocks) and adds them to G in one pass; 4 visits the
- * sites in windows of up to 8, keeping the window's accepted updates as factor pairs in
- * every workgroup and adding them to G once per window (one group barrier per window);
+ * sites in windows of up to 16 or 20, keeping G between the window's sites in every workgroup
+ * and updating the rest of G once per window (one exchange between workgroups per window);
  * 0 (default) picks 4, else 2, else 3, else 1, by what fits in LDS. Same results to
  * rounding; an error when a forced variant does not fit. */
 int dqmc_set_local_variant(dqmc_ctx* ctx, int variant);
 /* how the stack's decompose_udt! (linalg.jl:20-39) factors inside build_stack /
  * add_slice_sequence_*: 0 (default) blocked Householder QR after pre-pivoting the
- * columns by decreasing norm (two group barriers per 16-column panel), 1 column-
- * pivoted QR with zgeqp3's pivot sequence (one barrier per column). Both are stable for
+ * columns by decreasing norm (one exchange between workgroups per panel), 1 column-
+ * pivoted QR with zgeqp3's pivot sequence (one exchange per column). Both are stable for
  * the stack's column-graded products and give the same G; only the stack's internal
  * U, D, T differ. Every other factorisation (dqmc_udt, the direct and time-displaced
  * Green's functions, whose chains are also row-graded) uses route 1. */
