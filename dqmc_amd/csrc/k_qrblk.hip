@@ -102,8 +102,15 @@ __device__ inline void stage_panel(cplx* P, const gcplx* A, const int* perm, int
 // 1850 -> 1320, n = 1024 5000 -> 3650. A panel at n = 400 takes 33,800 cycles: 15,700 in the eight
 // column steps, 4,600 writing it back, 3,700 in V^H X, 3,300 for the next block's flag and loads,
 // 2,100 each in the update, the move to rows and the wait for the loads. Above n = 512 a thread's
-// rows and tiles exceed its 256 registers: RQ = 3 spills 18 of them (76 bytes per lane), RQ = 4 154
-// (548 bytes), inside the panel chain; RQ = 1 and 2 spill none.
+// rows and tiles exceed its 512 registers: RQ = 3 spills 18 (76 bytes per lane), RQ = 4 154 (548
+// bytes), inside the panel chain; RQ = 1 and 2 spill none.
+//
+// WIDE: every trailing update of the launch is the 16-column one, workgroup 0's too when it is
+// alone. It serves n > 512 with few workgroups per chain (launch_qr_blocked): one workgroup in the
+// tile form waits for each block's loads in turn and was slower than the vector kernel that k_qr_pipe
+// replaced (ms per factorisation, vector / tile form / this: n = 576 23.3 / 26.3 / 17.0, n = 1024 104 /
+// 138 / 85), and with two to nine the instance without the block loop spills less (RQ = 4: 134
+// registers; n = 1024, W = 2: 84 / 92 / 82, W = 4: 41 / 41 / 37; RQ = 3 the same either way).
 // ---------------------------------------------------------------------------
 // Bounded wait of a whole workgroup for *f >= want: thread 0 polls (relaxed loads, one acquire
 // fence after the last), everyone learns the outcome through LDS. false: the wait timed out here
@@ -166,7 +173,7 @@ __device__ inline double recip(double x) {
   return fma(r, fma(-x, r, 1.0), r);
 }
 
-template <int RQ>
+template <int RQ, bool WIDE>
 __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef Ar, VecRef Dr, int prepivot, int ps,
                                                  const int* bmap) {
   constexpr int NB = 8, V = 2 * NB, LS = 2;  // V doubles per butterfly; after it, lane l holds value l >> LS
@@ -190,8 +197,8 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
   const int nblk = (n + NB - 1) / NB;
   const int off = n - 256 * RQ;
   // with many columns per trailing workgroup (at least 128 at the start) a wave takes 16 of them
-  // at a time instead of the workgroup 8: no barriers, but X streams from memory twice
-  const bool mt = W > 1 && n >= 128 * (W - 1);
+  // at a time instead of the workgroup 8: no barriers, but X streams from memory twice (WIDE: always)
+  const bool mt = WIDE || (W > 1 && n >= 128 * (W - 1));
 
   extern __shared__ double smem[];
   cplx* P = reinterpret_cast<cplx*>(smem);  // [NB][ps] panel V (rows k0..n-1 used, row r at 16 + r)
@@ -543,8 +550,8 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
     }
   };
   const int ws = W == 1 ? 1 : W - 1;  // workgroups of the trailing blocks
-  // Trailing update of panel p (rows >= k0) on the matrix cores (mt), for workgroups w >= 1: the
-  // own blocks from fb on in tiles of two blocks, 16 columns, tile q to wave q mod 4.
+  // Trailing update of panel p (rows >= k0) on the matrix cores (mt), for workgroups w >= 1 or the
+  // only one: the own blocks from fb on in tiles of two blocks, 16 columns, tile q to wave q mod 4.
   // Per tile: W = V^H X (K = rows, A(i, k) = conj V(r, i), B(k, j) = X(r, col_j)), then
   // Z = T^H W with the vector units (lane (j, k) forms Z(k, j) and Z(k + 4, j), exactly its B
   // operands of the second product), then X -= V Z in 16-row tiles. X streams from global
@@ -655,6 +662,11 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
     if (W > 1 && w != 0) loaded = true;
     if (W == 1) {
       fb = p < 0 ? nblk : p + 2;
+      if (WIDE && fb < nblk) {
+        trailing_mfma(k0, fb, -1);
+        __syncthreads();  // wscr is in part's place
+        fb = nblk;
+      }
     } else if (w != 0) {
       if (p < 0) continue;
       while (own < p + 2) own += ws;
@@ -671,6 +683,8 @@ __global__ __launch_bounds__(256) void k_qr_pipe(const ChainDesc* chains, MatRef
       }
     }
     // the own trailing blocks first, then, on workgroup 0, panel p+1 itself, which stays in X
+    // (WIDE: the panel alone)
+    if (WIDE) fb = nblk;
     for (;; fb += ws) {
       const bool next = fb >= nblk;
       if (next && w != 0) break;
@@ -1794,10 +1808,13 @@ hipError_t launch_qr_blocked(hipStream_t s, const ChainDesc* chains, int nchains
     return launch_qr_kernel((const void*)k_qr_blocked<16, 2>, (size_t)16 * ps * sizeof(cplx), s, chains, nchains, ps, A,
                             D, prepivot, wg, bmap, nblocks);
   if (nb != 8) return hipErrorInvalidValue;
-  const void* fn = nmax <= 256   ? (const void*)k_qr_pipe<1>
-                   : nmax <= 512 ? (const void*)k_qr_pipe<2>
-                   : nmax <= 768 ? (const void*)k_qr_pipe<3>
-                                 : (const void*)k_qr_pipe<4>;
+  // (a block map gives the chains of each size their workgroups, more for the larger)
+  const bool wide = nmax > 512 && !bmap && (wg == 1 || nmax >= 128 * (wg - 1));
+  const void* fn = nmax <= 256   ? (const void*)k_qr_pipe<1, false>
+                   : nmax <= 512 ? (const void*)k_qr_pipe<2, false>
+                   : nmax <= 768 ? (wide ? (const void*)k_qr_pipe<3, true> : (const void*)k_qr_pipe<3, false>)
+                   : wide        ? (const void*)k_qr_pipe<4, true>
+                                 : (const void*)k_qr_pipe<4, false>;
   ps = mfma_ld(nmax + 16);
   return launch_qr_kernel(fn, ((size_t)8 * ps + 512) * sizeof(cplx), s, chains, nchains, ps, A, D, prepivot, wg, bmap,
                           nblocks);
