@@ -3,8 +3,8 @@ first ones the process creates none.
 
 An event is an object of the runtime on this thread's heap, about 1.1 KB (mallinfo2 counts it), and
 a timed launch records two. The runtime's heap grows by itself from launch to launch, so profiled
-evaluations are compared with as many plain ones: they may grow it by 256 bytes more per record,
-where creating the events anew takes some 2 KB.
+evaluations are compared with as many plain ones: they may grow it by 1 KB more per record,
+half of what creating the events anew takes.
 """
 import ctypes
 
@@ -46,5 +46,5 @@ def test_events_are_reused(what):
     assert cnt.sum() == 0
     profiled = growth((1 << _capi.K_NCLASS) - 1)
     assert cnt.sum() > 20 and ms.sum() > 0
-    assert profiled - plain < 50 * 256 * int(cnt.sum())
+    assert profiled - plain < 50 * 1024 * int(cnt.sum())
     c.close()
