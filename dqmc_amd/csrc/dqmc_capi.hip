@@ -2317,7 +2317,7 @@ Group job_group(Group& g, ChainDesc* d_desc, int nj) {
 // as inv_sum_udts_scalettar, but as with calculate_greens_scalesep N is well conditioned and one
 // unpivoted QR and a solve take the place of two factorisations, an inverse and three products;
 // Tb^-1 likewise. [1 + U D T]^-1 of slice 1 is the case Ua = Da = Ta = 1. L = 8, M = 100:
-// measure_tdgfs 350 -> 42 ms.
+// measure_tdgfs 350 -> 42 ms (26 with the pivoted QR by tagged candidates).
 constexpr int kMaxTdgfJobs = 32;
 enum : int { TA_SRC, TA_SD, TA_DD, TA_Q, TA_T, TA_GC, TA_GA, TA_GB, kTdgfChainRoles };
 enum : int { TB_AU, TB_AD, TB_AT, TB_BU, TB_BD, TB_BT, TB_RES, TB_NEG, kTdgfInvRoles };
@@ -3025,7 +3025,7 @@ namespace {
 // left operand and (B_l .. B_1)^H into the right one of calculate_greens, l half the slices,
 // instead of all of them into the right one: half as deep, and fewer factorisations behind each
 // operand. Descriptor 0 is the left chain, under the names of the right operand, 1 the chain
-// itself. L = 8, M = 100: dqmc_measure_greens 35 -> 17 ms.
+// itself. L = 8, M = 100: dqmc_measure_greens 35 -> 17 ms (12 with the pivoted QR by tagged candidates).
 int meas_jobs_create(const Group& g, ChainMem& cm) {
   JobSet& js = cm.meas_jobs;
   const int R = g.M / g.s, sm = g.s, h1 = R / 2;

@@ -99,7 +99,7 @@ __device__ inline void stage_panel(cplx* P, const gcplx* A, const int* perm, int
 //
 // Measured (one chain, default workgroups, us per factorisation, one group barrier per panel and
 // vector updates -> this): n = 64 163 -> 77, n = 256 631 -> 350, n = 400 1008 -> 730, n = 576
-// 1850 -> 1320, n = 1024 5000 -> 3650. A panel at n = 400 takes 33,800 cycles: 15,700 in the eight
+// 1850 -> 1320, n = 1024 5000 -> 3390. A panel at n = 400 takes 33,800 cycles: 15,700 in the eight
 // column steps, 4,600 writing it back, 3,700 in V^H X, 3,300 for the next block's flag and loads,
 // 2,100 each in the update, the move to rows and the wait for the loads. Above n = 512 a thread's
 // rows and tiles exceed its 512 registers: RQ = 3 spills 18 (76 bytes per lane), RQ = 4 154 (548
